@@ -720,8 +720,31 @@ static int prof_collect(md_ctx* c) {
     return MD_OK;
 }
 
+// Particles expected within `radius` of one another, the largest of the
+// replicas at the boxes of C.
+static double expected_neighbours(const md_ctx* c, const std::vector<RepCtrl>& C, double radius) {
+    double ne = 0.0;
+    for (int r = 0; r < c->R; ++r) {
+        const double v = C[r].box[0] * C[r].box[1] * C[r].box[2];
+        if (v > 0.0) ne = std::max(ne, (double)c->reps[r].n_atoms / v * (4.0 / 3.0 * M_PI) * radius * radius * radius);
+    }
+    return ne;
+}
+
+// Which kernel instances the next launches use (DevState::dense).  List
+// paths: long lists expected.  All-pairs path: k_ap_force keeps the pairs in
+// range of a particle in a list of kApCap = 96 entries and puts them in order
+// afterwards; above half of that on average too many particles overflow it and
+// are summed one thread each, and the ordering costs more than it saves.
+static void choose_instances(md_ctx* c, const std::vector<RepCtrl>& C) {
+    if (c->list_mode)
+        c->d.dense = expected_neighbours(c, C, c->rlist) >= (double)kLaneWalk ? 1 : 0;
+    else
+        c->d.dense = expected_neighbours(c, C, c->rc_max) > 48.0 ? 1 : 0;
+}
+
 // One step launch: list paths k_step + k_fin (which also builds lists),
-// all-pairs path k_drift + k_allpairs + k_fin.
+// all-pairs path k_drift + k_ap_force + k_ap_finish (or k_allpairs) + k_fin.
 static hipError_t launch_once(md_ctx* c) {
     hipError_t e;
     c->d.par = c->par;
@@ -735,7 +758,12 @@ static hipError_t launch_once(md_ctx* c) {
         if ((e = launch_step(c->d, c->fp32, c->bs, c->st))) return e;
     } else {
         if ((e = launch_drift(c->d, c->bs, c->st))) return e;
-        if ((e = launch_allpairs(c->d, c->bs, false, c->st))) return e;
+        if (c->d.dense) {
+            if ((e = launch_allpairs(c->d, c->bs, false, c->st))) return e;
+        } else {
+            if ((e = launch_ap_force(c->d, c->bs, false, c->st))) return e;
+            if ((e = launch_ap_finish(c->d, c->bs, c->st))) return e;
+        }
     }
     return finalize(c, M_STEP);
 }
@@ -992,17 +1020,8 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
             } else if ((rc = snapshot(c, true))) {
                 return rc;
             }
-            // dense systems (long lists expected at the current densities)
-            // step and build with the long-list kernel instances
-            double ne = 0.0;
-            for (int r = 0; r < c->R; ++r) {
-                const double v = C[r].box[0] * C[r].box[1] * C[r].box[2];
-                if (v > 0.0)
-                    ne = std::max(ne, (double)c->reps[r].n_atoms / v * (4.0 / 3.0 * M_PI) * c->rlist * c->rlist *
-                                          c->rlist);
-            }
-            c->d.dense = ne >= (double)kLaneWalk ? 1 : 0;
         }
+        choose_instances(c, C);
         for (int r = 0; r < c->R; ++r) {
             P[r].target_step = step0 + done + cn;
             P[r].use_psi_in = first ? 1 : 0;
@@ -1622,10 +1641,18 @@ int md_update_force(md_ctx* c) {
     std::vector<RepParams> P((size_t)c->R, base_params(c));
     int rc = write_params(c, P);
     if (rc) return rc;
+    std::vector<RepCtrl> C;
+    if ((rc = read_ctrl(c, C))) return rc;
+    choose_instances(c, C);
     c->d.par = c->par;
-    if (c->n_blocks > 0) HIPCHK(c, launch_allpairs(c->d, c->bs, true, c->st));
-    HIPCHK(c, finalize(c, M_REDUCE));
-    if ((rc = reduce_state_sums(c, 1))) return rc;
+    if (c->d.dense) {
+        if (c->n_blocks > 0) HIPCHK(c, launch_allpairs(c->d, c->bs, true, c->st));
+        HIPCHK(c, finalize(c, M_REDUCE));
+        if ((rc = reduce_state_sums(c, 1))) return rc;
+    } else {
+        if (c->n_blocks > 0) HIPCHK(c, launch_ap_force(c->d, c->bs, true, c->st));
+        if ((rc = reduce_state_sums(c, 2))) return rc;
+    }
     HIPCHK(c, hipStreamSynchronize(c->st));
     c->sums_valid = true;
     return MD_OK;

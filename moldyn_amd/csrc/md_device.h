@@ -214,6 +214,7 @@ struct DevState {
     const uint8_t* slot_type;  // type of every slot (padding slots: the group's type)
     int32_t compact;         // the list path steps on crec (k_fin builds from crec)
     int32_t dense;           // long lists expected: lanes walk their own lists, builds sort long lists in LDS
+                             // (all-pairs path: many pairs in range, a thread per particle sums as it goes)
     double* pot;
     double* vir;
     int32_t* nbr;
@@ -440,6 +441,8 @@ hipError_t launch_epilogue(const DevState& d, int par, RepCtrl* h_ctrl, RepStats
 hipError_t launch_finalize(const DevState& d, int mode, bool build, bool fp32, hipStream_t st);
 hipError_t launch_drift(const DevState& d, int bs, hipStream_t st);
 hipError_t launch_allpairs(const DevState& d, int bs, bool force_only, hipStream_t st);
+hipError_t launch_ap_force(const DevState& d, int bs, bool force_only, hipStream_t st);
+hipError_t launch_ap_finish(const DevState& d, int bs, hipStream_t st);
 hipError_t launch_insert_all(const DevState& d, bool fp32, int bs, hipStream_t st);
 hipError_t launch_force_eval(const DevState& d, bool fp32, int bs, hipStream_t st);
 hipError_t launch_reduce_state(const DevState& d, bool fp32, int bs, hipStream_t st);

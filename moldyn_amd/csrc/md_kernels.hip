@@ -1464,6 +1464,226 @@ __global__ __launch_bounds__(BS) void k_allpairs(DevState d) {
     if (!FORCE_ONLY) prof_block(d, P_STEP, t_start, true, 0);
 }
 
+// The same sums for systems with few pairs in range, spread over the whole
+// chip.  A thread per particle leaves most of it idle (27,000 particles are 422
+// waves for 1,024 SIMDs) and runs a branch per minimum-image component of every
+// pair.  Here a block of eight waves owns 16 particles: j tiles of 512
+// candidates are staged through LDS, each wave tests its 64 of a tile against
+// the 16 particles (four candidates at a time, one a lane group), and a pair in
+// range goes into the particle's LDS list.  Then the lists are put in ascending
+// j order, the pair terms are computed a thread each, and one thread per
+// particle adds them in that order: the sums are bitwise those of k_allpairs.
+// The test takes min(|d|, |b - |d||), which is the magnitude of the reference's
+// minimum image bit for bit (rounding is monotonic, so the smaller of the two
+// is the branch the reference takes): 15 FP64 operations a pair, no branch.
+// They are the bound: 1.54e12 pairs/s of the 2.6e12 that 64 FP64 lanes per CU
+// and cycle allow.  Forces of 27,000 liquid particles: 6.80 ms with k_allpairs,
+// 0.47 ms here; of 1,000: 13 us.  16, 32 and 64 particles per block (one per
+// lane, fewer lane groups) measured 0.47 / 0.54 / 0.50 ms at 27,000 and 55 / 66
+// / 104 us at 8,000; two and four particles per lane (a half and a quarter of
+// the LDS reads) 0.62 and 0.49 ms at 27,000, 61 and 103 us at 8,000.
+constexpr int kApBS = 512, kApJ = kApBS, kApCap = 96, kApIT = 16;
+template <bool MULTI, bool FORCE_ONLY>
+__global__ __launch_bounds__(kApBS) void k_ap_force(DevState d, int bs) {
+    constexpr int IT = kApIT;
+    constexpr int Q = 64 / IT;       // candidates a wave tests at a time, one a lane group
+    constexpr int RPR = kApBS / IT;  // list entries per particle and round of the evaluation
+    __shared__ double term[5][kApBS];  // the j tiles first, then the pair terms
+    double* const tx = term[0];
+    double* const ty = term[1];
+    double* const tz = term[2];
+    __shared__ int32_t raw[kApCap][IT], srt[kApCap][IT];
+    __shared__ int cnt[IT];
+    const int subs = bs / IT;
+    const int b = blockIdx.x / subs, sub = blockIdx.x % subs;
+    const GroupInfo G = d.groups[d.blk_group[b]];
+    const int r = G.rep;
+    const RepCtrl& C = ctrl_in(d, r);
+    if (!FORCE_ONLY && (C.flags & F_EXIT)) return;
+    if (!FORCE_ONLY && d.prof && sub == 0 && threadIdx.x == 0)
+        d.prof_blk[((int64_t)P_STEP * d.n_blocks + b) * 3] = (unsigned long long)wall_clock64();
+    const RepInfo R = d.reps[r];
+    const TileRange tr = block_tiles(d, G, b, bs);
+    const int cur = C.cur;
+    Rec<double>* src = (Rec<double>*)d.rec[FORCE_ONLY ? cur : (cur ^ 1)];
+    const double bx = C.box[0], by = C.box[1], bz = C.box[2];
+    const int ti = G.type, T = d.n_types;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int il = lane % IT, q = lane / IT;
+    for (int64_t t = tr.t0; t < tr.t1; ++t) {
+        const int64_t s0 = t * bs + (int64_t)sub * IT;  // the block's first particle, within the group
+        if (s0 >= G.count) break;
+        const int64_t s = G.start + s0 + il;
+        double xi = __builtin_nan(""), yi = xi, zi = xi;  // fails every test
+        if (s0 + il < G.count) {
+            xi = src[s].x;
+            yi = src[s].y;
+            zi = src[s].z;
+        }
+        if (threadIdx.x < IT) cnt[threadIdx.x] = 0;
+        // candidates: the particles of the own and the later types
+        // (potential.rs:171-177)
+        for (int tj = ti; tj < (MULTI ? T : ti + 1); ++tj) {
+            const GroupInfo& H = d.groups[R.first_group + tj];
+            const int64_t h0 = H.start, n = H.count;
+            const double r2max = d.pairs[ti * T + tj].r2max;
+            double nx = __builtin_nan(""), ny = nx, nz = nx;  // the next tile's candidate of this thread
+            if ((int64_t)threadIdx.x < n) {
+                const Rec<double>& o = src[h0 + threadIdx.x];
+                nx = o.x;
+                ny = o.y;
+                nz = o.z;
+            }
+            for (int64_t j0 = 0; j0 < n; j0 += kApJ) {
+                __syncthreads();
+                tx[threadIdx.x] = nx;
+                ty[threadIdx.x] = ny;
+                tz[threadIdx.x] = nz;
+                __syncthreads();
+                const int64_t jn = j0 + kApJ + threadIdx.x;
+                nx = ny = nz = __builtin_nan("");
+                if (jn < n) {
+                    const Rec<double>& o = src[h0 + jn];
+                    nx = o.x;
+                    ny = o.y;
+                    nz = o.z;
+                }
+                // four candidates at a time: their LDS reads overlap the tests
+                for (int k = 0; k < 64 / Q; k += 4) {
+                    bool hit[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const int jl = w * 64 + (k + u) * Q + q;
+                        double ex = fabs(tx[jl] - xi), ey = fabs(ty[jl] - yi), ez = fabs(tz[jl] - zi);
+                        ex = fmin(ex, fabs(bx - ex));
+                        ey = fmin(ey, fabs(by - ey));
+                        ez = fmin(ez, fabs(bz - ez));
+                        hit[u] = (ex * ex + ey * ey) + ez * ez <= r2max;
+                    }
+                    if (!(hit[0] || hit[1] || hit[2] || hit[3])) continue;
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const int64_t j = h0 + j0 + w * 64 + (k + u) * Q + q;
+                        if (!hit[u] || j == s) continue;
+                        const int p = atomicAdd(&cnt[il], 1);
+                        if (p < kApCap) raw[p][il] = (int32_t)j;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        // ascending j: each entry goes to its rank (the j of a particle are distinct)
+        const int ei = threadIdx.x % IT, eq = threadIdx.x / IT;
+        const int m = cnt[ei] <= kApCap ? cnt[ei] : 0;  // a longer list is summed below
+        for (int p = eq; p < m; p += RPR) {
+            const int32_t v = raw[p][ei];
+            int rank = 0;
+            for (int o = 0; o < m; ++o) rank += raw[o][ei] < v ? 1 : 0;
+            srt[rank][ei] = v;
+        }
+        const int64_t se = G.start + s0 + ei;
+        double ax = 0.0, ay = 0.0, az = 0.0;
+        if (s0 + ei < G.count) {
+            ax = src[se].x;
+            ay = src[se].y;
+            az = src[se].z;
+        }
+        double fx = 0.0, fy = 0.0, fz = 0.0, pot = 0.0, vir = 0.0;
+        int mx = 0;
+        for (int k = 0; k < IT; ++k) mx = cnt[k] <= kApCap && cnt[k] > mx ? cnt[k] : mx;
+        for (int p0 = 0; p0 < mx; p0 += RPR) {
+            __syncthreads();
+            if (p0 + eq < m) {
+                const int32_t j = srt[p0 + eq][ei];
+                const Rec<double>& o = src[j];
+                const double dx = min_image(o.x - ax, bx), dy = min_image(o.y - ay, by), dz = min_image(o.z - az, bz);
+                const double r2 = (dx * dx + dy * dy) + dz * dz;
+                const PairTerms64 e = pair_exact_terms(dx, dy, dz, r2, d.pairs[ti * T + (MULTI ? (int)o.type : ti)]);
+                term[0][threadIdx.x] = e.gx;
+                term[1][threadIdx.x] = e.gy;
+                term[2][threadIdx.x] = e.gz;
+                term[3][threadIdx.x] = e.u;
+                term[4][threadIdx.x] = e.t;
+            }
+            __syncthreads();
+            if (threadIdx.x < IT)
+                for (int p = 0; p < RPR && p0 + p < m; ++p) {
+                    const int e = p * IT + ei;
+                    fx += term[0][e];
+                    fy += term[1][e];
+                    fz += term[2][e];
+                    pot += term[3][e];
+                    vir += term[4][e];
+                }
+        }
+        if (threadIdx.x < IT && s0 + ei < G.count) {
+            if (cnt[ei] > kApCap)  // more pairs than a list holds (a local cluster): in order from memory
+                for (int64_t j = G.start; j < R.end; ++j) {
+                    if (j == se) continue;
+                    const Rec<double>& o = src[j];
+                    const double dx = min_image(o.x - ax, bx), dy = min_image(o.y - ay, by), dz = min_image(o.z - az, bz);
+                    const double r2 = (dx * dx + dy * dy) + dz * dz;
+                    const PairParam& pp = d.pairs[ti * T + (MULTI ? (int)o.type : ti)];
+                    if (r2 <= pp.r2max) pair_exact(dx, dy, dz, r2, pp, fx, fy, fz, pot, vir);
+                }
+            src[se].fx = fx;
+            src[se].fy = fy;
+            src[se].fz = fz;
+            d.pot[se] = pot;
+            d.vir[se] = vir;
+        }
+        __syncthreads();  // cnt is cleared for the next tile
+    }
+}
+
+// The rest of a step after k_ap_force (integrator.rs:47-58): second half kick
+// and barostat scale from the drift buffer, and the block partials.
+template <int BS>
+__global__ __launch_bounds__(BS) void k_ap_finish(DevState d) {
+    const int b = blockIdx.x;
+    const GroupInfo G = d.groups[d.blk_group[b]];
+    const RepCtrl& C = ctrl_in(d, G.rep);
+    if (C.flags & F_EXIT) {
+        prof_block(d, P_STEP, 0, false, 0);
+        return;
+    }
+    // the launch's time starts with k_ap_force, which left its start here
+    const uint64_t t_start = d.prof ? d.prof_blk[((int64_t)P_STEP * d.n_blocks + b) * 3] : 0ull;
+    const TileRange tr = block_tiles(d, G, b, BS);
+    const int cur = C.cur;
+    const Rec<double>* __restrict__ src = (const Rec<double>*)d.rec[cur ^ 1];
+    Rec<double>* __restrict__ dst = (Rec<double>*)d.rec[cur];
+    const double m = G.mass, c = d.params[G.rep].cm[G.type], mu = C.myu;
+    const double* gs = d.sums + (int64_t)d.blk_group[b] * NS;
+    const double vr[3] = {sums_vref(gs, G.sum_m, 0), sums_vref(gs, G.sum_m, 1), sums_vref(gs, G.sum_m, 2)};
+    double part[NS];
+#pragma unroll
+    for (int k = 0; k < NS; ++k) part[k] = 0.0;
+    for (int64_t t = tr.t0; t < tr.t1; ++t) {
+        const int64_t s = G.start + t * BS + threadIdx.x;
+        if (t * BS + threadIdx.x >= G.count) continue;
+        Rec<double> a = src[s];
+        a.vx = a.vx + a.fx * c;
+        a.vy = a.vy + a.fy * c;
+        a.vz = a.vz + a.fz * c;
+        a.x = a.x * mu;
+        a.y = a.y * mu;
+        a.z = a.z * mu;
+        dst[s] = a;
+        part[S_MVX] += a.vx * m;
+        part[S_MVY] += a.vy * m;
+        part[S_MVZ] += a.vz * m;
+        const double wx = a.vx - vr[0], wy = a.vy - vr[1], wz = a.vz - vr[2];
+        part[S_MV2] += m * ((wx * wx + wy * wy) + wz * wz);
+        part[S_POT] += d.pot[s];
+        part[S_VIR] += d.vir[s];
+        part[S_WV] = fmax(part[S_WV], (a.vx * a.vx + a.vy * a.vy) + a.vz * a.vz);
+        part[S_WA] = fmax(part[S_WA], ((a.fx * a.fx + a.fy * a.fy) + a.fz * a.fz) / (m * m));
+    }
+    partial_store<BS>(d, part, b, kColsState);
+    prof_block(d, P_STEP, t_start, true, 0);
+}
+
 // ---------------------------------------------------------------- finalize
 
 __device__ __forceinline__ void thermo(const double* S, const GroupInfo& G, const double* box,
@@ -2204,6 +2424,27 @@ hipError_t launch_allpairs(const DevState& d, int bs, bool force_only, hipStream
         if (multi) hipLaunchKernelGGL((k_allpairs<B, true, false>), dim3(d.n_blocks), dim3(B), 0, st, d); \
         else hipLaunchKernelGGL((k_allpairs<B, false, false>), dim3(d.n_blocks), dim3(B), 0, st, d);      \
     }
+    MD_BS_SWITCH(bs, L)
+#undef L
+    return hipGetLastError();
+}
+
+hipError_t launch_ap_force(const DevState& d, int bs, bool force_only, hipStream_t st) {
+    const bool multi = d.n_types > 1;
+    if (d.n_blocks <= 0) return hipSuccess;
+    const dim3 grid((unsigned)(d.n_blocks * (bs / kApIT)));
+    if (force_only) {
+        if (multi) hipLaunchKernelGGL((k_ap_force<true, true>), grid, dim3(kApBS), 0, st, d, bs);
+        else hipLaunchKernelGGL((k_ap_force<false, true>), grid, dim3(kApBS), 0, st, d, bs);
+    } else {
+        if (multi) hipLaunchKernelGGL((k_ap_force<true, false>), grid, dim3(kApBS), 0, st, d, bs);
+        else hipLaunchKernelGGL((k_ap_force<false, false>), grid, dim3(kApBS), 0, st, d, bs);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_ap_finish(const DevState& d, int bs, hipStream_t st) {
+#define L(B) hipLaunchKernelGGL((k_ap_finish<B>), dim3(d.n_blocks), dim3(B), 0, st, d);
     MD_BS_SWITCH(bs, L)
 #undef L
     return hipGetLastError();
