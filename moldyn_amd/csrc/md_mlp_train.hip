@@ -17,8 +17,10 @@
 //              + T V1 silu''(A1), dW2 = G2^T H1 + D2^T PP, dW1 = G1^T X + D1^T U~,
 //              db2 = sum G2, db1 = sum G1, dw3 = sum (V2 silu'(A2) + dy H2), db3 = sum dy,
 //   update     Adam.
-// Matrix products run on one tiled SGEMM kernel (NN, NT and TN forms, split-K
-// partial sums added in a fixed order for the parameter gradients).
+// The network runs in two kernels on the FP32 matrix cores, k_tr_net (forward
+// and force backward) and k_tr_net_grad (double backward and parameter
+// gradients); between them only the pre-activations A1, A2 and T go through
+// memory.  The blocks' gradients are added in a fixed order.
 #include "md_common.h"
 #include "md_train.h"
 
@@ -26,91 +28,381 @@ namespace md {
 
 constexpr float kPiT = 3.14159265358979323846f;
 
-__device__ __forceinline__ void silu3(float a, float& h, float& d1, float& d2) {
+// silu(a) and its first two derivatives
+struct Silu3 {
+    float h, d1, d2;
+};
+__device__ __forceinline__ Silu3 silu3(float a) {
     const float s = 1.0f / (1.0f + expf(-a));
-    h = a * s;
-    d1 = s * (1.0f + a * (1.0f - s));
-    d2 = s * (1.0f - s) * (2.0f + a * (1.0f - 2.0f * s));
+    return {a * s, s * (1.0f + a * (1.0f - s)), s * (1.0f - s) * (2.0f + a * (1.0f - 2.0f * s))};
 }
 
-// ---------------------------------------------------------------- SGEMM
+// ---------------------------------------------------------------- network (FP32 MFMA)
+//
+// A block of eight waves takes tiles of 32 rows (atoms); wave w owns columns
+// 16 w .. 16 w + 15 of every 128-column matrix, and its slices of the weights
+// stay in its registers as matrix operands over all tiles.  The rows' matrices
+// pass from layer to layer through LDS.  Tiles of 64 rows spill registers in
+// k_tr_net_grad (65,536 rows: 162 us, 128 us with 32) and leave CUs idle on
+// small minibatches (6,655 rows: 44 and 25 us).
+// What bounds them is the FP32 matrix rate with the SiLU evaluations between
+// the products (two waves per SIMD: the products and the elementwise work
+// overlap little): 65,536 rows take 76 us (82 kFLOP a row, 71 TFLOP/s) and 128 us
+// (155 kFLOP, 79 TFLOP/s) of the 154 TFLOP/s a large FP32 product reaches here.
+// Before, a tiled FP32 product on the vector units per layer with elementwise
+// passes in between and the weight gradients in 128 splits: 1.93 ms per
+// minibatch of 65,536 rows in all, 0.44 ms now.
+// v_mfma_f32_16x16x4_f32, lane l = 16 g + c: operand A holds row c, operand B
+// column c, both at the k of lane group g; the result holds rows 4 g + i
+// (i = 0..3) of column c.  The k of a product may come in any order that A and
+// B share: four products in a row take k = 16 kk + 4 g + i, so that a lane reads
+// its four A values as one 16-byte word of a row.
+// LDS rows are 132 (36) words apart: the 16-byte reads of 16 rows, and the
+// 4-byte accesses of rows 4 g + i, each fall on all 64 banks.
+// A1, A2 and T are stored as the result fragments lie in the registers (16
+// bytes a lane, consecutive lanes on consecutive words), for k_tr_net_grad to
+// read in the same way.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kTrBS = 512, kTrW = kTrBS / 64;
+constexpr int kLdH = kMlpH + 4, kLdX = kMlpK + 4;
 
-// C[z] = alpha op(A) op(B) + beta C[z] over K range [z kc, (z + 1) kc);
-// op(A) is M x K (TA: A stored K x M), op(B) is K x N (TB: B stored N x K).
-constexpr int kGB = 64, kGK = 16;
-template <bool TA, bool TB>
-__global__ __launch_bounds__(256) void k_sgemm(int M, int N, int K, int kc, float alpha, const float* __restrict__ A,
-                                               int lda, const float* __restrict__ B, int ldb, float beta,
-                                               float* __restrict__ C, int ldc, int64_t c_split) {
-    __shared__ float As[kGK][kGB + 4];
-    __shared__ float Bs[kGK][kGB + 4];
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-    const int m0 = blockIdx.y * kGB, n0 = blockIdx.x * kGB;
-    const int k_lo = blockIdx.z * kc;
-    const int k_hi = min(K, k_lo + kc);
-    float acc[4][4] = {};
-    for (int k0 = k_lo; k0 < k_hi; k0 += kGK) {
-        for (int e = threadIdx.x; e < kGB * kGK; e += 256) {
-            // A tile: element (m, k)
-            int m, k;
-            if (TA) {
-                k = e / kGB;
-                m = e % kGB;
-            } else {
-                m = e / kGK;
-                k = e % kGK;
-            }
-            const int gm = m0 + m, gk = k0 + k;
-            As[k][m] = (gm < M && gk < k_hi) ? (TA ? A[(int64_t)gk * lda + gm] : A[(int64_t)gm * lda + gk]) : 0.0f;
-            int n, kb;
-            if (TB) {
-                n = e / kGK;
-                kb = e % kGK;
-            } else {
-                kb = e / kGB;
-                n = e % kGB;
-            }
-            const int gn = n0 + n, gkb = k0 + kb;
-            Bs[kb][n] = (gn < N && gkb < k_hi) ? (TB ? B[(int64_t)gn * ldb + gkb] : B[(int64_t)gkb * ldb + gn]) : 0.0f;
+// acc[t] += rows 16 t .. of `act` (LDS, stride LD, K = 16 KK columns) times the
+// wave's weight slice
+template <int KK, int LD, int TT>
+__device__ __forceinline__ void tile_gemm(const float* act, const f32x4 (&wgt)[KK], f32x4 (&acc)[TT]) {
+    const int c = threadIdx.x & 15, g = (threadIdx.x >> 4) & 3;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+            const f32x4 a = *reinterpret_cast<const f32x4*>(act + (16 * t + c) * LD + 16 * kk + 4 * g);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], wgt[kk][i], acc[t], 0, 0, 0);
         }
-        __syncthreads();
+}
+
+// acc[ct] += (columns m0 .. m0 + 15 of P)^T times columns 16 ct .. of Q, over
+// the tile's TR rows (both in LDS)
+template <int TR, int LDP, int LDQ, int CT>
+__device__ __forceinline__ void tile_outer(const float* P, int m0, const float* Q, f32x4 (&acc)[CT]) {
+    const int c = threadIdx.x & 15, g = (threadIdx.x >> 4) & 3;
 #pragma unroll
-        for (int k = 0; k < kGK; ++k) {
-            float a[4], b[4];
+    for (int kk = 0; kk < TR / 16; ++kk)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[k][ty + 16 * i];
+        for (int i = 0; i < 4; ++i) {
+            const int r = 16 * kk + 4 * g + i;
+            const float a = P[r * LDP + m0 + c];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[k][tx + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+            for (int ct = 0; ct < CT; ++ct)
+                acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, Q[r * LDQ + 16 * ct + c], acc[ct], 0, 0, 0);
         }
-        __syncthreads();
+}
+
+// a result fragment into rows 16 t + 4 g + i, column n of an LDS matrix
+template <int LD>
+__device__ __forceinline__ void frag_to_lds(float* m, int t, int n, const f32x4& v) {
+    const int g = (threadIdx.x >> 4) & 3;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m[(16 * t + 4 * g + i) * LD + n] = v[i];
+}
+
+// the weight slice B[k][n] = W[n * ldn + k * ldk], k = 16 kk + 4 g + i
+template <int KK>
+__device__ __forceinline__ void load_slice(f32x4 (&wgt)[KK], const float* W, int n, int ldn, int ldk) {
+    const int g = (threadIdx.x >> 4) & 3;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) wgt[kk][i] = W[n * ldn + (16 * kk + 4 * g + i) * ldk];
+}
+
+// normalised features of the tile's rows (0 past the last)
+__device__ __forceinline__ void stage_x(const TrainState& t, int64_t row0, int64_t M, float* sx) {
+    for (int e = threadIdx.x; e < kTrRows * (kMlpK / 4); e += kTrBS) {
+        const int r = e / (kMlpK / 4), k = 4 * (e % (kMlpK / 4));
+        f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
+        const int64_t row = row0 + r;
+        if (row < M) {
+            const int64_t b = row / t.n_atoms, i = row - b * t.n_atoms;
+            x = *reinterpret_cast<const f32x4*>(t.G + ((int64_t)t.bf[b] * t.n_atoms + i) * kMlpK + k);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) x[q] = (x[q] - t.g_mean[k + q]) * t.g_inv_std[k + q];
+        }
+        *reinterpret_cast<f32x4*>(sx + r * kLdX + k) = x;
     }
-    float* Cz = C + blockIdx.z * c_split;
+}
+
+// Forward, and the backward to dE/dG: E and Gam of the M rows; `keep` stores
+// A1, A2 and T for k_tr_net_grad.
+__global__ __launch_bounds__(kTrBS) void k_tr_net(TrainState t, int64_t M, int64_t n_tiles, int keep) {
+    constexpr int TR = kTrRows, TT = TR / 16;
+    __shared__ __align__(16) float sx[TR * kLdX], sh[TR * kLdH], sd[TR * kLdH];
+    __shared__ float sy[kTrW][TR];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+    const int n = 16 * w + c;
+    const float* th = t.theta;
+    f32x4 w1t[2], w2t[8], w2[8], w1[8];
+    load_slice(w1t, th + kMlpOffW1, n, kMlpK, 1);
+    load_slice(w2t, th + kMlpOffW2, n, kMlpH, 1);
+    load_slice(w2, th + kMlpOffW2, n, 1, kMlpH);
+    load_slice(w1, th + kMlpOffW1, 16 * (w & 1) + c, 1, kMlpK);
+    const float b1 = th[kMlpOffB1 + n], b2 = th[kMlpOffB2 + n], w3 = th[kMlpOffW3 + n];
+    const float gsc = t.e_scale * t.g_inv_std[16 * (w & 1) + c];
+    for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+        const int64_t row0 = tile * TR;
+        const int64_t fo = (tile * kTrW + w) * TT * 64 + lane;  // this lane's words of the tile's fragments
+        stage_x(t, row0, M, sx);
+        __syncthreads();
+        f32x4 s1[TT];
+        {
+            f32x4 a[TT];
+#pragma unroll
+            for (int q = 0; q < TT; ++q) a[q] = f32x4{b1, b1, b1, b1};
+            tile_gemm<2, kLdX, TT>(sx, w1t, a);
+#pragma unroll
+            for (int q = 0; q < TT; ++q) {
+                if (keep) reinterpret_cast<f32x4*>(t.A1)[fo + q * 64] = a[q];
+                f32x4 h;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const Silu3 f = silu3(a[q][i]);
+                    h[i] = f.h;
+                    s1[q][i] = f.d1;
+                }
+                frag_to_lds<kLdH>(sh, q, n, h);
+            }
+        }
+        __syncthreads();
+        {
+            f32x4 a[TT];
+#pragma unroll
+            for (int q = 0; q < TT; ++q) a[q] = f32x4{b2, b2, b2, b2};
+            tile_gemm<8, kLdH, TT>(sh, w2t, a);
+#pragma unroll
+            for (int q = 0; q < TT; ++q) {
+                if (keep) reinterpret_cast<f32x4*>(t.A2)[fo + q * 64] = a[q];
+                f32x4 d, y;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const Silu3 f = silu3(a[q][i]);
+                    d[i] = w3 * f.d1;
+                    y[i] = w3 * f.h;
+                }
+                frag_to_lds<kLdH>(sd, q, n, d);
+                // the wave's 16 columns of each row's y
+#pragma unroll
+                for (int o = 1; o < 16; o <<= 1)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) y[i] += __shfl_xor(y[i], o, 16);
+                if (c == 0)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) sy[w][16 * q + 4 * g + i] = y[i];
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x < TR && row0 + threadIdx.x < M) {
+            float y = th[kMlpOffB3];
+#pragma unroll
+            for (int q = 0; q < kTrW; ++q) y += sy[q][threadIdx.x];
+            t.E[row0 + threadIdx.x] = t.e_scale * y + t.e_shift;
+        }
+        {
+            f32x4 a[TT];
+#pragma unroll
+            for (int q = 0; q < TT; ++q) a[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            tile_gemm<8, kLdH, TT>(sd, w2, a);
+#pragma unroll
+            for (int q = 0; q < TT; ++q) {
+                if (keep) reinterpret_cast<f32x4*>(t.T)[fo + q * 64] = a[q];
+                frag_to_lds<kLdH>(sh, q, n, a[q] * s1[q]);
+            }
+        }
+        __syncthreads();
+        // 2 TT tiles of 16 x 16: wave w takes column half w % 2 of row tiles
+        // w / 2, w / 2 + 4, ...
+        for (int q = w >> 1; q < TT; q += kTrW / 2) {
+            f32x4 a[1] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+            tile_gemm<8, kLdH, 1>(sh + 16 * q * kLdH, w1, a);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int64_t row = row0 + 16 * q + 4 * g + i;
+                if (row < M) t.Gam[row * kMlpK + 16 * (w & 1) + c] = gsc * a[0][i];
+            }
+        }
+    }
+}
+
+// Gradient of the loss through E (dy) and through dE/dG (U, the adjoint of
+// Gam), summed over the block's rows: parameters in theta's order at
+// gpart[block][kMlpNP].  Rows past M add nothing: their U, X and dy are 0.
+__global__ __launch_bounds__(kTrBS) void k_tr_net_grad(TrainState t, int64_t M, int64_t n_tiles) {
+    constexpr int TR = kTrRows, TT = TR / 16;
+    __shared__ __align__(16) float su[TR * kLdX], sx[TR * kLdX];
+    __shared__ __align__(16) float sp[TR * kLdH], sh[TR * kLdH], sg[TR * kLdH], sd[TR * kLdH];
+    __shared__ float sdy[TR];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+    const int n = 16 * w + c;
+    const float* th = t.theta;
+    f32x4 w1t[2], w2t[8], w2[8];
+    load_slice(w1t, th + kMlpOffW1, n, kMlpK, 1);
+    load_slice(w2t, th + kMlpOffW2, n, kMlpH, 1);
+    load_slice(w2, th + kMlpOffW2, n, 1, kMlpH);
+    const float w3 = th[kMlpOffW3 + n];
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 gw2[8], gw1[2];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) gw2[q] = zero;
+    gw1[0] = gw1[1] = zero;
+    float gw3 = 0.0f, gb2 = 0.0f, gb1 = 0.0f, gb3 = 0.0f;
+    for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+        const int64_t row0 = tile * TR;
+        const int64_t fo = (tile * kTrW + w) * TT * 64 + lane;
+        __syncthreads();  // the last tile's reads of su, sx, sg and sh
+        stage_x(t, row0, M, sx);
+        for (int e = threadIdx.x; e < TR * (kMlpK / 4); e += kTrBS) {
+            const int r = e / (kMlpK / 4), k = 4 * (e % (kMlpK / 4));
+            f32x4 u = zero;
+            if (row0 + r < M) {
+                u = *reinterpret_cast<const f32x4*>(t.U + (row0 + r) * kMlpK + k);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) u[q] *= t.e_scale * t.g_inv_std[k + q];
+            }
+            *reinterpret_cast<f32x4*>(su + r * kLdX + k) = u;
+        }
+        if (threadIdx.x < TR) {
+            const float dy = row0 + threadIdx.x < M ? t.dy[row0 + threadIdx.x] : 0.0f;
+            sdy[threadIdx.x] = dy;
+            gb3 += dy;
+        }
+        __syncthreads();
+        f32x4 s1[TT], q1[TT], d1[TT];  // silu'(A1), T V1 silu''(A1), D1
+        {
+            f32x4 v[TT];
+#pragma unroll
+            for (int q = 0; q < TT; ++q) v[q] = zero;
+            tile_gemm<2, kLdX, TT>(su, w1t, v);  // V1 = Ut W1^T
+#pragma unroll
+            for (int q = 0; q < TT; ++q) {
+                const f32x4 a = reinterpret_cast<const f32x4*>(t.A1)[fo + q * 64];
+                const f32x4 tt = reinterpret_cast<const f32x4*>(t.T)[fo + q * 64];
+                f32x4 h;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const Silu3 f = silu3(a[i]);
+                    h[i] = f.h;
+                    s1[q][i] = f.d1;
+                    q1[q][i] = tt[i] * v[q][i] * f.d2;
+                    d1[q][i] = tt[i] * s1[q][i];
+                }
+                frag_to_lds<kLdH>(sh, q, n, h);
+                frag_to_lds<kLdH>(sp, q, n, v[q] * s1[q]);  // PP
+            }
+        }
+        __syncthreads();
+        {
+            f32x4 v[TT];
+#pragma unroll
+            for (int q = 0; q < TT; ++q) v[q] = zero;
+            tile_gemm<8, kLdH, TT>(sp, w2t, v);  // V2 = PP W2^T
+#pragma unroll
+            for (int q = 0; q < TT; ++q) {
+                const f32x4 a = reinterpret_cast<const f32x4*>(t.A2)[fo + q * 64];
+                f32x4 g2, d2;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const Silu3 f = silu3(a[i]);
+                    const float dy = sdy[16 * q + 4 * g + i];
+                    d2[i] = w3 * f.d1;
+                    g2[i] = v[q][i] * w3 * f.d2 + dy * d2[i];
+                    gw3 += v[q][i] * f.d1 + dy * f.h;
+                    gb2 += g2[i];
+                }
+                frag_to_lds<kLdH>(sg, q, n, g2);
+                frag_to_lds<kLdH>(sd, q, n, d2);
+            }
+        }
+        __syncthreads();
+        // dW2 += G2^T H1 + D2^T PP
+        tile_outer<TR, kLdH, kLdH, 8>(sg, 16 * w, sh, gw2);
+        tile_outer<TR, kLdH, kLdH, 8>(sd, 16 * w, sp, gw2);
+        {
+            f32x4 v[TT];
+#pragma unroll
+            for (int q = 0; q < TT; ++q) v[q] = zero;
+            tile_gemm<8, kLdH, TT>(sg, w2, v);  // G2 W2
+            __syncthreads();                    // sg and sh are read: G1 and D1 take their place
+#pragma unroll
+            for (int q = 0; q < TT; ++q) {
+                f32x4 g1;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    g1[i] = v[q][i] * s1[q][i] + q1[q][i];
+                    gb1 += g1[i];
+                }
+                frag_to_lds<kLdH>(sg, q, n, g1);
+                frag_to_lds<kLdH>(sh, q, n, d1[q]);
+            }
+        }
+        __syncthreads();
+        // dW1 += G1^T X + D1^T Ut
+        tile_outer<TR, kLdH, kLdX, 2>(sg, 16 * w, sx, gw1);
+        tile_outer<TR, kLdH, kLdX, 2>(sh, 16 * w, su, gw1);
+    }
+    float* out = t.gpart + (int64_t)blockIdx.x * kMlpNP;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int gm = m0 + ty + 16 * i;
-        if (gm >= M) continue;
+        const int m = 16 * w + 4 * g + i;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int gn = n0 + tx + 16 * j;
-            if (gn >= N) continue;
-            float* cp = Cz + (int64_t)gm * ldc + gn;
-            *cp = alpha * acc[i][j] + (beta != 0.0f ? beta * *cp : 0.0f);
-        }
+        for (int ct = 0; ct < 8; ++ct) out[kMlpOffW2 + m * kMlpH + 16 * ct + c] = gw2[ct][i];
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct) out[kMlpOffW1 + m * kMlpK + 16 * ct + c] = gw1[ct][i];
+    }
+    // column sums over the four lane groups
+#pragma unroll
+    for (int o = 16; o < 64; o <<= 1) {
+        gw3 += __shfl_xor(gw3, o, 64);
+        gb2 += __shfl_xor(gb2, o, 64);
+        gb1 += __shfl_xor(gb1, o, 64);
+    }
+    if (g == 0) {
+        out[kMlpOffW3 + n] = gw3;
+        out[kMlpOffB2 + n] = gb2;
+        out[kMlpOffB1 + n] = gb1;
+    }
+    if (w == 0) {  // threads < TR took the rows' dy
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) gb3 += __shfl_xor(gb3, o, 64);
+        if (lane == 0) out[kMlpOffB3] = gb3;
     }
 }
 
-// out[i] (+)= sum_z part[z][i] in split order
-__global__ __launch_bounds__(256) void k_split_sum(const float* __restrict__ part, int splits, int64_t n,
-                                                   float* __restrict__ out, int accumulate) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.0f;
-    for (int z = 0; z < splits; ++z) s += part[(int64_t)z * n + i];
-    out[i] = accumulate ? out[i] + s : s;
+// The blocks' gradients added in block order, four interleaved FP64 sums per
+// parameter, then what the caller asked for: stored (accumulate 0) or added
+// (accumulate 1) to t.grad, or one Adam step on theta (adam).
+struct AdamArgs {
+    float lr, b1, b2, eps, c1, c2;  // c1 = 1 - b1^step, c2 = 1 - b2^step
+};
+template <bool ADAM>
+__global__ __launch_bounds__(256) void k_tr_grad_sum(TrainState t, int nb, int accumulate, AdamArgs a) {
+    __shared__ double s[4][64];
+    const int q = threadIdx.x >> 6, p = blockIdx.x * 64 + (threadIdx.x & 63);
+    double v = 0.0;
+    if (p < kMlpNP)
+#pragma unroll 8
+        for (int b = q; b < nb; b += 4) v += (double)t.gpart[(int64_t)b * kMlpNP + p];
+    s[q][threadIdx.x & 63] = v;
+    __syncthreads();
+    if (q != 0 || p >= kMlpNP) return;
+    const float gi = (float)((s[0][threadIdx.x] + s[1][threadIdx.x]) + (s[2][threadIdx.x] + s[3][threadIdx.x]));
+    if (!ADAM) {
+        t.grad[p] = accumulate ? t.grad[p] + gi : gi;
+        return;
+    }
+    const float mi = a.b1 * t.adam_m[p] + (1.0f - a.b1) * gi;
+    const float vi = a.b2 * t.adam_v[p] + (1.0f - a.b2) * gi * gi;
+    t.adam_m[p] = mi;
+    t.adam_v[p] = vi;
+    t.theta[p] -= a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
 }
 
 // ---------------------------------------------------------------- pairs, features
@@ -253,77 +545,6 @@ __global__ __launch_bounds__(256) void k_tr_feature_stats(TrainState t, int64_t 
     }
 }
 
-// ---------------------------------------------------------------- elementwise
-
-// X = (G - mean) inv_std for the M rows of the minibatch (slot b = frame bf[b])
-__global__ __launch_bounds__(256) void k_tr_normalize(TrainState t, int64_t M) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= M * kMlpK) return;
-    const int k = (int)(e % kMlpK);
-    const int64_t r = e / kMlpK;
-    const int64_t b = r / t.n_atoms, i = r % t.n_atoms;
-    const int64_t src = ((int64_t)t.bf[b] * t.n_atoms + i) * kMlpK + k;
-    t.X[e] = (t.G[src] - t.g_mean[k]) * t.g_inv_std[k];
-}
-
-// layer activations: H = silu(A + b), S = silu', Sp = silu'' (in place over A -> H)
-__global__ __launch_bounds__(256) void k_tr_act(int64_t M, const float* __restrict__ b, float* __restrict__ AH,
-                                                float* __restrict__ S, float* __restrict__ Sp) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= M * kMlpH) return;
-    float h, d1, d2;
-    silu3(AH[e] + b[e % kMlpH], h, d1, d2);
-    AH[e] = h;
-    S[e] = d1;
-    Sp[e] = d2;
-}
-
-// per row: y = H2 . w3 + b3, E = e_scale y + e_shift; D2 = w3 * S2
-__global__ __launch_bounds__(256) void k_tr_head(TrainState t, int64_t M) {
-    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (r >= M) return;
-    const float* w3 = t.theta + kMlpOffW3;
-    float y = t.theta[kMlpOffB3];
-    for (int m = 0; m < kMlpH; ++m) {
-        y = fmaf(t.H2[r * kMlpH + m], w3[m], y);
-        t.D2[r * kMlpH + m] = w3[m] * t.S2[r * kMlpH + m];
-    }
-    t.E[r] = t.e_scale * y + t.e_shift;
-}
-
-// D1 = T * S1
-__global__ __launch_bounds__(256) void k_tr_mul(int64_t n, const float* __restrict__ a, const float* __restrict__ b,
-                                                float* __restrict__ out) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e < n) out[e] = a[e] * b[e];
-}
-
-// Gam = e_scale inv_std GX (in place), Ut likewise for U
-__global__ __launch_bounds__(256) void k_tr_scale_in(TrainState t, int64_t M, float* __restrict__ v) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= M * kMlpK) return;
-    v[e] *= t.e_scale * t.g_inv_std[e % kMlpK];
-}
-
-// G2 = V2 w3 S2p + dy D2 (V2 in place -> G2), and the w3 gradient terms
-// W3T = V2 S2 + dy H2 (row-wise, summed later)
-__global__ __launch_bounds__(256) void k_tr_g2(TrainState t, int64_t M) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= M * kMlpH) return;
-    const int m = (int)(e % kMlpH);
-    const int64_t r = e / kMlpH;
-    const float v2 = t.V2[e], dy = t.dy[r];
-    t.W3T[e] = v2 * t.S2[e] + dy * t.H2[e];
-    t.V2[e] = v2 * t.theta[kMlpOffW3 + m] * t.S2p[e] + dy * t.D2[e];
-}
-
-// G1 = R1a * S1 + T * V1 * S1p (R1a in place -> G1); PP = V1 * S1 computed earlier
-__global__ __launch_bounds__(256) void k_tr_g1(TrainState t, int64_t M) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= M * kMlpH) return;
-    t.R1[e] = t.R1[e] * t.S1[e] + t.T[e] * t.V1[e] * t.S1p[e];
-}
-
 // ---------------------------------------------------------------- pair kernels
 
 // Forces of the minibatch frames from Gam (rows r = b n + i), the loss terms
@@ -437,62 +658,9 @@ __global__ __launch_bounds__(256) void k_tr_u(TrainState t) {
     for (int k = 0; k < kMlpK; ++k) t.U[ri * kMlpK + k] = u[k];
 }
 
-// column sums of an M x ncol matrix into out[0..ncol) (block partials, fixed order)
-__global__ __launch_bounds__(256) void k_tr_colsum(const float* __restrict__ A, int64_t M, int ncol,
-                                                   float* __restrict__ part) {
-    // block b sums rows [b * rows_per, ...) for column threadIdx.x (ncol <= 256)
-    const int c = threadIdx.x;
-    if (c >= ncol) return;
-    const int64_t per = (M + gridDim.x - 1) / gridDim.x;
-    const int64_t r0 = (int64_t)blockIdx.x * per, r1 = min(M, r0 + per);
-    float s = 0.0f;
-    for (int64_t r = r0; r < r1; ++r) s += A[r * ncol + c];
-    part[(int64_t)blockIdx.x * ncol + c] = s;
-}
-
-// Adam on the flat parameter vector; the step count t is 1-based.
-__global__ __launch_bounds__(256) void k_tr_adam(float* __restrict__ theta, const float* __restrict__ g,
-                                                 float* __restrict__ m, float* __restrict__ v, int n, float lr,
-                                                 float b1, float b2, float eps, int step) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float mh = mi / (1.0f - powf(b1, (float)step));
-    const float vh = vi / (1.0f - powf(b2, (float)step));
-    theta[i] -= lr * mh / (sqrtf(vh) + eps);
-}
-
 // ---------------------------------------------------------------- launchers
 
 static inline unsigned nblk(int64_t n) { return (unsigned)((n + 255) / 256); }
-
-hipError_t tr_gemm(bool ta, bool tb, int M, int N, int K, float alpha, const float* A, int lda, const float* B,
-                   int ldb, float beta, float* C, int ldc, int splits, hipStream_t st) {
-    if (splits < 1) splits = 1;
-    const int kc = ((K + splits - 1) / splits + kGK - 1) / kGK * kGK;
-    splits = (K + kc - 1) / kc;
-    const dim3 grid((N + kGB - 1) / kGB, (M + kGB - 1) / kGB, splits);
-    const int64_t cs = (int64_t)M * ldc;
-    if (!ta && !tb) hipLaunchKernelGGL((k_sgemm<false, false>), grid, dim3(256), 0, st, M, N, K, kc, alpha, A, lda, B, ldb, beta, C, ldc, cs);
-    if (!ta && tb) hipLaunchKernelGGL((k_sgemm<false, true>), grid, dim3(256), 0, st, M, N, K, kc, alpha, A, lda, B, ldb, beta, C, ldc, cs);
-    if (ta && !tb) hipLaunchKernelGGL((k_sgemm<true, false>), grid, dim3(256), 0, st, M, N, K, kc, alpha, A, lda, B, ldb, beta, C, ldc, cs);
-    if (ta && tb) hipLaunchKernelGGL((k_sgemm<true, true>), grid, dim3(256), 0, st, M, N, K, kc, alpha, A, lda, B, ldb, beta, C, ldc, cs);
-    return hipGetLastError();
-}
-
-int tr_gemm_splits(int K, int splits) {
-    const int kc = ((K + splits - 1) / splits + kGK - 1) / kGK * kGK;
-    return (K + kc - 1) / kc;
-}
-
-hipError_t tr_split_sum(const float* part, int splits, int64_t n, float* out, bool accumulate, hipStream_t st) {
-    hipLaunchKernelGGL(k_split_sum, dim3(nblk(n)), dim3(256), 0, st, part, splits, n, out, accumulate ? 1 : 0);
-    return hipGetLastError();
-}
 
 hipError_t tr_count_pairs(const TrainState& t, int f0, int nf, int32_t* max_cnt, hipStream_t st) {
     hipLaunchKernelGGL(k_tr_count, dim3(nblk(t.n_atoms), nf), dim3(256), 0, st, t, f0, nf, max_cnt);
@@ -514,23 +682,10 @@ hipError_t tr_feature_stats(const TrainState& t, int64_t rows, double* part, int
     return hipGetLastError();
 }
 
-hipError_t tr_forward_backward(const TrainState& t, int nf, hipStream_t st) {
-    hipError_t e;
-    const float* th = t.theta;
-    const int64_t M = (int64_t)nf * t.n_atoms;
-    hipLaunchKernelGGL(k_tr_normalize, dim3(nblk(M * kMlpK)), dim3(256), 0, st, t, M);
-    // A1 = X W1^T -> H1
-    if ((e = tr_gemm(false, true, (int)M, kMlpH, kMlpK, 1.f, t.X, kMlpK, th + kMlpOffW1, kMlpK, 0.f, t.H1, kMlpH, 1, st))) return e;
-    hipLaunchKernelGGL(k_tr_act, dim3(nblk(M * kMlpH)), dim3(256), 0, st, M, th + kMlpOffB1, t.H1, t.S1, t.S1p);
-    // A2 = H1 W2^T -> H2
-    if ((e = tr_gemm(false, true, (int)M, kMlpH, kMlpH, 1.f, t.H1, kMlpH, th + kMlpOffW2, kMlpH, 0.f, t.H2, kMlpH, 1, st))) return e;
-    hipLaunchKernelGGL(k_tr_act, dim3(nblk(M * kMlpH)), dim3(256), 0, st, M, th + kMlpOffB2, t.H2, t.S2, t.S2p);
-    hipLaunchKernelGGL(k_tr_head, dim3(nblk(M)), dim3(256), 0, st, t, M);
-    // T = D2 W2, D1 = T S1, Gam = e_scale inv_std (D1 W1)
-    if ((e = tr_gemm(false, false, (int)M, kMlpH, kMlpH, 1.f, t.D2, kMlpH, th + kMlpOffW2, kMlpH, 0.f, t.T, kMlpH, 1, st))) return e;
-    hipLaunchKernelGGL(k_tr_mul, dim3(nblk(M * kMlpH)), dim3(256), 0, st, M * kMlpH, t.T, t.S1, t.D1);
-    if ((e = tr_gemm(false, false, (int)M, kMlpK, kMlpH, 1.f, t.D1, kMlpH, th + kMlpOffW1, kMlpK, 0.f, t.Gam, kMlpK, 1, st))) return e;
-    hipLaunchKernelGGL(k_tr_scale_in, dim3(nblk(M * kMlpK)), dim3(256), 0, st, t, M, t.Gam);
+hipError_t tr_forward_backward(const TrainState& t, int nf, bool keep, hipStream_t st) {
+    const int64_t M = (int64_t)nf * t.n_atoms, tiles = (M + kTrRows - 1) / kTrRows;
+    hipLaunchKernelGGL(k_tr_net, dim3((unsigned)(tiles < t.n_cu ? tiles : t.n_cu)), dim3(kTrBS), 0, st, t, M, tiles,
+                       keep ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -544,50 +699,25 @@ hipError_t tr_loss_sum(const TrainState& t, int nf, const double* loss_part, dou
     return hipGetLastError();
 }
 
-// Gradient of the minibatch loss added into t.grad (which the caller clears).
-hipError_t tr_gradient(const TrainState& t, int nf, hipStream_t st) {
-    hipError_t e;
-    const float* th = t.theta;
+// Gradient of the minibatch loss: the blocks' sums at t.gpart, their number in *parts.
+hipError_t tr_gradient(const TrainState& t, int nf, int* parts, hipStream_t st) {
     const int64_t M = (int64_t)nf * t.n_atoms;
     hipLaunchKernelGGL(k_tr_u, dim3(nblk(t.n_atoms), nf), dim3(256), 0, st, t);
-    hipLaunchKernelGGL(k_tr_scale_in, dim3(nblk(M * kMlpK)), dim3(256), 0, st, t, M, t.U);
-    // V1 = Ut W1^T, PP = V1 S1, V2 = PP W2^T
-    if ((e = tr_gemm(false, true, (int)M, kMlpH, kMlpK, 1.f, t.U, kMlpK, th + kMlpOffW1, kMlpK, 0.f, t.V1, kMlpH, 1, st))) return e;
-    hipLaunchKernelGGL(k_tr_mul, dim3(nblk(M * kMlpH)), dim3(256), 0, st, M * kMlpH, t.V1, t.S1, t.PP);
-    if ((e = tr_gemm(false, true, (int)M, kMlpH, kMlpH, 1.f, t.PP, kMlpH, th + kMlpOffW2, kMlpH, 0.f, t.V2, kMlpH, 1, st))) return e;
-    // G2 (in V2) and the w3 terms
-    hipLaunchKernelGGL(k_tr_g2, dim3(nblk(M * kMlpH)), dim3(256), 0, st, t, M);
-    // R1 = G2 W2, G1 (in R1)
-    if ((e = tr_gemm(false, false, (int)M, kMlpH, kMlpH, 1.f, t.V2, kMlpH, th + kMlpOffW2, kMlpH, 0.f, t.R1, kMlpH, 1, st))) return e;
-    hipLaunchKernelGGL(k_tr_g1, dim3(nblk(M * kMlpH)), dim3(256), 0, st, t, M);
-    // parameter gradients: split-K over the atoms, partial sums in split order
-    const int S = t.splits;
-    float* g = t.grad;
-    const int sW2 = tr_gemm_splits((int)M, S);
-    if ((e = tr_gemm(true, false, kMlpH, kMlpH, (int)M, 1.f, t.V2, kMlpH, t.H1, kMlpH, 0.f, t.gpart, kMlpH, S, st))) return e;
-    if ((e = tr_split_sum(t.gpart, sW2, kMlpH * kMlpH, g + kMlpOffW2, true, st))) return e;
-    if ((e = tr_gemm(true, false, kMlpH, kMlpH, (int)M, 1.f, t.D2, kMlpH, t.PP, kMlpH, 0.f, t.gpart, kMlpH, S, st))) return e;
-    if ((e = tr_split_sum(t.gpart, sW2, kMlpH * kMlpH, g + kMlpOffW2, true, st))) return e;
-    if ((e = tr_gemm(true, false, kMlpH, kMlpK, (int)M, 1.f, t.R1, kMlpH, t.X, kMlpK, 0.f, t.gpart, kMlpK, S, st))) return e;
-    if ((e = tr_split_sum(t.gpart, sW2, kMlpH * kMlpK, g + kMlpOffW1, true, st))) return e;
-    if ((e = tr_gemm(true, false, kMlpH, kMlpK, (int)M, 1.f, t.D1, kMlpH, t.U, kMlpK, 0.f, t.gpart, kMlpK, S, st))) return e;
-    if ((e = tr_split_sum(t.gpart, sW2, kMlpH * kMlpK, g + kMlpOffW1, true, st))) return e;
-    // bias and w3 gradients: column sums
-    const int cb = t.colsum_blocks;
-    hipLaunchKernelGGL(k_tr_colsum, dim3(cb), dim3(256), 0, st, t.V2, M, kMlpH, t.gpart);
-    if ((e = tr_split_sum(t.gpart, cb, kMlpH, g + kMlpOffB2, true, st))) return e;
-    hipLaunchKernelGGL(k_tr_colsum, dim3(cb), dim3(256), 0, st, t.R1, M, kMlpH, t.gpart);
-    if ((e = tr_split_sum(t.gpart, cb, kMlpH, g + kMlpOffB1, true, st))) return e;
-    hipLaunchKernelGGL(k_tr_colsum, dim3(cb), dim3(256), 0, st, t.W3T, M, kMlpH, t.gpart);
-    if ((e = tr_split_sum(t.gpart, cb, kMlpH, g + kMlpOffW3, true, st))) return e;
-    hipLaunchKernelGGL(k_tr_colsum, dim3(cb), dim3(256), 0, st, t.dy, M, 1, t.gpart);
-    if ((e = tr_split_sum(t.gpart, cb, 1, g + kMlpOffB3, true, st))) return e;
+    const int64_t tiles = (M + kTrRows - 1) / kTrRows;
+    *parts = (int)(tiles < t.n_cu ? tiles : t.n_cu);
+    hipLaunchKernelGGL(k_tr_net_grad, dim3(*parts), dim3(kTrBS), 0, st, t, M, tiles);
     return hipGetLastError();
 }
 
-hipError_t tr_adam(const TrainState& t, float lr, int step, hipStream_t st) {
-    hipLaunchKernelGGL(k_tr_adam, dim3(nblk(kMlpNP)), dim3(256), 0, st, t.theta, t.grad, t.adam_m, t.adam_v, kMlpNP, lr,
-                       0.9f, 0.999f, 1e-8f, step);
+hipError_t tr_grad_sum(const TrainState& t, int parts, bool accumulate, hipStream_t st) {
+    hipLaunchKernelGGL(k_tr_grad_sum<false>, dim3((kMlpNP + 63) / 64), dim3(256), 0, st, t, parts, accumulate ? 1 : 0,
+                       AdamArgs{});
+    return hipGetLastError();
+}
+
+hipError_t tr_adam(const TrainState& t, int parts, float lr, int step, hipStream_t st) {
+    const AdamArgs a{lr, 0.9f, 0.999f, 1e-8f, 1.0f - powf(0.9f, (float)step), 1.0f - powf(0.999f, (float)step)};
+    hipLaunchKernelGGL(k_tr_grad_sum<true>, dim3((kMlpNP + 63) / 64), dim3(256), 0, st, t, parts, 0, a);
     return hipGetLastError();
 }
 

@@ -6,6 +6,8 @@
 
 namespace md {
 
+constexpr int kTrRows = 32;  // rows (atoms) per tile of the network kernels
+
 struct TrainState {
     // data set: n_frames frames of n_atoms atoms
     const double* pos;    // n_frames x n_atoms x 3
@@ -32,13 +34,12 @@ struct TrainState {
     float* adam_m;
     float* adam_v;
     // minibatch work arrays (rows = atoms of the minibatch)
-    float *X, *Gam, *U;                                  // M x 32
-    float *H1, *S1, *S1p, *H2, *S2, *S2p;                // M x 128
-    float *D2, *T, *D1, *V1, *PP, *V2, *R1, *W3T;        // M x 128
-    float *E, *dy;                                       // M
-    float *F, *phi;                                      // M x 3
-    float* gpart;         // split-K / column-sum partials
-    int32_t splits, colsum_blocks;
+    float *Gam, *U;       // M x 32
+    float *A1, *A2, *T;   // M x 128 (rows up to a multiple of kTrRows), as matrix-core result fragments
+    float *E, *dy;        // M
+    float *F, *phi;       // M x 3
+    float* gpart;         // n_cu x kMlpNP gradients of blocks
+    int32_t n_cu;
 };
 
 hipError_t tr_count_pairs(const TrainState& t, int f0, int nf, int32_t* max_cnt, hipStream_t st);
@@ -46,12 +47,11 @@ hipError_t tr_fill_pairs(const TrainState& t, int f0, int nf, hipStream_t st);
 hipError_t tr_features(const TrainState& t, int f0, int nf, hipStream_t st);
 hipError_t tr_feature_stats(const TrainState& t, int64_t rows, double* part, int blocks, hipStream_t st);
 // minibatch of nf frames t.bf[0..nf): M = nf n_atoms rows
-hipError_t tr_forward_backward(const TrainState& t, int nf, hipStream_t st);
+hipError_t tr_forward_backward(const TrainState& t, int nf, bool keep, hipStream_t st);
 hipError_t tr_forces(const TrainState& t, int nf, double* loss_part, hipStream_t st);
 hipError_t tr_loss_sum(const TrainState& t, int nf, const double* loss_part, double* out, hipStream_t st);
-hipError_t tr_gradient(const TrainState& t, int nf, hipStream_t st);
-hipError_t tr_adam(const TrainState& t, float lr, int step, hipStream_t st);
-hipError_t tr_gemm(bool ta, bool tb, int M, int N, int K, float alpha, const float* A, int lda, const float* B,
-                   int ldb, float beta, float* C, int ldc, int splits, hipStream_t st);
+hipError_t tr_gradient(const TrainState& t, int nf, int* parts, hipStream_t st);
+hipError_t tr_grad_sum(const TrainState& t, int parts, bool accumulate, hipStream_t st);
+hipError_t tr_adam(const TrainState& t, int parts, float lr, int step, hipStream_t st);
 
 }  // namespace md

@@ -67,14 +67,14 @@ static int talloc_t(md_trainer* c, T** p, size_t n) {
 static int ensure_batch(md_trainer* c, int64_t rows) {
     if (rows <= c->batch_rows) return MD_OK;
     TrainState& t = c->t;
-    const size_t r = (size_t)rows;
+    const size_t r = (size_t)rows, rp = (r + kTrRows - 1) / kTrRows * kTrRows;
     int rc;
-    float** m32[] = {&t.X, &t.Gam, &t.U};
+    float** m32[] = {&t.Gam, &t.U};
     for (float** p : m32)
         if ((rc = talloc_t(c, p, r * kMlpK))) return rc;
-    float** m128[] = {&t.H1, &t.S1, &t.S1p, &t.H2, &t.S2, &t.S2p, &t.D2, &t.T, &t.D1, &t.V1, &t.PP, &t.V2, &t.R1, &t.W3T};
+    float** m128[] = {&t.A1, &t.A2, &t.T};
     for (float** p : m128)
-        if ((rc = talloc_t(c, p, r * kMlpH))) return rc;
+        if ((rc = talloc_t(c, p, rp * kMlpH))) return rc;
     if ((rc = talloc_t(c, &t.E, r))) return rc;
     if ((rc = talloc_t(c, &t.dy, r))) return rc;
     if ((rc = talloc_t(c, &t.F, r * 3))) return rc;
@@ -85,19 +85,20 @@ static int ensure_batch(md_trainer* c, int64_t rows) {
     return MD_OK;
 }
 
-// Forward, forces and (optionally) gradient of the nf frames frames[0..nf)
-// (device array); the summed squared energy and force errors go to
-// out[0..1] (device).  Nothing waits for the device.
-static int run_batch(md_trainer* c, const int32_t* frames, int nf, bool grad, double* out) {
+// Forward, forces and (with parts != NULL) the blocks' gradients of the nf
+// frames frames[0..nf) (device array), their number in *parts; the summed
+// squared energy and force errors go to out[0..1] (device).  Nothing waits for
+// the device.
+static int run_batch(md_trainer* c, const int32_t* frames, int nf, int* parts, double* out) {
     TrainState& t = c->t;
     const int64_t M = (int64_t)nf * t.n_atoms;
     int rc;
     if ((rc = ensure_batch(c, M))) return rc;
     t.bf = frames;
-    TCHK(c, tr_forward_backward(t, nf, c->st));
+    TCHK(c, tr_forward_backward(t, nf, parts != nullptr, c->st));
     TCHK(c, tr_forces(t, nf, c->loss_part, c->st));
     TCHK(c, tr_loss_sum(t, nf, c->loss_part, out, c->st));
-    if (grad) TCHK(c, tr_gradient(t, nf, c->st));
+    if (parts) TCHK(c, tr_gradient(t, nf, parts, c->st));
     return MD_OK;
 }
 
@@ -147,8 +148,13 @@ int md_trainer_create(md_trainer** out, int n_frames, int n_atoms, const double*
     t.inv_2w2 = (float)(1.0 / (2.0 * w * w));
     t.inv_w2 = (float)(1.0 / (w * w));
     t.e_scale = 1.0f;
-    t.splits = 128;
-    t.colsum_blocks = 256;
+    t.n_cu = 256;
+    {
+        int dev = 0, v = 0;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
+            t.n_cu = v;
+    }
     int rc;
     double *dpos, *dbox;
     float *de, *df;
@@ -159,7 +165,7 @@ int md_trainer_create(md_trainer** out, int n_frames, int n_atoms, const double*
         (rc = talloc_t(c, &de, na)) || (rc = talloc_t(c, &df, na * 3)) || (rc = talloc_t(c, &t.G, na * kMlpK)) ||
         (rc = talloc_t(c, &t.theta, kMlpNP)) || (rc = talloc_t(c, &t.grad, kMlpNP)) ||
         (rc = talloc_t(c, &t.adam_m, kMlpNP)) || (rc = talloc_t(c, &t.adam_v, kMlpNP)) ||
-        (rc = talloc_t(c, &t.gpart, (size_t)std::max(t.splits, t.colsum_blocks) * kMlpH * kMlpH)) ||
+        (rc = talloc_t(c, &t.gpart, (size_t)t.n_cu * kMlpNP)) ||
         (rc = talloc_t(c, &t.ncnt, na)) || (rc = talloc_t(c, &c->frames_seq, (size_t)n_frames)) ||
         (rc = talloc_t(c, &c->frames_ord, (size_t)n_frames)) ||
         (rc = talloc_t(c, &c->batch_loss, (size_t)2 * n_frames + 2))) {
@@ -276,12 +282,13 @@ int md_trainer_loss(md_trainer* c, double w_e, double w_f, int batch_frames, dou
     t.w_e = (float)w_e;
     t.w_f = (float)w_f;
     t.n_total = (int64_t)t.n_frames * t.n_atoms;
-    if (grad) TCHK(c, hipMemsetAsync(t.grad, 0, sizeof(float) * kMlpNP, c->st));
     int nb = 0;
     for (int f0 = 0; f0 < t.n_frames; f0 += batch_frames, ++nb) {
         const int nf = std::min(batch_frames, t.n_frames - f0);
-        int rc = run_batch(c, c->frames_seq + f0, nf, grad != nullptr, c->batch_loss + 2 * nb);
+        int parts = 0;
+        int rc = run_batch(c, c->frames_seq + f0, nf, grad ? &parts : nullptr, c->batch_loss + 2 * nb);
         if (rc) return rc;
+        if (grad) TCHK(c, tr_grad_sum(t, parts, nb > 0, c->st));
     }
     std::vector<double> bl;
     int rc = read_batch_loss(c, nb, bl);
@@ -324,10 +331,10 @@ int md_trainer_epoch(md_trainer* c, int batch_frames, double lr, double w_e, dou
         const int nf = std::min(batch_frames, t.n_frames - b0);
         t.n_total = (int64_t)nf * t.n_atoms;
         rows.push_back(t.n_total);
-        TCHK(c, hipMemsetAsync(t.grad, 0, sizeof(float) * kMlpNP, c->st));
-        int rc = run_batch(c, frames + b0, nf, true, c->batch_loss + 2 * nb);
+        int parts = 0;
+        int rc = run_batch(c, frames + b0, nf, &parts, c->batch_loss + 2 * nb);
         if (rc) return rc;
-        TCHK(c, tr_adam(t, (float)lr, ++c->step, c->st));
+        TCHK(c, tr_adam(t, parts, (float)lr, ++c->step, c->st));
     }
     std::vector<double> bl;
     int rc = read_batch_loss(c, nb, bl);
@@ -350,7 +357,7 @@ int md_trainer_predict(md_trainer* c, int frame, double* e_out, double* f_out) {
     if (!c || frame < 0 || frame >= c->t.n_frames) return tfail(c, MD_ERR_ARG, "bad argument");
     TrainState& t = c->t;
     t.n_total = t.n_atoms;
-    int rc = run_batch(c, c->frames_seq + frame, 1, false, c->batch_loss);
+    int rc = run_batch(c, c->frames_seq + frame, 1, nullptr, c->batch_loss);
     if (rc) return rc;
     const int n = t.n_atoms;
     std::vector<float> he((size_t)n), hf((size_t)n * 3);
