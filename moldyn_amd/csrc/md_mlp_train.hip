@@ -51,7 +51,7 @@ __device__ __forceinline__ Silu3 silu3(float a) {
 // (155 kFLOP, 79 TFLOP/s) of the 154 TFLOP/s a large FP32 product reaches here.
 // Before, a tiled FP32 product on the vector units per layer with elementwise
 // passes in between and the weight gradients in 128 splits: 1.93 ms per
-// minibatch of 65,536 rows in all, 0.44 ms now.
+// minibatch of 65,536 rows with the pair kernels, 0.31 ms now.
 // v_mfma_f32_16x16x4_f32, lane l = 16 g + c: operand A holds row c, operand B
 // column c, both at the k of lane group g; the result holds rows 4 g + i
 // (i = 0..3) of column c.  The k of a product may come in any order that A and
@@ -546,13 +546,44 @@ __global__ __launch_bounds__(256) void k_tr_feature_stats(TrainState t, int64_t 
 }
 
 // ---------------------------------------------------------------- pair kernels
+//
+// L lanes per atom share its pairs (pair q goes to lane q % L) and add their
+// sums at the end: a lane per atom leaves 65,536 atoms one wave per SIMD, with
+// nothing to run while a neighbour's row is on its way.  The 32 basis values of
+// a pair are bound by the exponentials: one base-2 hardware exponential each,
+// with the factor log2(e) / (2 w^2) rounded once (the argument carries the same
+// two roundings as before).  L = 8 below four waves per SIMD at L = 4.
+// Minibatch of 65,536 atoms of about 33 pairs: forces 88 -> 47 us, adjoint 76 ->
+// 48 us; of 6,655 atoms: 66 -> 12 and 56 -> 17 us.
+struct TrBasis {
+    float r, fcw, dfc;  // distance, cutoff / w^2, derivative of the cutoff
+};
+__device__ __forceinline__ TrBasis tr_basis(const TrainState& t, float r) {
+    float sn, cs;
+    sincospif(r / t.rc, &sn, &cs);
+    return {r, 0.5f * (cs + 1.0f) * t.inv_w2, -0.5f * kPiT / t.rc * sn};
+}
+// d/dr of basis function k: exp(-u^2 / 2 w^2) (f_c' - u f_c / w^2), u = r - mu_k
+__device__ __forceinline__ float tr_dg(const TrainState& t, const TrBasis& b, int k) {
+    const float u = b.r - t.mu[k];
+    return __builtin_amdgcn_exp2f(-(u * u) * t.exp2_2w2) * fmaf(-u, b.fcw, b.dfc);
+}
+
+// sum over the L lanes of an atom (every lane gets it)
+template <int L>
+__device__ __forceinline__ float lanes_sum(float v) {
+#pragma unroll
+    for (int o = 1; o < L; o <<= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
 
 // Forces of the minibatch frames from Gam (rows r = b n + i), the loss terms
 // and their derivatives phi = dL/dF, dy = dL/dy.
+template <int L>
 __global__ __launch_bounds__(256) void k_tr_forces(TrainState t, double* loss_part) {
     const int b = blockIdx.y, f = t.bf[b];
     const int n = t.n_atoms;
-    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int i = blockIdx.x * (256 / L) + threadIdx.x / L, sub = threadIdx.x % L;
     double le = 0.0, lf = 0.0;
     if (i < n) {
         const int64_t ri = (int64_t)b * n + i;  // row in the minibatch
@@ -560,74 +591,86 @@ __global__ __launch_bounds__(256) void k_tr_forces(TrainState t, double* loss_pa
         const double* P = t.pos + (int64_t)f * n * 3;
         const double bx = t.box[3 * f], by = t.box[3 * f + 1], bz = t.box[3 * f + 2];
         const double xi = P[3 * i], yi = P[3 * i + 1], zi = P[3 * i + 2];
-        float gi[kMlpK];
+        f32x4 gi[kMlpK / 4];
 #pragma unroll
-        for (int k = 0; k < kMlpK; ++k) gi[k] = t.Gam[ri * kMlpK + k];
+        for (int k = 0; k < kMlpK / 4; ++k) gi[k] = reinterpret_cast<const f32x4*>(t.Gam + ri * kMlpK)[k];
         float fx = 0.f, fy = 0.f, fz = 0.f;
         const int cnt = t.ncnt[di];
         const int32_t* nb = t.nbr + di * t.cap;
-        for (int q = 0; q < cnt; ++q) {
+        for (int q = sub; q < cnt; q += L) {
             const int j = nb[q];
+            const f32x4* gj = reinterpret_cast<const f32x4*>(t.Gam + ((int64_t)b * n + j) * kMlpK);
+            f32x4 gs[kMlpK / 4];
+#pragma unroll
+            for (int k = 0; k < kMlpK / 4; ++k) gs[k] = gj[k];
             const TrPair p = tr_pair(P, xi, yi, zi, bx, by, bz, j);
-            const float a = kPiT * p.r / t.rc;
-            const float fc = 0.5f * (cosf(a) + 1.0f), dfc = -0.5f * kPiT / t.rc * sinf(a);
-            const float* gj = t.Gam + ((int64_t)b * n + j) * kMlpK;
+            const TrBasis bs = tr_basis(t, p.r);
             float c = 0.f;
 #pragma unroll
-            for (int k = 0; k < kMlpK; ++k) {
-                const float u = p.r - t.mu[k];
-                const float e = expf(-u * u * t.inv_2w2);
-                c = fmaf(gi[k] + gj[k], e * fmaf(-u * t.inv_w2, fc, dfc), c);
-            }
+            for (int k = 0; k < kMlpK; ++k) c = fmaf(gi[k / 4][k % 4] + gs[k / 4][k % 4], tr_dg(t, bs, k), c);
             const float s = c / p.r;
             fx = fmaf(s, (float)p.dx, fx);
             fy = fmaf(s, (float)p.dy, fy);
             fz = fmaf(s, (float)p.dz, fz);
         }
-        const float ex = fx - t.Fref[3 * di], ey = fy - t.Fref[3 * di + 1], ez = fz - t.Fref[3 * di + 2];
-        const float ee = t.E[ri] - t.Eref[di];
-        t.F[3 * ri] = fx;
-        t.F[3 * ri + 1] = fy;
-        t.F[3 * ri + 2] = fz;
-        const float cf = 2.0f * t.w_f / (3.0f * (float)t.n_total);
-        t.phi[3 * ri] = cf * ex;
-        t.phi[3 * ri + 1] = cf * ey;
-        t.phi[3 * ri + 2] = cf * ez;
-        t.dy[ri] = 2.0f * t.w_e / (float)t.n_total * ee * t.e_scale;
-        le = (double)ee * ee;
-        lf = ((double)ex * ex + (double)ey * ey) + (double)ez * ez;
+        fx = lanes_sum<L>(fx);
+        fy = lanes_sum<L>(fy);
+        fz = lanes_sum<L>(fz);
+        if (sub == 0) {
+            const float ex = fx - t.Fref[3 * di], ey = fy - t.Fref[3 * di + 1], ez = fz - t.Fref[3 * di + 2];
+            const float ee = t.E[ri] - t.Eref[di];
+            t.F[3 * ri] = fx;
+            t.F[3 * ri + 1] = fy;
+            t.F[3 * ri + 2] = fz;
+            const float cf = 2.0f * t.w_f / (3.0f * (float)t.n_total);
+            t.phi[3 * ri] = cf * ex;
+            t.phi[3 * ri + 1] = cf * ey;
+            t.phi[3 * ri + 2] = cf * ez;
+            t.dy[ri] = 2.0f * t.w_e / (float)t.n_total * ee * t.e_scale;
+            le = (double)ee * ee;
+            lf = ((double)ex * ex + (double)ey * ey) + (double)ez * ez;
+        }
     }
     // block sums of the squared errors (fixed order)
-    __shared__ double sl[2][256];
-    sl[0][threadIdx.x] = le;
-    sl[1][threadIdx.x] = lf;
+    __shared__ double sl[2][4];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        le += __shfl_xor(le, o, 64);
+        lf += __shfl_xor(lf, o, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        sl[0][threadIdx.x >> 6] = le;
+        sl[1][threadIdx.x >> 6] = lf;
+    }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double sa = 0, sb = 0;
-        for (int q = 0; q < 256; ++q) {
-            sa += sl[0][q];
-            sb += sl[1][q];
-        }
+    if (threadIdx.x < 2) {
         const int64_t blk = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-        loss_part[2 * blk] = sa;
-        loss_part[2 * blk + 1] = sb;
+        const double* v = sl[threadIdx.x];
+        loss_part[2 * blk + threadIdx.x] = (v[0] + v[1]) + (v[2] + v[3]);
     }
 }
 
-// out[0..1] = block partials of the squared errors summed in block order
-__global__ __launch_bounds__(64) void k_tr_loss_sum(const double* __restrict__ part, int64_t blocks,
-                                                   double* __restrict__ out) {
-    if (threadIdx.x >= 2) return;
-    double s = 0.0;
-    for (int64_t q = 0; q < blocks; ++q) s += part[2 * q + threadIdx.x];
-    out[threadIdx.x] = s;
+// out[0..1] = block partials of the squared errors, summed in a fixed order
+__global__ __launch_bounds__(256) void k_tr_loss_sum(const double* __restrict__ part, int64_t blocks,
+                                                    double* __restrict__ out) {
+    __shared__ double s[256];
+    const int col = threadIdx.x & 1, row = threadIdx.x >> 1;
+    double v = 0.0;
+    for (int64_t q = row; q < blocks; q += 128) v += part[2 * q + col];
+    s[threadIdx.x] = v;
+    for (int o = 128; o >= 2; o >>= 1) {
+        __syncthreads();
+        if ((int)threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
+    }
+    if (threadIdx.x < 2) out[threadIdx.x] = s[threadIdx.x];
 }
 
 // U_i = sum_j ((phi_i - phi_j) . d_ij / r_ij) dg(r_ij)
+template <int L>
 __global__ __launch_bounds__(256) void k_tr_u(TrainState t) {
     const int b = blockIdx.y, f = t.bf[b];
     const int n = t.n_atoms;
-    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int i = blockIdx.x * (256 / L) + threadIdx.x / L, sub = threadIdx.x % L;
     if (i >= n) return;
     const int64_t ri = (int64_t)b * n + i;
     const int64_t di = (int64_t)f * n + i;
@@ -640,22 +683,34 @@ __global__ __launch_bounds__(256) void k_tr_u(TrainState t) {
     for (int k = 0; k < kMlpK; ++k) u[k] = 0.0f;
     const int cnt = t.ncnt[di];
     const int32_t* nb = t.nbr + di * t.cap;
-    for (int q = 0; q < cnt; ++q) {
+    for (int q = sub; q < cnt; q += L) {
         const int j = nb[q];
-        const TrPair p = tr_pair(P, xi, yi, zi, bx, by, bz, j);
         const float* pj = t.phi + 3 * ((int64_t)b * n + j);
-        const float proj = ((px - pj[0]) * (float)p.dx + (py - pj[1]) * (float)p.dy + (pz - pj[2]) * (float)p.dz) / p.r;
-        const float a = kPiT * p.r / t.rc;
-        const float fc = 0.5f * (cosf(a) + 1.0f), dfc = -0.5f * kPiT / t.rc * sinf(a);
+        const float qx = px - pj[0], qy = py - pj[1], qz = pz - pj[2];
+        const TrPair p = tr_pair(P, xi, yi, zi, bx, by, bz, j);
+        const float proj = (qx * (float)p.dx + qy * (float)p.dy + qz * (float)p.dz) / p.r;
+        const TrBasis bs = tr_basis(t, p.r);
 #pragma unroll
-        for (int k = 0; k < kMlpK; ++k) {
-            const float w = p.r - t.mu[k];
-            const float e = expf(-w * w * t.inv_2w2);
-            u[k] = fmaf(proj, e * fmaf(-w * t.inv_w2, fc, dfc), u[k]);
+        for (int k = 0; k < kMlpK; ++k) u[k] = fmaf(proj, tr_dg(t, bs, k), u[k]);
+    }
+    // the lanes' sums: each halving leaves a lane half of the values to add up
+    // (lane group o keeps the upper half), L lanes then hold 32 / L values each
+#pragma unroll
+    for (int o = 1, w = kMlpK / 2; o < L; o <<= 1, w >>= 1) {
+        const bool up = sub & o;
+#pragma unroll
+        for (int k = 0; k < kMlpK / 2; ++k) {
+            if (k >= w) break;
+            const float keep = up ? u[k + w] : u[k], give = up ? u[k] : u[k + w];
+            u[k] = keep + __shfl_xor(give, o, 64);
         }
     }
+    int k0 = 0;
 #pragma unroll
-    for (int k = 0; k < kMlpK; ++k) t.U[ri * kMlpK + k] = u[k];
+    for (int o = 1, w = kMlpK / 2; o < L; o <<= 1, w >>= 1) k0 += (sub & o) ? w : 0;
+    f32x4* out = reinterpret_cast<f32x4*>(t.U + ri * kMlpK + k0);
+#pragma unroll
+    for (int k = 0; k < kMlpK / L / 4; ++k) out[k] = f32x4{u[4 * k], u[4 * k + 1], u[4 * k + 2], u[4 * k + 3]};
 }
 
 // ---------------------------------------------------------------- launchers
@@ -689,20 +744,36 @@ hipError_t tr_forward_backward(const TrainState& t, int nf, bool keep, hipStream
     return hipGetLastError();
 }
 
+// lanes per atom of the pair kernels
+static inline int pair_lanes(const TrainState& t, int nf) {
+    return (int64_t)nf * t.n_atoms * 4 >= (int64_t)t.n_cu * 16 * 64 ? 4 : 8;
+}
+
+int64_t tr_loss_blocks(const TrainState& t, int nf) {
+    const int a = 256 / pair_lanes(t, nf);  // atoms per block
+    return (int64_t)((t.n_atoms + a - 1) / a) * nf;
+}
+
 hipError_t tr_forces(const TrainState& t, int nf, double* loss_part, hipStream_t st) {
-    hipLaunchKernelGGL(k_tr_forces, dim3(nblk(t.n_atoms), nf), dim3(256), 0, st, t, loss_part);
+    const int l = pair_lanes(t, nf), a = 256 / l;
+    const dim3 grid((unsigned)((t.n_atoms + a - 1) / a), nf);
+    if (l == 4) hipLaunchKernelGGL(k_tr_forces<4>, grid, dim3(256), 0, st, t, loss_part);
+    else hipLaunchKernelGGL(k_tr_forces<8>, grid, dim3(256), 0, st, t, loss_part);
     return hipGetLastError();
 }
 
 hipError_t tr_loss_sum(const TrainState& t, int nf, const double* loss_part, double* out, hipStream_t st) {
-    hipLaunchKernelGGL(k_tr_loss_sum, dim3(1), dim3(64), 0, st, loss_part, (int64_t)nblk(t.n_atoms) * nf, out);
+    hipLaunchKernelGGL(k_tr_loss_sum, dim3(1), dim3(256), 0, st, loss_part, tr_loss_blocks(t, nf), out);
     return hipGetLastError();
 }
 
 // Gradient of the minibatch loss: the blocks' sums at t.gpart, their number in *parts.
 hipError_t tr_gradient(const TrainState& t, int nf, int* parts, hipStream_t st) {
     const int64_t M = (int64_t)nf * t.n_atoms;
-    hipLaunchKernelGGL(k_tr_u, dim3(nblk(t.n_atoms), nf), dim3(256), 0, st, t);
+    const int l = pair_lanes(t, nf), a = 256 / l;
+    const dim3 grid((unsigned)((t.n_atoms + a - 1) / a), nf);
+    if (l == 4) hipLaunchKernelGGL(k_tr_u<4>, grid, dim3(256), 0, st, t);
+    else hipLaunchKernelGGL(k_tr_u<8>, grid, dim3(256), 0, st, t);
     const int64_t tiles = (M + kTrRows - 1) / kTrRows;
     *parts = (int)(tiles < t.n_cu ? tiles : t.n_cu);
     hipLaunchKernelGGL(k_tr_net_grad, dim3(*parts), dim3(kTrBS), 0, st, t, M, tiles);

@@ -26,7 +26,7 @@ struct TrainState {
     const int32_t* bf;
     // basis and normalisation
     float mu[kMlpK], g_mean[kMlpK], g_inv_std[kMlpK];
-    float rc, inv_2w2, inv_w2;
+    float rc, inv_2w2, inv_w2, exp2_2w2;  // exp2_2w2 = log2(e) / (2 w^2)
     float e_scale, e_shift, w_e, w_f;
     // parameters and optimiser
     float* theta;         // kMlpNP
@@ -49,6 +49,8 @@ hipError_t tr_feature_stats(const TrainState& t, int64_t rows, double* part, int
 // minibatch of nf frames t.bf[0..nf): M = nf n_atoms rows
 hipError_t tr_forward_backward(const TrainState& t, int nf, bool keep, hipStream_t st);
 hipError_t tr_forces(const TrainState& t, int nf, double* loss_part, hipStream_t st);
+// blocks of tr_forces (pairs of loss_part)
+int64_t tr_loss_blocks(const TrainState& t, int nf);
 hipError_t tr_loss_sum(const TrainState& t, int nf, const double* loss_part, double* out, hipStream_t st);
 hipError_t tr_gradient(const TrainState& t, int nf, int* parts, hipStream_t st);
 hipError_t tr_grad_sum(const TrainState& t, int parts, bool accumulate, hipStream_t st);

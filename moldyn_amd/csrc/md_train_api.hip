@@ -79,7 +79,7 @@ static int ensure_batch(md_trainer* c, int64_t rows) {
     if ((rc = talloc_t(c, &t.dy, r))) return rc;
     if ((rc = talloc_t(c, &t.F, r * 3))) return rc;
     if ((rc = talloc_t(c, &t.phi, r * 3))) return rc;
-    const int64_t blocks = (int64_t)((c->t.n_atoms + 255) / 256) * (rows / c->t.n_atoms + 1);
+    const int64_t blocks = (int64_t)((c->t.n_atoms + 31) / 32) * (rows / c->t.n_atoms + 1);
     if ((rc = talloc_t(c, &c->loss_part, (size_t)(2 * blocks + 2)))) return rc;
     c->batch_rows = rows;
     return MD_OK;
@@ -147,6 +147,7 @@ int md_trainer_create(md_trainer** out, int n_frames, int n_atoms, const double*
     t.rc = (float)(2.5 * sigma);
     t.inv_2w2 = (float)(1.0 / (2.0 * w * w));
     t.inv_w2 = (float)(1.0 / (w * w));
+    t.exp2_2w2 = (float)(M_LOG2E / (2.0 * w * w));
     t.e_scale = 1.0f;
     t.n_cu = 256;
     {
