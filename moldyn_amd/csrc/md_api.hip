@@ -88,6 +88,7 @@ struct md_ctx {
     int64_t kspan_count[P_NUM] = {};
     int64_t list_visits = 0;
     md_stats stats{};
+    int longest_list = 0;  // of the last builds, as far as they report it (choose_instances)
     int64_t last_rebuilds = 0, last_refresh = 0, last_splits = 0;
     bool ctrl_valid = false;  // ctrl holds epochs of fills into the current grid buffers
     // the step records still hold every replica's state as (x, v + F dt / 2m)
@@ -458,6 +459,7 @@ static int alloc_base(md_ctx* c) {
     DevState& d = c->d;
     d = DevState{};
     c->ctrl_valid = false;  // new control blocks: no state, no epochs yet
+    c->longest_list = 0;
     const int64_t N = c->n_slots;
     const size_t nd = sizeof(double) * (size_t)std::max<int64_t>(N, 1);
     void* p;
@@ -526,7 +528,12 @@ static int alloc_base(md_ctx* c) {
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(double) * NS * c->groups.size()))) return rc;
     d.sums = (double*)p;
     HIPCHK(c, hipMemset(p, 0, sizeof(double) * NS * c->groups.size()));
+    if (c->list_mode) {
+        if ((rc = dalloc(c, c->base_allocs, &p, sizeof(float4) * (size_t)std::max<int64_t>(N, 1)))) return rc;
+        d.cpos = (float4*)p;
+    }
     d.n_types = c->T;
+    d.n_cu = c->n_cu;
     d.n_blocks = c->n_blocks;
     d.n_reps = c->R;
     d.tpb = c->tpb;
@@ -731,16 +738,36 @@ static double expected_neighbours(const md_ctx* c, const std::vector<RepCtrl>& C
     return ne;
 }
 
-// Which kernel instances the next launches use (DevState::dense).  List
-// paths: long lists expected.  All-pairs path: k_ap_force keeps the pairs in
-// range of a particle in a list of kApCap = 96 entries and puts them in order
-// afterwards; above half of that on average too many particles overflow it and
-// are summed one thread each, and the ordering costs more than it saves.
-static void choose_instances(md_ctx* c, const std::vector<RepCtrl>& C) {
+// Which kernel instances the next launches use (DevState::dense), from the
+// control blocks C.
+// List paths: long lists expected at the mean density, or lists longer than
+// kClumpedList seen (a droplet in a gas): bricks sized for the mean density
+// overflow over a cluster and insert its long lists entry by entry (2,900
+// atoms, 2,048 of them in a droplet: update_force 6.1 ms, 0.24 ms with a wave
+// per cell; an FP32 step 1,030 and 67 us).  A wave per cell over
+// the many empty cells of a large dilute system costs more than that: stepping
+// (`stepping`) takes it for clusters up to 2^18 cells only.
+// All-pairs path: k_ap_force keeps the pairs in range of a particle in a list
+// of kApCap = 96 entries and puts them in order afterwards; above half of that
+// on average too many particles overflow it and are summed one thread each, and
+// the ordering costs more than it saves.
+static int choose_instances(md_ctx* c, std::vector<RepCtrl>& C, bool stepping) {
+    const int was = c->d.dense;
     if (c->list_mode)
-        c->d.dense = expected_neighbours(c, C, c->rlist) >= (double)kLaneWalk ? 1 : 0;
+        c->d.dense = expected_neighbours(c, C, c->rlist) >= (double)kLaneWalk ||
+                             (c->longest_list > kClumpedList && (!stepping || c->total_cells <= (int64_t)1 << 18))
+                         ? 1
+                         : 0;
     else
         c->d.dense = expected_neighbours(c, C, c->rc_max) > 48.0 ? 1 : 0;
+    // grids filled while sparse hold no FP32 positions for the dense builder
+    if (!c->list_mode || was || !c->d.dense) return MD_OK;
+    bool fresh = false;
+    for (RepCtrl& X : C) {
+        fresh = fresh || (X.flags & F_GRID_FRESH);
+        X.flags &= ~F_GRID_FRESH;
+    }
+    return fresh ? write_ctrl(c, C) : MD_OK;
 }
 
 // One step launch: list paths k_step + k_fin (which also builds lists),
@@ -874,11 +901,16 @@ static int read_ctrl_stats(md_ctx* c, std::vector<RepCtrl>& C, RepStats& s) {
     return MD_OK;
 }
 
+// The longest list the builds behind s report: cell by cell builds any above
+// kClumpedList, brick builds those near the capacity.
+static void note_lists(md_ctx* c, const RepStats& s) {
+    if (!c->d.dense) c->longest_list = std::max(c->longest_list, s.max_list);
+    else if (s.max_len > 0) c->longest_list = s.max_len;
+}
+
 // Grow list / cell capacity; returns 1 when grown.  After an overflow (the
 // chunk is replayed) the capacity at least doubles; ahead of one (a list or
-// cell within a quarter of its capacity) it grows by a quarter: dense
-// builds keep each centre particle's list column in a fixed LDS pool, so a
-// capacity far above the longest list costs build passes.
+// cell within a quarter of its capacity) it grows by a quarter.
 static int grow_capacity(md_ctx* c, const RepStats& s, int* grown, bool ahead = false) {
     *grown = 0;
     if (s.list_overflow) {
@@ -901,6 +933,7 @@ static int list_force_eval(md_ctx* c) {
     for (int attempt = 0; attempt < 8; ++attempt) {
         std::vector<RepCtrl> C;
         if ((rc = read_ctrl(c, C))) return rc;
+        if ((rc = choose_instances(c, C, false))) return rc;
         for (int r = 0; r < c->R; ++r) {
             RepCtrl& X = C[r];
             X.ins_epoch = X.fill_epoch + 1u;
@@ -932,6 +965,7 @@ static int list_force_eval(md_ctx* c) {
         if ((rc = reduce_state_sums(c, 1))) return rc;
         RepStats s;
         if ((rc = read_stats(c, s))) return rc;
+        note_lists(c, s);
         int grown = 0;
         if ((rc = grow_capacity(c, s, &grown))) return rc;
         if (grown) continue;
@@ -1012,6 +1046,7 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
         // the snapshot in one prologue kernel instead of several copies
         const bool one = c->R == 1;
         bool snap_in_prologue = false;
+        if ((rc = choose_instances(c, C, true))) return rc;
         if (c->list_mode) {
             if (one && !records_in_snapshot(c)) {
                 if ((rc = snapshot_alloc(c))) return rc;
@@ -1021,7 +1056,6 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
                 return rc;
             }
         }
-        choose_instances(c, C);
         for (int r = 0; r < c->R; ++r) {
             P[r].target_step = step0 + done + cn;
             P[r].use_psi_in = first ? 1 : 0;
@@ -1057,6 +1091,7 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
         RepStats s;
         for (int iter = 0;; ++iter) {
             if ((rc = read_ctrl_stats(c, C, s))) return rc;
+            note_lists(c, s);
             int64_t behind = 0;
             for (int r = 0; r < c->R; ++r) behind = std::max(behind, P[r].target_step - C[r].step);
             if (behind <= 0) break;
@@ -1643,7 +1678,7 @@ int md_update_force(md_ctx* c) {
     if (rc) return rc;
     std::vector<RepCtrl> C;
     if ((rc = read_ctrl(c, C))) return rc;
-    choose_instances(c, C);
+    if ((rc = choose_instances(c, C, false))) return rc;
     c->d.par = c->par;
     if (c->d.dense) {
         if (c->n_blocks > 0) HIPCHK(c, launch_allpairs(c->d, c->bs, true, c->st));

@@ -159,7 +159,8 @@ struct RepCtrl {
 struct RepStats {
     unsigned int list_overflow, cell_overflow;
     int max_list, max_cell;
-    unsigned int brick_fallback, pad;
+    unsigned int brick_fallback;
+    int max_len;  // wave-per-cell builds: the longest list above kClumpedList, 1 when none is
 };
 
 // Learned per-atom energy surrogate: 32 radial features, 128-128 SiLU MLP.
@@ -213,7 +214,8 @@ struct DevState {
     double4* dpos;           // dense list path: every slot's drifted position (x, y, z, unused)
     const uint8_t* slot_type;  // type of every slot (padding slots: the group's type)
     int32_t compact;         // the list path steps on crec (k_fin builds from crec)
-    int32_t dense;           // long lists expected: lanes walk their own lists, builds sort long lists in LDS
+    float4* cpos;            // list paths: FP32 position of every slot at the last grid fill (dense systems)
+    int32_t dense;           // long lists expected: lanes walk their own lists, a wave per cell builds them
                              // (all-pairs path: many pairs in range, a thread per particle sums as it goes)
     double* pot;
     double* vir;
@@ -263,7 +265,8 @@ struct DevState {
     int32_t n_reps;
     int32_t par;             // control buffer this launch reads
     int32_t tpb;             // tiles per block of the per-slot kernels
-    int32_t n_bld;           // list-build blocks
+    int32_t n_bld;           // brick-building blocks
+    int32_t n_cu;
     int64_t n_slots;
 };
 
@@ -319,7 +322,7 @@ constexpr int kBrickAtoms = 1024;
 constexpr int kBrickTarget = 900;  // expected staged particles a brick is sized for
 constexpr int kBrickOwn = 440;     // expected centre particles: one per thread of a 512-thread block
 constexpr int kListReg = 16;       // list entries kept (sorted) in registers while building
-constexpr int kBrickSeg = 16384;   // LDS entries for lists longer than kListReg (per brick)
+constexpr int kClumpedList = 32;   // a longer list in a system that is sparse on average marks a local cluster
 constexpr int kLaneWalk = 6;       // mean list entries per particle from which lanes walk their own lists
 
 // Cell grid of a fill: per axis floor(L / (r_list (1 + 1e-9))) cells in

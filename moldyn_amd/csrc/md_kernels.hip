@@ -60,41 +60,17 @@ __device__ __forceinline__ void list_close(const DevState& d, int64_t slot, int 
     }
 }
 
-// A list under construction.  Without an LDS column, the first kListReg
-// entries stay sorted in registers (compile-time indexed insertion) and a
-// longer list continues in global memory (sorted insertion); store() writes
-// the register part.  With SEG and a column the builder hands over (room for
-// the list capacity, at a stride of seg_stride; dense systems), the scan
-// lanes append the staging index of every candidate the FP32 test accepts
-// (brick_build), and one lane then runs the FP64 test, compacts and sorts
-// the column once (store_seg), in loops every lane runs at the same time:
-// in a dense brick some lane of the wave accepts a candidate at nearly every
-// step of the scan, and work per accepted entry inside the scan would make
-// the whole wave execute it each time.
-template <bool SEG>
+// A list under construction: the first kListReg entries stay sorted in
+// registers (compile-time indexed insertion), a longer list continues in global
+// memory (sorted insertion); store() writes the register part.
 struct RegList {
     int32_t v[kListReg];
     int n;
     int32_t* __restrict__ col;
     int64_t N;
     int cap;
-    int32_t* seg = nullptr;  // LDS column of cap entries at a stride of seg_stride (SEG)
-    int seg_stride = 0;
     __device__ __forceinline__ RegList(int32_t* c, int64_t stride, int capacity)
         : n(0), col(c), N(stride), cap(capacity) {}
-    // SEG: sort the column's first m entries (slot ids) and store them
-    __device__ __forceinline__ void store_seg(int m) {
-        for (int q = 1; q < m; ++q) {
-            const int32_t x = seg[q * seg_stride];
-            int p = q;
-            while (p > 0 && seg[(p - 1) * seg_stride] > x) {
-                seg[p * seg_stride] = seg[(p - 1) * seg_stride];
-                --p;
-            }
-            seg[p * seg_stride] = x;
-        }
-        for (int p = 0; p < m; ++p) col[(int64_t)p * N] = seg[p * seg_stride];
-    }
     __device__ __forceinline__ void push(int32_t j) {
         if (n < kListReg) {
 #pragma unroll
@@ -201,7 +177,6 @@ struct BrickLds {
     uint16_t cidx[kBrickAtoms];  // centre particle k -> its staging index
     uint16_t hc[kBrickAtoms];    // staged particle -> its halo cell
     uint8_t ty[kBrickAtoms];
-    int32_t seg[kBrickSeg];  // long lists of the centre particles, one column each
 };
 __device__ __forceinline__ BrickLds& brick_lds() {
     __shared__ BrickLds l;
@@ -226,8 +201,7 @@ __device__ __forceinline__ int brick_count(const RepCtrl& C) {
 }
 
 // Bricks bi0, bi0 + stride, ... of a replica (all threads of the block).
-// SEG: lists longer than kListReg continue in LDS columns (dense systems).
-template <typename RT, int BS, bool MULTI, bool SEG>
+template <typename RT, int BS, bool MULTI>
 __device__ __forceinline__ void brick_build(const DevState& d, const RepCtrl& C, const RepParams& P,
                             const RepInfo& R, const RT* __restrict__ recs, int bi0, int stride) {
     const uint32_t ep = C.fill_epoch;
@@ -479,13 +453,6 @@ __device__ __forceinline__ void brick_build(const DevState& d, const RepCtrl& C,
             if (MULTI) s_ty[a] = (uint8_t)rec_type(d, recs, j);
         }
         lds_barrier();
-        // LDS list columns (dense instances): every centre particle of a pass
-        // owns a column of list_cap entries in the pool, so a long capacity
-        // splits the centre particles into passes instead of sending their
-        // lists to global memory
-        const int dl = d.list_cap > 1 ? d.list_cap : 1;
-        const int per_pass = SEG ? (n_own < kBrickSeg / dl ? n_own : (kBrickSeg / dl > 1 ? kBrickSeg / dl : 1))
-                                 : n_own;
         // the stencil of staged centre particle a: its halo cell hc, the x and
         // y offsets [lo, hi], and its z cells as at most two runs of
         // consecutive halo cells, whose particles are consecutive in the
@@ -520,210 +487,7 @@ __device__ __forceinline__ void brick_build(const DevState& d, const RepCtrl& C,
                 za1 = hc[2] + 2;
             }
         };
-        for (int p0 = 0; p0 < n_own; p0 += per_pass) {
-        const int p1 = n_own - p0 < per_pass ? n_own : p0 + per_pass;
-        const int seg_cap = kBrickSeg / (p1 - p0);
-        if (SEG && seg_cap >= d.list_cap) {
-            // Dense bricks, every list in an LDS column: T lanes per centre
-            // particle share its nine stencil rows (a brick has fewer centre
-            // particles than the block has threads) and append the
-            // FP32-accepted candidates to the particle's column through a
-            // counter in s_cen (free once the staging is done).  Then the
-            // FP64 test and the ordering by slot id, so the list does not
-            // depend on the order of the appends: a wave per particle (lists
-            // up to 128 entries), else one lane per particle sorting its
-            // column.
-            const int npp = p1 - p0;
-            const int T = BS / npp < 1 ? 1 : (BS / npp > 4 ? 4 : BS / npp);
-            int* const s_cnt = s_cen;
-            for (int k = threadIdx.x; k < npp; k += BS) s_cnt[k] = 0;
-            lds_barrier();
-            for (int kk = threadIdx.x; kk < npp * T; kk += BS) {
-                const int k = p0 + kk / T, sub = kk % T;
-                const int a = s_cidx[k];
-                int hc[3], lo[2], hi[2], za0, za1, zb0, zb1;
-                stencil(a, hc, lo, hi, za0, za1, zb0, zb1);
-                const int ti = MULTI ? (int)s_ty[a] : 0;
-                const float4 pi = s_pf[a];
-                const float xf = pi.x, yf = pi.y, zf = pi.z;
-                int32_t* const col = L.seg + (k - p0);
-                int* const cnt = s_cnt + (k - p0);
-                const int cap = d.list_cap;
-                // uw: std::true_type when the FP32 copies are unwrapped
-                auto scan = [&](auto uw, int b0, int b1) {
-                    constexpr bool UW = decltype(uw)::value;
-                    // the next candidate's position is read while this one is
-                    // tested (the index stays in the run)
-                    float4 pn = s_pf[b0 < b1 ? b0 : 0];
-                    for (int b2 = b0; b2 < b1; ++b2) {
-                        // FP32 test first: it never rejects a pair the FP64 test keeps
-                        const float4 pj = pn;
-                        pn = s_pf[b2 + 1 < b1 ? b2 + 1 : b2];
-                        const float ex = UW ? pj.x - xf : min_image_f(pj.x - xf, bxf);
-                        const float ey = UW ? pj.y - yf : min_image_f(pj.y - yf, byf);
-                        const float ez = UW ? pj.z - zf : min_image_f(pj.z - zf, bzf);
-                        if (!((ex * ex + ey * ey) + ez * ez <= rl2f)) continue;
-                        // a particle is staged once per region: b2 == a is j == i
-                        if (b2 == a) continue;
-                        if (MULTI && (int)s_ty[b2] < ti) continue;
-                        // past the capacity a candidate is only counted (an
-                        // overflow: the chunk is replayed with a larger one)
-                        const int pos = atomicAdd(cnt, 1);
-                        if (pos < cap) col[pos * npp] = b2;
-                    }
-                };
-                auto rows = [&](auto uw) {
-                    int row_i = 0;  // the particle's stencil rows dealt out over its T lanes
-                    for (int o0 = lo[0]; o0 <= hi[0]; ++o0) {
-                        const int g0 = ((whole & 1) ? (hc[0] + o0 + gd[0]) % gd[0] : hc[0] + o0);
-                        for (int o1 = lo[1]; o1 <= hi[1]; ++o1) {
-                            if (row_i++ % T != sub) continue;
-                            const int g1 = ((whole & 2) ? (hc[1] + o1 + gd[1]) % gd[1] : hc[1] + o1);
-                            const int row = (g0 * hd[1] + g1) * hd[2];
-                            scan(uw, s_off[row + za0], s_off[row + za1]);
-                            if (zb1 > zb0) scan(uw, s_off[row + zb0], s_off[row + zb1]);
-                        }
-                    }
-                };
-                if (unwrap)
-                    rows(std::true_type{});
-                else
-                    rows(std::false_type{});
-            }
-            lds_barrier();
-            if (d.dense && d.list_cap <= 128) {
-                // one wave per centre particle: lane q runs the FP64 test of
-                // column entries q and q + 64, and each kept slot id goes
-                // straight to its sorted position, its rank among the kept
-                // ids (distinct), counted over the wave's lanes (sparse
-                // systems, whose columns hold a few entries, keep one lane
-                // per particle: a wave per particle would serialize them)
-                // PP particles per wave and iteration, their loads and
-                // tests interleaved (each particle's chain of dependent LDS
-                // reads would otherwise run alone).
-                constexpr int NW = BS / 64, PP = 4;
-                const int wv = threadIdx.x >> 6, wl = threadIdx.x & 63;
-                const int cap = d.list_cap;
-                for (int k0 = p0 + wv; k0 < p1; k0 += PP * NW) {
-                    int n[PP], m[PP];
-                    int32_t ii[PP];
-                    double xi[PP], yi[PP], zi[PP];
-                    const int32_t* colp[PP];
-#pragma unroll
-                    for (int p = 0; p < PP; ++p) {
-                        const bool has = k0 + p * NW < p1;
-                        const int k = has ? k0 + p * NW : k0;
-                        const int a = s_cidx[k];
-                        ii[p] = s_id[a];
-                        xi[p] = s_x[a];
-                        yi[p] = s_y[a];
-                        zi[p] = s_z[a];
-                        n[p] = has ? s_cnt[k - p0] : 0;
-                        m[p] = n[p] < cap ? n[p] : cap;
-                        colp[p] = L.seg + (k - p0);
-                    }
-                    auto kept_id = [&](int p, int q) -> uint32_t {  // ~0u: rejected
-                        const int b2 = colp[p][q * npp];
-                        const double dx = min_image_sel(s_x[b2] - xi[p], bx);
-                        const double dy = min_image_sel(s_y[b2] - yi[p], by);
-                        const double dz = min_image_sel(s_z[b2] - zi[p], bz);
-                        const double r2 = (dx * dx + dy * dy) + dz * dz;
-                        return r2 <= rl2 ? (uint32_t)s_id[b2] : ~0u;
-                    };
-                    uint32_t v0[PP], v1[PP];
-#pragma unroll
-                    for (int p = 0; p < PP; ++p) {
-                        v0[p] = wl < m[p] ? kept_id(p, wl) : ~0u;
-                        v1[p] = wl + 64 < m[p] ? kept_id(p, wl + 64) : ~0u;
-                    }
-                    // ranks of the kept ids (lanes past a particle's m hold
-                    // ~0u, below no id)
-                    int r0[PP], r1[PP];
-                    int mx = 0;
-#pragma unroll
-                    for (int p = 0; p < PP; ++p) {
-                        r0[p] = r1[p] = 0;
-                        mx = m[p] > mx ? m[p] : mx;
-                    }
-                    if (mx <= 64) {
-                        // one entry per lane: a bitonic sort over the wave
-                        // (ids ascending, the ~0u of rejected entries last),
-                        // after which lane r holds the entry of rank r
-#pragma unroll
-                        for (int kb = 2; kb <= 64; kb <<= 1) {
-#pragma unroll
-                            for (int jb = kb >> 1; jb > 0; jb >>= 1) {
-                                const bool keep_min = ((wl & kb) == 0) == ((wl & jb) == 0);
-#pragma unroll
-                                for (int p = 0; p < PP; ++p) {
-                                    const uint32_t o = (uint32_t)__shfl_xor((int)v0[p], jb, 64);
-                                    v0[p] = keep_min ? (o < v0[p] ? o : v0[p]) : (o > v0[p] ? o : v0[p]);
-                                }
-                            }
-                        }
-#pragma unroll
-                        for (int p = 0; p < PP; ++p) r0[p] = wl;
-                    } else {
-                        const int mx0 = mx < 64 ? mx : 64;
-                        for (int l = 0; l < mx0; ++l) {
-#pragma unroll
-                            for (int p = 0; p < PP; ++p) {
-                                const uint32_t x = __builtin_amdgcn_readlane(v0[p], l);
-                                r0[p] += x < v0[p] ? 1 : 0;
-                                r1[p] += x < v1[p] ? 1 : 0;
-                            }
-                        }
-                    }
-                    for (int l = 64; l < mx; ++l) {
-#pragma unroll
-                        for (int p = 0; p < PP; ++p) {
-                            const uint32_t x = __builtin_amdgcn_readlane(v1[p], l - 64);
-                            r0[p] += x < v0[p] ? 1 : 0;
-                            r1[p] += x < v1[p] ? 1 : 0;
-                        }
-                    }
-#pragma unroll
-                    for (int p = 0; p < PP; ++p) {
-                        if (k0 + p * NW >= p1) break;
-                        int32_t* const col = d.nbr + ii[p];
-                        if (v0[p] != ~0u) col[(int64_t)r0[p] * N] = (int32_t)v0[p];
-                        if (v1[p] != ~0u) col[(int64_t)r1[p] * N] = (int32_t)v1[p];
-                        const int kept = __popcll(__ballot(v0[p] != ~0u)) + __popcll(__ballot(v1[p] != ~0u));
-                        // more FP32-accepted candidates than the capacity
-                        // counts as an overflow (the chunk is replayed with
-                        // a larger one)
-                        if (wl == 0) list_close(d, ii[p], n[p] > cap ? n[p] : kept);
-                    }
-                }
-            } else
-            for (int k = p0 + threadIdx.x; k < p1; k += BS) {
-                const int a = s_cidx[k];
-                const int32_t i = s_id[a];
-                const double xi = s_x[a], yi = s_y[a], zi = s_z[a];
-                const int n = s_cnt[k - p0];
-                RegList<SEG> lst(d.nbr + i, N, d.list_cap);
-                lst.seg = L.seg + (k - p0);
-                lst.seg_stride = npp;
-                // the FP64 test (the reference's minimum image) over the
-                // FP32-accepted candidates, in a loop every lane runs at once
-                int kept = 0;
-                const int m = n < d.list_cap ? n : d.list_cap;
-                // the next entry is read before this one is kept (kept <= q)
-                int bn = m > 0 ? lst.seg[0] : 0;
-                for (int q = 0; q < m; ++q) {
-                    const int b2 = bn;
-                    if (q + 1 < m) bn = lst.seg[(q + 1) * lst.seg_stride];
-                    const double dx = min_image_sel(s_x[b2] - xi, bx);
-                    const double dy = min_image_sel(s_y[b2] - yi, by);
-                    const double dz = min_image_sel(s_z[b2] - zi, bz);
-                    const double r2 = (dx * dx + dy * dy) + dz * dz;
-                    if (r2 <= rl2) lst.seg[kept++ * lst.seg_stride] = s_id[b2];
-                }
-                lst.store_seg(kept);
-                list_close(d, i, n > d.list_cap ? n : kept);
-            }
-        } else
-        for (int k = p0 + threadIdx.x; k < p1; k += BS) {
+        for (int k = threadIdx.x; k < n_own; k += BS) {
             const int a = s_cidx[k];
             int hc[3], lo[2], hi[2], za0, za1, zb0, zb1;
             stencil(a, hc, lo, hi, za0, za1, zb0, zb1);
@@ -732,7 +496,7 @@ __device__ __forceinline__ void brick_build(const DevState& d, const RepCtrl& C,
             const double xi = s_x[a], yi = s_y[a], zi = s_z[a];
             const float4 pi = s_pf[a];
             const float xf = pi.x, yf = pi.y, zf = pi.z;
-            RegList<SEG> lst(d.nbr + i, N, d.list_cap);
+            RegList lst(d.nbr + i, N, d.list_cap);
             // uw: std::true_type when the FP32 copies are unwrapped
             auto scan = [&](auto uw, int b0, int b1) {
                 constexpr bool UW = decltype(uw)::value;
@@ -777,8 +541,6 @@ __device__ __forceinline__ void brick_build(const DevState& d, const RepCtrl& C,
             lst.store();
             list_close(d, i, lst.n);
         }
-        if (p1 < n_own) lds_barrier();  // the next pass reuses the columns
-        }  // passes
         }  // the region fitted in LDS
         lds_barrier();
         // the next region: the sub-brick's next cell, the brick's next
@@ -801,6 +563,231 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+// ---------------------------------------------------------------- dense lists, a wave per cell
+//
+// Ascending sort of 64 CH keys, CH consecutive ones per lane (bitonic; the
+// exchanges within a lane need no other lane).
+template <int CH>
+__device__ __forceinline__ void wave_sort(uint32_t (&v)[CH]) {
+    const int wl = threadIdx.x & 63;
+#pragma unroll
+    for (int kb = 2; kb <= 64 * CH; kb <<= 1)
+#pragma unroll
+        for (int jb = kb >> 1; jb > 0; jb >>= 1)
+            if (jb >= CH) {
+                const int m = jb / CH;
+                const bool keep_min = ((wl & (kb / CH)) == 0) == ((wl & m) == 0);
+#pragma unroll
+                for (int r = 0; r < CH; ++r) {
+                    const uint32_t o = (uint32_t)__shfl_xor((int)v[r], m, 64);
+                    v[r] = keep_min ? min(o, v[r]) : max(o, v[r]);
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < CH; ++r) {
+                    if (r & jb) continue;
+                    const bool up = kb < CH ? (r & kb) == 0 : (wl & (kb / CH)) == 0;
+                    const uint32_t lo = min(v[r], v[r | jb]), hi = max(v[r], v[r | jb]);
+                    v[r] = up ? lo : hi;
+                    v[r | jb] = up ? hi : lo;
+                }
+            }
+}
+
+constexpr int kCellCand = 1024;  // candidates (particles of a cell's 27-cell stencil) a wave sorts
+
+// Positions in an array of records of any kind (x, y, z come first).
+struct PosView {
+    const char* p;
+    int stride;
+    __device__ __forceinline__ const double* operator[](int64_t j) const {
+        return reinterpret_cast<const double*>(p + j * stride);
+    }
+};
+__device__ __forceinline__ double pos_r2(const double* a, const double* o, double bx, double by, double bz) {
+    const double dx = min_image(o[0] - a[0], bx), dy = min_image(o[1] - a[1], by), dz = min_image(o[2] - a[2], bz);
+    return (dx * dx + dy * dy) + dz * dz;
+}
+
+// The ids of a cell's candidates, sorted, to sid[0 .. 64 CH).  Candidate e is
+// entry map[e] >> 5 of the cell of lane map[e] & 31 (cid); map and sid share
+// the wave's LDS.
+template <int CH>
+__device__ __forceinline__ void sort_candidates(const DevState& d, const int32_t* __restrict__ cs, int64_t cid,
+                                                const uint16_t* map, uint32_t* sid, int total) {
+    const int wl = threadIdx.x & 63;
+    uint32_t id[CH];
+#pragma unroll
+    for (int r = 0; r < CH; ++r) {
+        const int e = wl + 64 * r;
+        const int m = e < total ? map[e] : 0;
+        const int64_t c = ((int64_t)__shfl((int)(cid >> 32), m & 31, 64) << 32) |
+                          (uint32_t)__shfl((int)(uint32_t)cid, m & 31, 64);
+        id[r] = e < total ? (uint32_t)cs[(int64_t)(m >> 5) * d.cell_plane + c] : ~0u;
+    }
+    wave_lds_sync();  // the map is read
+    wave_sort<CH>(id);
+#pragma unroll
+    for (int r = 0; r < CH; ++r) sid[wl * CH + r] = id[r];
+    wave_lds_sync();
+}
+
+// Lists of a replica whose cells hold several particles each (dense systems),
+// a wave per cell: cells wave0, wave0 + n_waves, ...  The particles of the
+// cell's stencil (up to 27 cells, 240 to 500 particles in a liquid) are the
+// candidates of every particle of the cell.  Their slot ids are sorted once;
+// 256 at a time they then sit in registers with their FP32 positions (left by
+// the fill in d.cpos), four per lane in ascending order, and each particle of
+// the cell takes one distance test per register, a ballot for each entry's
+// place, and one store: the entries come out in ascending order without a sort
+// per particle.
+// FP32 test: an FP32 component differs from the FP64 one by at most
+// (1.01 + 1.01 + 2.02 + 1 + 1.01) 2^-24 L for positions within 1.01 L (roundings
+// of the two positions, the difference, the box and the image); 20 2^-24 L
+// covers positions up to 3 L; |r| by 2 sqrt(3) times that, and the squared sum
+// adds less than 2^-20.  min(|d|, |b - |d||) is the magnitude of the reference's
+// minimum image.  Pairs the FP32 distance leaves open take the FP64 test.
+// What bounds it: the chain header - ids - sort - positions of a cell with four
+// waves per SIMD to cover it, and the sort's lane exchanges.  Bricks of cells
+// staged in LDS by 512 threads, one lane scanning per particle and a sort per
+// list (the dense builder before, one block per CU) took 920 us for 262,144
+// liquid particles, this 151 us; 685 and 35 us for 4,096 (343 cells on 256 CUs).
+// A sparse gas (a cell per particle or more) would leave a wave one particle
+// at a time: it keeps the bricks (1,000,000 particles: 146 us).
+template <bool MULTI>
+__device__ __forceinline__ void cell_build(const DevState& d, const RepCtrl& C, const RepParams& P, const RepInfo& R,
+                                           PosView recs, int wave0, int n_waves, uint32_t* sid) {
+    const uint32_t ep = C.fill_epoch;
+    const int buf = ep & 1;
+    const int g0 = C.gdim[buf][0], g1 = C.gdim[buf][1], g2 = C.gdim[buf][2];
+    const unsigned long long* __restrict__ hdr = d.cell_hdr[buf];
+    const int32_t* __restrict__ cs = d.cell_slots[buf];
+    const int cc = d.cell_cap, cap = d.list_cap;
+    const int64_t N = d.n_slots;
+    const int wl = threadIdx.x & 63;
+    const double bx = C.box[0], by = C.box[1], bz = C.box[2], rl2 = P.rlist * P.rlist;
+    const float bxf = (float)bx, byf = (float)by, bzf = (float)bz;
+    const double eps = 2.0 * 1.7320508075688772 * 20.0 * 0x1p-24 * fmax(bx, fmax(by, bz));
+    const double ro = P.rlist + eps, ri = fmax(P.rlist - eps, 0.0);
+    const float in2 = __double2float_rd(ri * ri * (1.0 - 0x1p-20)), out2 = __double2float_ru(ro * ro * (1.0 + 0x1p-20));
+    // lane l < 27: stencil offset (l / 9, l / 3 % 3, l % 3) along the axes,
+    // each cell once (three cells per axis, or all of one or two)
+    const int a0 = wl / 9, a1 = (wl / 3) % 3, a2 = wl % 3;
+    const bool in = wl < 27 && a0 < g0 && a1 < g1 && a2 < g2;
+    const int n_cells = g0 * g1 * g2;
+    for (int cell = wave0; cell < n_cells; cell += n_waves) {
+        const int c0 = cell / (g1 * g2), c1 = (cell / g2) % g1, c2 = cell % g2;
+        auto at = [](int c, int a, int g) {
+            const int q = g >= 3 ? c + a - 1 : a;
+            return q < 0 ? q + g : (q >= g ? q - g : q);
+        };
+        int64_t cid = 0;
+        int cnt = 0;
+        if (in) {
+            cid = R.cell_base + ((int64_t)at(c0, a0, g0) * g1 + at(c1, a1, g1)) * g2 + at(c2, a2, g2);
+            const unsigned long long h = hdr[cid];
+            if ((uint32_t)(h >> 32) == ep) cnt = (int)(uint32_t)h < cc ? (int)(uint32_t)h : cc;
+        }
+        // the cell's own lane (with one or two cells along an axis the offsets are cell indices)
+        const int hl = 9 * (g0 >= 3 ? 1 : c0) + 3 * (g1 >= 3 ? 1 : c1) + (g2 >= 3 ? 1 : c2);
+        const int n_home = __builtin_amdgcn_readlane(cnt, hl);
+        if (n_home == 0) continue;
+        const int incl = wave_scan_incl(cnt);
+        const int total = __builtin_amdgcn_readlane(incl, 63);
+        const int64_t home = R.cell_base + cell;
+        if (total <= kCellCand) {
+            uint16_t* const map = reinterpret_cast<uint16_t*>(sid);
+            wave_lds_sync();  // the last cell's reads of sid
+            for (int k = 0; k < cnt; ++k) map[incl - cnt + k] = (uint16_t)(wl | (k << 5));
+            wave_lds_sync();
+            if (total <= 256) sort_candidates<4>(d, cs, cid, map, sid, total);
+            else if (total <= 512) sort_candidates<8>(d, cs, cid, map, sid, total);
+            else sort_candidates<16>(d, cs, cid, map, sid, total);
+        }
+        for (int hb = 0; hb < n_home; hb += 64) {  // 64 home particles at a time, one per lane
+            const int nh = n_home - hb < 64 ? n_home - hb : 64;
+            const int32_t hi = wl < nh ? cs[(int64_t)(hb + wl) * d.cell_plane + home] : 0;
+            int32_t hf = 0;  // the first slot of the particle's type: a list holds no earlier type (potential.rs:171-180)
+            if (MULTI)
+                for (int t = 0; t < R.n_types; ++t) {
+                    const int32_t s = (int32_t)d.groups[R.first_group + t].start;
+                    hf = hi >= s ? s : hf;
+                }
+            int hn = 0;  // entries so far
+            if (total > kCellCand) {
+                // more than the wave sorts (a local cluster): a lane per particle, straight from the grid
+                for (int l = 0; l < 27; ++l) {
+                    const int64_t c = ((int64_t)__builtin_amdgcn_readlane((int)(cid >> 32), l) << 32) |
+                                      (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)cid, l);
+                    const int m = __builtin_amdgcn_readlane(cnt, l);
+                    for (int q = 0; q < m; ++q) {
+                        const int32_t j = cs[(int64_t)q * d.cell_plane + c];
+                        if (wl >= nh || j == hi || (MULTI && j < hf)) continue;
+                        if (!(pos_r2(recs[hi], recs[j], bx, by, bz) <= rl2)) continue;
+                        list_push(d.nbr + hi, N, hn, cap, j);
+                        ++hn;
+                    }
+                }
+            } else {
+                const float4 hp = d.cpos[hi];
+                for (int w0 = 0; w0 < total; w0 += 256) {
+                    float x[4], y[4], z[4];
+                    int32_t id[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int e = w0 + 64 * r + wl;
+                        id[r] = e < total ? (int32_t)sid[e] : 0;
+                        const float4 p = d.cpos[id[r]];
+                        x[r] = e < total ? p.x : __builtin_nanf("");
+                        y[r] = p.y;
+                        z[r] = p.z;
+                    }
+                    for (int h = 0; h < nh; ++h) {
+                        auto lane_f = [&](float v) {
+                            return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), h));
+                        };
+                        const int32_t i = __builtin_amdgcn_readlane(hi, h);
+                        const int32_t first = MULTI ? __builtin_amdgcn_readlane(hf, h) : 0;
+                        const float xi = lane_f(hp.x), yi = lane_f(hp.y), zi = lane_f(hp.z);
+                        bool ok[4], maybe[4];
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            float ex = fabsf(x[r] - xi), ey = fabsf(y[r] - yi), ez = fabsf(z[r] - zi);
+                            ex = fminf(ex, fabsf(bxf - ex));
+                            ey = fminf(ey, fabsf(byf - ey));
+                            ez = fminf(ez, fabsf(bzf - ez));
+                            const float r2 = fmaf(ex, ex, fmaf(ey, ey, ez * ez));
+                            const bool can = r2 <= out2 && id[r] != i && (!MULTI || id[r] >= first);
+                            ok[r] = can && r2 <= in2;
+                            maybe[r] = can && !(r2 <= in2);
+                        }
+                        if (__any(maybe[0] || maybe[1] || maybe[2] || maybe[3])) {
+#pragma unroll
+                            for (int r = 0; r < 4; ++r)
+                                if (maybe[r]) ok[r] = pos_r2(recs[i], recs[id[r]], bx, by, bz) <= rl2;
+                        }
+                        int pos = __builtin_amdgcn_readlane(hn, h);
+                        int32_t* const col = d.nbr + i;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const unsigned long long m = __ballot(ok[r]);
+                            const int q = pos + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+                            if (ok[r] && q < cap) col[(int64_t)q * N] = id[r];
+                            pos += __popcll(m);
+                        }
+                        if (wl == h) hn = pos;
+                    }
+                }
+            }
+            if (wl < nh) list_close(d, hi, hn);
+            if (hn > kClumpedList &&
+                hn > __hip_atomic_load(&d.stats->max_len, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                atomicMax(&d.stats->max_len, hn);
+        }
+    }
 }
 
 // LDS a wave's list forces use (owner positions and slots, pair terms and
@@ -1201,19 +1188,6 @@ __global__ __launch_bounds__(BS) void k_pack(DevState d) {
         o.uz = a.vz + (double)a.fz * c;
         out[s] = o;
     }
-}
-
-// Stand-alone list build (md_update_force on the list paths): replicas whose
-// control block is flagged F_BUILD build their lists from grid `fill_epoch`.
-template <typename FT, bool MULTI>
-__global__ __launch_bounds__(kFinBS) void k_build(DevState d) {
-    const int b = blockIdx.x;
-    const int r = d.bld_rep[b];
-    const RepCtrl& C = ctrl_in(d, r);
-    if ((C.flags & (F_BUILD | F_EXIT)) != F_BUILD) return;
-    const RepInfo R = d.reps[r];
-    brick_build<Rec<FT>, kFinBS, MULTI, true>(d, C, d.params[r], R, (const Rec<FT>*)d.rec[C.build_src],
-                                        b - R.bld_first, R.bld_count);
 }
 
 // Force evaluation at the current positions through the current lists
@@ -2088,29 +2062,50 @@ __device__ __forceinline__ void prof_fold(const DevState& d, int64_t launch, boo
     }
 }
 
-template <typename FT, bool MULTI, bool BUILD, bool REPS, bool DENSE>
-__global__ __launch_bounds__(kFinBS) void k_fin(DevState d, int mode) {
-    const int b = blockIdx.x;
-    const uint64_t t_start = prof_now(d);
-    // the last block folds the per-block records of k_step (or k_drift +
-    // k_allpairs) while the first blocks finalize
-    if (d.prof && mode == M_STEP && b == (int)gridDim.x - 1)
-        prof_fold(d, ctrl_in(d, 0).launches, !BUILD || d.mlp_w != nullptr);
+// Build block b's share of the lists of the replicas flagged F_BUILD in this
+// launch, from the step records (compact) or the full ones; returns the launch index when it built any, else -1.
+template <typename FT, bool MULTI, bool REPS, bool DENSE>
+__device__ __forceinline__ int64_t build_lists(const DevState& d, int b, bool compact) {
+    if constexpr (DENSE) {
+        // the cells of every building replica, numbered replica after replica,
+        // are shared out among the grid's waves; few cells go to as many blocks
+        // as there are, many keep neighbours in a block
+        __shared__ uint32_t s_sid[kFinBS / 64][kCellCand];
+        const int w = threadIdx.x >> 6, nw = (int)gridDim.x * (kFinBS / 64);
+        int64_t launch = -1, base = 0;
+        for (int r = 0; r < (REPS ? d.n_reps : 1); ++r) {
+            const RepCtrl& C = ctrl_in(d, r);
+            if ((C.flags & (F_BUILD | F_EXIT)) != F_BUILD) continue;
+            if (b == 0 && threadIdx.x == 0) atomicMax(&d.stats->max_len, 1);
+            const int buf = C.fill_epoch & 1;
+            const int64_t cells = (int64_t)C.gdim[buf][0] * C.gdim[buf][1] * C.gdim[buf][2];
+            const int gw = REPS || cells < nw ? w * (int)gridDim.x + b : b * (kFinBS / 64) + w;
+            const int w0 = (int)((gw - base % nw + nw) % nw);
+            const RepInfo R = d.reps[r];
+            const PosView recs = compact ? PosView{(const char*)d.crec[C.build_src], (int)sizeof(CRec)}
+                                           : PosView{(const char*)d.rec[C.build_src], (int)sizeof(Rec<FT>)};
+            cell_build<MULTI>(d, C, d.params[r], R, recs, w0, nw, s_sid[w]);
+            launch = C.launches;
+            base += cells;
+        }
+        return launch;
+    } else {
     int64_t launch = -1;
-    if (b < d.n_reps) launch = finalize_replica(d, b, mode);
-    if (BUILD && !REPS && b < d.n_bld) {
+    if constexpr (!REPS) {
+        if (b >= d.n_bld) return -1;
         // one system: the build blocks share its bricks
         const RepCtrl& C = ctrl_in(d, 0);
         if ((C.flags & (F_BUILD | F_EXIT)) == F_BUILD) {
             const RepInfo R = d.reps[0];
-            if (d.compact)
-                brick_build<CRec, kFinBS, MULTI, DENSE>(d, C, d.params[0], R, d.crec[C.build_src], b, d.n_bld);
+            if (compact)
+                brick_build<CRec, kFinBS, MULTI>(d, C, d.params[0], R, d.crec[C.build_src], b, d.n_bld);
             else
-                brick_build<Rec<FT>, kFinBS, MULTI, DENSE>(d, C, d.params[0], R, (const Rec<FT>*)d.rec[C.build_src], b,
+                brick_build<Rec<FT>, kFinBS, MULTI>(d, C, d.params[0], R, (const Rec<FT>*)d.rec[C.build_src], b,
                                                     d.n_bld);
             launch = C.launches;
         }
-    } else if (BUILD && b < d.n_bld) {
+    } else {
+        if (b >= d.n_bld) return -1;
         // several replicas: the bricks of every replica building in this
         // launch, numbered replica after replica, are shared out among all
         // build blocks: block b takes bricks b, b + n_bld, ... (replicas
@@ -2149,10 +2144,10 @@ __global__ __launch_bounds__(kFinBS) void k_fin(DevState d, int mode) {
                 const int bi0 = (int)(((b - lo % nb) % nb + nb) % nb);
                 const RepCtrl& C = ctrl_in(d, r);
                 const RepInfo R = d.reps[r];
-                if (d.compact)
-                    brick_build<CRec, kFinBS, MULTI, DENSE>(d, C, d.params[r], R, d.crec[C.build_src], bi0, nb);
+                if (compact)
+                    brick_build<CRec, kFinBS, MULTI>(d, C, d.params[r], R, d.crec[C.build_src], bi0, nb);
                 else
-                    brick_build<Rec<FT>, kFinBS, MULTI, DENSE>(d, C, d.params[r], R,
+                    brick_build<Rec<FT>, kFinBS, MULTI>(d, C, d.params[r], R,
                                                                (const Rec<FT>*)d.rec[C.build_src], bi0, nb);
                 launch = C.launches;
             }
@@ -2160,10 +2155,35 @@ __global__ __launch_bounds__(kFinBS) void k_fin(DevState d, int mode) {
             lds_barrier();  // s_rb and s_work are read before the next chunk rewrites them
         }
     }
+    return launch;
+    }
+}
+
+template <typename FT, bool MULTI, bool BUILD, bool REPS, bool DENSE>
+__global__ __launch_bounds__(kFinBS, DENSE ? 4 : 2) void k_fin(DevState d, int mode) {
+    const int b = blockIdx.x;
+    const uint64_t t_start = prof_now(d);
+    // the last block folds the per-block records of k_step (or k_drift +
+    // k_allpairs) while the first blocks finalize
+    if (d.prof && mode == M_STEP && b == (int)gridDim.x - 1)
+        prof_fold(d, ctrl_in(d, 0).launches, !BUILD || d.mlp_w != nullptr);
+    int64_t launch = -1;
+    if (b < d.n_reps) launch = finalize_replica(d, b, mode);
+    if (BUILD) {
+        const int64_t l = build_lists<FT, MULTI, REPS, DENSE>(d, b, d.compact != 0);
+        launch = l >= 0 ? l : launch;
+    }
     if (launch >= 0) {
         __syncthreads();
         prof_mark(d, launch, P_FIN, t_start);
     }
+}
+
+// Stand-alone list build (md_update_force on the list paths): the replicas
+// whose flags ask for it, from the full records.
+template <typename FT, bool MULTI, bool REPS, bool DENSE>
+__global__ __launch_bounds__(kFinBS, DENSE ? 4 : 2) void k_build(DevState d) {
+    build_lists<FT, MULTI, REPS, DENSE>(d, blockIdx.x, false);
 }
 
 // ---------------------------------------------------------------- small helpers
@@ -2312,16 +2332,33 @@ hipError_t launch_pack(const DevState& d, bool fp32, int bs, hipStream_t st) {
     return hipGetLastError();
 }
 
+// Blocks of a build: one per CU and brick-building block (158 KB of LDS), two
+// per CU where waves build cell by cell.
+static inline int build_grid(const DevState& d) { return d.dense ? 2 * d.n_cu : d.n_bld; }
+
 hipError_t launch_build(const DevState& d, bool fp32, hipStream_t st) {
-    const bool multi = d.n_types > 1;
+    const bool multi = d.n_types > 1, reps = d.n_reps > 1;
     if (d.n_bld <= 0) return hipSuccess;
+    const dim3 grid(build_grid(d));
+#define KB(FT, M, RP)                                                                               \
+    do {                                                                                             \
+        if (d.dense) hipLaunchKernelGGL((k_build<FT, M, RP, true>), grid, dim3(kFinBS), 0, st, d);  \
+        else hipLaunchKernelGGL((k_build<FT, M, RP, false>), grid, dim3(kFinBS), 0, st, d);         \
+    } while (0)
+#define KBR(FT, M)               \
+    do {                         \
+        if (reps) KB(FT, M, true); \
+        else KB(FT, M, false);   \
+    } while (0)
     if (fp32) {
-        if (multi) hipLaunchKernelGGL((k_build<float, true>), dim3(d.n_bld), dim3(kFinBS), 0, st, d);
-        else hipLaunchKernelGGL((k_build<float, false>), dim3(d.n_bld), dim3(kFinBS), 0, st, d);
+        if (multi) KBR(float, true);
+        else KBR(float, false);
     } else {
-        if (multi) hipLaunchKernelGGL((k_build<double, true>), dim3(d.n_bld), dim3(kFinBS), 0, st, d);
-        else hipLaunchKernelGGL((k_build<double, false>), dim3(d.n_bld), dim3(kFinBS), 0, st, d);
+        if (multi) KBR(double, true);
+        else KBR(double, false);
     }
+#undef KBR
+#undef KB
     return hipGetLastError();
 }
 
@@ -2375,7 +2412,8 @@ hipError_t launch_force_eval(const DevState& d, bool fp32, int bs, hipStream_t s
 hipError_t launch_finalize(const DevState& d, int mode, bool build, bool fp32, hipStream_t st) {
     const bool multi = d.n_types > 1;
     if (build && mode == M_STEP && d.n_bld > 0) {
-        const int grid = d.n_bld > d.n_reps ? d.n_bld : d.n_reps;
+        const int bld = build_grid(d);
+        const int grid = bld > d.n_reps ? bld : d.n_reps;
         const bool reps = d.n_reps > 1;
 #define KF2(FT, M, DN)                                                                                \
     do {                                                                                               \
