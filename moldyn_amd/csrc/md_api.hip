@@ -15,6 +15,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <chrono>
 #include <map>
 #include <string>
 #include <vector>
@@ -97,13 +98,22 @@ struct md_ctx {
     double crec_dt = 0.0;
     // pinned staging of every control block, statistics and parameter copy
     // of the stepping loop (no pageable transfer there)
+    void* h_pin = nullptr;  // the one allocation behind all of them (pinned_staging)
     RepCtrl* h_ctrl = nullptr;
     RepStats* h_stats = nullptr;
     RepParams* h_params = nullptr;
-    RepCtrl* h_ctrl_dev = nullptr;    // device addresses of h_ctrl / h_stats (the epilogue writes there)
-    RepStats* h_stats_dev = nullptr;
+    void* h_rec = nullptr;            // DevState::h_rec and h_pv as the host sees them
+    double* h_pv = nullptr;
+    uint32_t* h_done = nullptr;       // number of the last kernel that signalled its end
+    uint32_t done_seq = 0;            // number of the last one asked to
     hipEvent_t params_ev = nullptr;  // the last parameter upload (h_params is reused after it)
     bool params_pending = false;
+    // staging of uploads and downloads: device memory (at most kIoBytes), and
+    // pinned host memory that kernels address directly for small states
+    void* io_dev = nullptr;
+    size_t io_cap = 0;
+    void* io_pin = nullptr;
+    void* io_pin_dev = nullptr;
     // host copy of the control blocks the next launch reads, valid while no
     // finalize, graph replay, snapshot restore or layout change has run since
     std::vector<RepCtrl> ctrl_cache;
@@ -238,20 +248,25 @@ static void free_all(md_ctx* c) {
     c->prof_blk = nullptr;
     if (c->prof_host) (void)hipHostFree(c->prof_host);
     c->prof_host = nullptr;
-    if (c->h_ctrl) (void)hipHostFree(c->h_ctrl);
-    c->h_ctrl = nullptr;
-    if (c->h_stats) (void)hipHostFree(c->h_stats);
-    c->h_stats = nullptr;
     if (c->params_ev) {
         if (c->params_pending) (void)hipEventSynchronize(c->params_ev);
         (void)hipEventDestroy(c->params_ev);
     }
     c->params_ev = nullptr;
     c->params_pending = false;
-    if (c->h_params) (void)hipHostFree(c->h_params);
+    if (c->h_pin) (void)hipHostFree(c->h_pin);
+    c->h_pin = nullptr;
+    c->h_ctrl = nullptr;
+    c->h_stats = nullptr;
     c->h_params = nullptr;
-    c->h_ctrl_dev = nullptr;
-    c->h_stats_dev = nullptr;
+    c->h_done = nullptr;
+    c->done_seq = 0;
+    c->h_rec = nullptr;
+    c->h_pv = nullptr;
+    c->io_pin = c->io_pin_dev = nullptr;
+    if (c->io_dev) (void)hipFree(c->io_dev);
+    c->io_dev = nullptr;
+    c->io_cap = 0;
     c->d.prof = nullptr;
     c->d.prof_blk = nullptr;
     c->prof = false;  // a new layout starts unprofiled
@@ -294,6 +309,7 @@ static void make_layout(md_ctx* c) {
             G.first_block = block;
             G.rep = r;
             G.type = t;
+            G.first_atom = c->n_atoms + R.n_atoms;
             G.mass = c->masses[t];
             G.sum_m = fold_mass(G.mass, G.count);
             for (int b = 0; b < G.nblocks; ++b) c->blk_group.push_back((int32_t)c->groups.size());
@@ -553,22 +569,67 @@ static int alloc_base(md_ctx* c) {
 // Control blocks of the buffer the next launch reads.
 static RepCtrl* ctrl_cur(md_ctx* c) { return c->d.ctrl + (size_t)c->par * c->R; }
 
+// States up to kIoPinned bytes pass through pinned host memory that the kernels
+// read and write themselves: one launch and no copy operation (a step and a
+// download of 1,000 atoms: SMALL_FIGURES).  Larger ones are copied between the
+// caller's arrays and device staging, at most kIoBytes at a time.
+constexpr size_t kIoPinned = (size_t)256 << 10, kIoBytes = (size_t)128 << 20;
+
+// Systems up to this many slots leave the state of a call's last step in host
+// memory as well, so that a download right after it needs no kernel, no copy and
+// no wait (1,000 atoms: 19 -> 7 us per download of positions and velocities).
+// The stores cross the host link while the step runs (1,000 atoms: 100 KB).
+constexpr int64_t kMirrorSlots = 2048;
+
 // Pinned host staging of the stepping loop's transfers (allocated once per
 // layout).
 static int pinned_staging(md_ctx* c) {
-    if (c->h_ctrl) return MD_OK;
-    void* p = nullptr;
-    HIPCHK(c, hipHostMalloc(&p, sizeof(RepCtrl) * c->R, hipHostMallocDefault));
-    c->h_ctrl = (RepCtrl*)p;
-    HIPCHK(c, hipHostMalloc(&p, sizeof(RepStats), hipHostMallocDefault));
-    c->h_stats = (RepStats*)p;
-    HIPCHK(c, hipHostMalloc(&p, sizeof(RepParams) * c->R, hipHostMallocDefault));
-    c->h_params = (RepParams*)p;
-    HIPCHK(c, hipHostGetDevicePointer(&p, c->h_ctrl, 0));
-    c->h_ctrl_dev = (RepCtrl*)p;
-    HIPCHK(c, hipHostGetDevicePointer(&p, c->h_stats, 0));
-    c->h_stats_dev = (RepStats*)p;
+    if (c->h_pin) return MD_OK;
+    // one allocation (each costs 150 us and more, and the device's first access
+    // to another one a page-table walk over the host link)
+    auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+    const size_t ctrl = up(sizeof(RepCtrl) * c->R), params = up(sizeof(RepParams) * c->R), stats = up(sizeof(RepStats));
+    const size_t io = up(std::min<size_t>(kIoPinned, (size_t)c->n_atoms * 11 * sizeof(double)));
+    const bool mirror = c->R == 1 && c->d.compact && c->n_slots > 0 && c->n_slots <= kMirrorSlots;
+    const size_t rec = mirror ? rec_size(c) * (size_t)c->n_slots : 0;
+    const size_t pv = mirror ? sizeof(double) * 2 * (size_t)c->n_slots : 0;
+    HIPCHK(c, hipHostMalloc(&c->h_pin, ctrl + params + stats + 256 + io + rec + pv, hipHostMallocDefault));
+    void* dv = nullptr;
+    HIPCHK(c, hipHostGetDevicePointer(&dv, c->h_pin, 0));
+    char *h = (char*)c->h_pin, *d = (char*)dv;
+    auto take = [&](size_t n, void** dev) {
+        char* p = h;
+        if (dev) *dev = d;
+        h += n;
+        d += n;
+        return (void*)p;
+    };
+    c->h_ctrl = (RepCtrl*)take(ctrl, (void**)&c->d.h_ctrl);
+    c->h_params = (RepParams*)take(params, nullptr);
+    c->h_stats = (RepStats*)take(stats, (void**)&c->d.h_stats);
+    c->h_done = (uint32_t*)take(256, (void**)&c->d.h_done);
+    *c->h_done = 0;
+    c->io_pin = take(io, &c->io_pin_dev);
+    c->h_rec = mirror ? take(rec, &c->d.h_rec) : nullptr;
+    c->h_pv = mirror ? (double*)take(pv, (void**)&c->d.h_pv) : nullptr;
     HIPCHK(c, hipEventCreateWithFlags(&c->params_ev, hipEventDisableTiming));
+    return MD_OK;
+}
+
+// Waits until a kernel has written done_seq to h_done (true), or until the
+// stream is done without it (false).  A kernel's own word arrives some
+// microseconds before the stream reports its end, which is what a step of a
+// small system and its download mostly consist of; after a while the wait
+// becomes the runtime's.
+static int wait_done(md_ctx* c, bool* done) {
+    const auto t0 = std::chrono::steady_clock::now();
+    auto seen = [&] { return __atomic_load_n(c->h_done, __ATOMIC_ACQUIRE) == c->done_seq; };
+    while (!(*done = seen())) {
+        if (std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(200)) continue;
+        HIPCHK(c, hipStreamSynchronize(c->st));
+        *done = seen();
+        break;
+    }
     return MD_OK;
 }
 
@@ -892,7 +953,7 @@ static int read_ctrl_stats(md_ctx* c, std::vector<RepCtrl>& C, RepStats& s) {
     if ((rc = pinned_staging(c))) return rc;
     // one kernel writes both into the pinned buffers (two copies would be
     // two device operations)
-    HIPCHK(c, launch_epilogue(c->d, c->par, c->h_ctrl_dev, c->h_stats_dev, c->st));
+    HIPCHK(c, launch_epilogue(c->d, c->par, c->d.h_ctrl, c->d.h_stats, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
     C.assign(c->h_ctrl, c->h_ctrl + c->R);
     s = *c->h_stats;
@@ -1042,16 +1103,16 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
     md_stats st{};
     while (done < n) {
         const int64_t cn = std::min(n - done, chunk);
-        // one replica: parameters, cleared statistics and (step-record path)
-        // the snapshot in one prologue kernel instead of several copies
+        // one replica: parameters, cleared statistics, (step-record path) the
+        // snapshot and the first controls in one kernel instead of several copies
         const bool one = c->R == 1;
-        bool snap_in_prologue = false;
+        bool snap_in_prime = false;
         if ((rc = choose_instances(c, C, true))) return rc;
         if (c->list_mode) {
             if (one && !records_in_snapshot(c)) {
                 if ((rc = snapshot_alloc(c))) return rc;
                 c->snap_par = c->par;
-                snap_in_prologue = true;
+                snap_in_prime = true;
             } else if ((rc = snapshot(c, true))) {
                 return rc;
             }
@@ -1062,16 +1123,24 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
             P[r].full_dst = c->d.compact ? ((C[r].cur & 1) ^ 1) : -1;
         }
         if (one) {
+            if ((rc = pinned_staging(c))) return rc;
+            P[0].done_seq = ++c->done_seq;
+            if (c->done_seq == 0) P[0].done_seq = c->done_seq = 1;
+            P[0].done_launch = C[0].launches + cn;
             // the snapshot's layout without records: the group sums, then the
             // surrogate's counters (snapshot())
             char* sb = (char*)c->snap;
             const size_t sums_bytes = sizeof(double) * NS * c->groups.size();
-            HIPCHK(c, launch_prologue(c->d, P[0], snap_in_prologue ? (double*)sb : nullptr, (int)c->groups.size(),
-                                      snap_in_prologue && c->d.mlp_stat ? (MlpStat*)(sb + sums_bytes) : nullptr,
-                                      snap_in_prologue ? c->snap_ctrl : nullptr, c->par, c->st));
+            c->ctrl_cache_valid = false;
+            c->d.par = c->par;
+            HIPCHK(c, launch_prime(c->d, P[0], snap_in_prime ? (double*)sb : nullptr, (int)c->groups.size(),
+                                   snap_in_prime && c->d.mlp_stat ? (MlpStat*)(sb + sums_bytes) : nullptr,
+                                   snap_in_prime ? c->snap_ctrl : nullptr, c->st));
+            c->par ^= 1;
         } else {
             if ((rc = write_params(c, P))) return rc;
             if ((rc = reset_stats(c))) return rc;
+            HIPCHK(c, finalize(c, M_PRIME));
         }
         if (c->d.compact && !(c->crec_valid && c->crec_dt == dt)) {
             // the chunk steps on step records; its last step writes the full
@@ -1079,7 +1148,6 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
             c->d.par = c->par;
             HIPCHK(c, launch_pack(c->d, c->fp32, c->bs, c->st));
         }
-        HIPCHK(c, finalize(c, M_PRIME));
         int64_t k = 0;
         if (K > 1 && cn >= K) {
             if ((rc = ensure_graph(c, K))) return rc;
@@ -1090,7 +1158,16 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
         int64_t launched = cn;
         RepStats s;
         for (int iter = 0;; ++iter) {
-            if ((rc = read_ctrl_stats(c, C, s))) return rc;
+            bool done = false;
+            if (one && iter == 0 && (rc = wait_done(c, &done))) return rc;
+            if (done) {
+                C.assign(c->h_ctrl, c->h_ctrl + 1);
+                s = *c->h_stats;
+                c->ctrl_cache = C;
+                c->ctrl_cache_valid = true;
+            } else if ((rc = read_ctrl_stats(c, C, s))) {
+                return rc;
+            }
             note_lists(c, s);
             int64_t behind = 0;
             for (int r = 0; r < c->R; ++r) behind = std::max(behind, P[r].target_step - C[r].step);
@@ -1171,6 +1248,9 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
     if (bad) return fail(c, MD_ERR_BAROSTAT, "non-finite temperature/pressure or mu^3 <= 0 during the run");
     return MD_OK;
 }
+
+// Positions, velocities (null: zeros) and boxes of a new state.
+static int put_state(md_ctx* c, const double* x, const double* v, const double* box);
 
 // ------------------------------------------------------------------ C ABI
 
@@ -1289,8 +1369,8 @@ int md_create_replicas(md_ctx** out, int n_replicas, int n_types, const int64_t*
         md_destroy(c);
         return rc;
     }
-    std::vector<double> zeros((size_t)total * 3, 0.0);
-    rc = md_upload_state(c, zeros.data(), zeros.data(), c->box0.data());
+    const std::vector<double> box(c->box0);
+    rc = put_state(c, nullptr, nullptr, box.data());
     if (rc) {
         g_error = c->err;
         md_destroy(c);
@@ -1321,146 +1401,71 @@ int md_get_options(const md_ctx* c, md_options* out) {
 
 }  // extern "C"
 
-// slots of a group: its tiles of bs records (a block may hold several tiles)
-static int64_t group_slots(const md_ctx* c, const GroupInfo& G) { return (G.count + c->bs - 1) / c->bs * c->bs; }
+// ------------------------------------------------------------------ state transfer
 
-// Record buffer holding each replica's current state.  Replicas may sit at
-// different buffers: a split step ends in the buffer it started from while
-// an ordinary step ends in the other one.
-static int replica_bufs(md_ctx* c, std::vector<int>& cur) {
-    std::vector<RepCtrl> C;
-    int rc = read_ctrl(c, C);
-    if (rc) return rc;
-    cur.resize(c->R);
-    for (int r = 0; r < c->R; ++r) cur[r] = C[r].cur & 1;
-    return MD_OK;
-}
-
-// Copy each replica's slot range between the host image and its own buffer.
-static int copy_replica_ranges(md_ctx* c, void* host, size_t rsize, const std::vector<int>& cur, bool to_device) {
-    for (int r = 0; r < c->R; ++r) {
-        const RepInfo& R = c->reps[r];
-        if (R.end <= R.start) continue;
-        char* h = (char*)host + rsize * (size_t)R.start;
-        char* dv = (char*)c->d.rec[cur[r]] + rsize * (size_t)R.start;
-        const size_t bytes = rsize * (size_t)(R.end - R.start);
-        if (to_device)
-            HIPCHK(c, hipMemcpy(dv, h, bytes, hipMemcpyHostToDevice));
-        else
-            HIPCHK(c, hipMemcpy(h, dv, bytes, hipMemcpyDeviceToHost));
-    }
-    return MD_OK;
-}
-
-// Host <-> device record transfer.  Host arrays are N x 3 (x, y, z per
-// particle) in the caller's order; slots add NaN-positioned padding.  With
-// `cur` the records go to (and, keeping forces, come from) each replica's
-// current buffer; without it to buffer `buf` of every replica.
-template <typename FT>
-static int put_records(md_ctx* c, int buf, const double* x, const double* v, const double* f,
-                       bool keep_forces, const std::vector<int>* cur = nullptr) {
-    const size_t N = (size_t)std::max<int64_t>(c->n_slots, 1);
-    std::vector<Rec<FT>> h(N);
-    if (keep_forces) {
-        if (cur) {
-            int rc = copy_replica_ranges(c, h.data(), sizeof(Rec<FT>), *cur, false);
-            if (rc) return rc;
-        } else {
-            HIPCHK(c, hipMemcpy(h.data(), c->d.rec[buf], sizeof(Rec<FT>) * N, hipMemcpyDeviceToHost));
+// Moves the arrays (3, 3, 3, 1, 1 doubles per atom; null ones skipped) to the
+// device with `put`, else from it, chunk by chunk; launch(io) runs the kernel.
+// A transfer to the device may still read the caller's arrays on return.
+template <typename Launch>
+static int io_run(md_ctx* c, double* const (&host)[5], bool put, Launch launch) {
+    static const int width[5] = {3, 3, 3, 1, 1};
+    size_t per = 0;
+    for (int k = 0; k < 5; ++k) per += host[k] ? sizeof(double) * width[k] : 0;
+    const int64_t n = c->n_atoms;
+    c->d.par = c->par;
+    const bool pinned = per > 0 && (size_t)n * per <= kIoPinned;
+    int rc;
+    if (pinned) {
+        if ((rc = pinned_staging(c))) return rc;
+    } else if (per > 0) {
+        const size_t need = std::min((size_t)n * per, kIoBytes);
+        if (need > c->io_cap) {
+            if (c->io_dev) HIPCHK(c, hipFree(c->io_dev));
+            c->io_dev = nullptr;
+            c->io_cap = 0;
+            if (hipMalloc(&c->io_dev, need) != hipSuccess) {
+                c->io_dev = nullptr;
+                return fail(c, MD_ERR_NOMEM, "hipMalloc(" + std::to_string(need) + "): transfer staging");
+            }
+            c->io_cap = need;
         }
     }
-    for (const GroupInfo& G : c->groups)
-        for (int64_t i = 0; i < group_slots(c, G); ++i) {
-            Rec<FT>& r = h[(size_t)(G.start + i)];
-            r.type = (uint32_t)G.type;
-            if (i >= G.count && !keep_forces) {
-                r.x = r.y = r.z = NAN;
-                r.vx = r.vy = r.vz = 0.0;
-                r.fx = r.fy = r.fz = (FT)0;
-            }
+    const int64_t chunk = pinned || per == 0 ? n : (int64_t)(c->io_cap / per);
+    int64_t a0 = 0;
+    do {
+        StateIO io{};
+        io.a0 = a0;
+        io.a1 = std::min(n, a0 + chunk);
+        double** dev[5] = {&io.x, &io.v, &io.f, &io.pot, &io.vir};
+        size_t off = 0;
+        size_t at[5];
+        for (int k = 0; k < 5; ++k) {
+            if (!host[k]) continue;
+            at[k] = off;
+            *dev[k] = (double*)((char*)(pinned ? c->io_pin_dev : c->io_dev) + off);
+            off += sizeof(double) * width[k] * (size_t)(io.a1 - io.a0);
         }
-    int64_t a = 0;
-    for (const GroupInfo& G : c->groups)
-        for (int64_t i = 0; i < G.count; ++i, ++a) {
-            Rec<FT>& r = h[(size_t)(G.start + i)];
-            if (x) {
-                r.x = x[3 * a];
-                r.y = x[3 * a + 1];
-                r.z = x[3 * a + 2];
+        auto move = [&](bool to_device) -> int {
+            for (int k = 0; k < 5; ++k) {
+                if (!host[k]) continue;
+                double* h = host[k] + (size_t)width[k] * a0;
+                const size_t bytes = sizeof(double) * width[k] * (size_t)(io.a1 - io.a0);
+                if (pinned && to_device) memcpy((char*)c->io_pin + at[k], h, bytes);
+                else if (pinned) memcpy(h, (char*)c->io_pin + at[k], bytes);
+                else if (to_device) HIPCHK(c, hipMemcpyAsync(*dev[k], h, bytes, hipMemcpyHostToDevice, c->st));
+                else HIPCHK(c, hipMemcpyAsync(h, *dev[k], bytes, hipMemcpyDeviceToHost, c->st));
             }
-            if (v) {
-                r.vx = v[3 * a];
-                r.vy = v[3 * a + 1];
-                r.vz = v[3 * a + 2];
-            }
-            if (f) {
-                r.fx = (FT)f[3 * a];
-                r.fy = (FT)f[3 * a + 1];
-                r.fz = (FT)f[3 * a + 2];
-            } else if (!keep_forces) {
-                r.fx = r.fy = r.fz = (FT)0;
-            }
+            return MD_OK;
+        };
+        if (put && (rc = move(true))) return rc;
+        HIPCHK(c, launch(io));
+        if (!put) {
+            if (pinned) HIPCHK(c, hipStreamSynchronize(c->st));
+            if ((rc = move(false))) return rc;
         }
-    if (cur) return copy_replica_ranges(c, h.data(), sizeof(Rec<FT>), *cur, true);
-    HIPCHK(c, hipMemcpy(c->d.rec[buf], h.data(), sizeof(Rec<FT>) * N, hipMemcpyHostToDevice));
-    return MD_OK;
-}
-
-// Records of each replica's current buffer (`cur`, one entry per replica).
-template <typename FT>
-static int get_records(md_ctx* c, const std::vector<int>& cur, double* x, double* v, double* f) {
-    const size_t N = (size_t)std::max<int64_t>(c->n_slots, 1);
-    std::vector<Rec<FT>> h(N);
-    int rc = copy_replica_ranges(c, h.data(), sizeof(Rec<FT>), cur, false);
-    if (rc) return rc;
-    int64_t a = 0;
-    for (const GroupInfo& G : c->groups)
-        for (int64_t i = 0; i < G.count; ++i, ++a) {
-            const Rec<FT>& r = h[(size_t)(G.start + i)];
-            if (x) {
-                x[3 * a] = r.x;
-                x[3 * a + 1] = r.y;
-                x[3 * a + 2] = r.z;
-            }
-            if (v) {
-                v[3 * a] = r.vx;
-                v[3 * a + 1] = r.vy;
-                v[3 * a + 2] = r.vz;
-            }
-            if (f) {
-                f[3 * a] = (double)r.fx;
-                f[3 * a + 1] = (double)r.fy;
-                f[3 * a + 2] = (double)r.fz;
-            }
-        }
-    return MD_OK;
-}
-
-static int put_pv(md_ctx* c, const double* pot, const double* vir) {
-    const size_t N = (size_t)std::max<int64_t>(c->n_slots, 1);
-    std::vector<double> hp(N, 0.0), hv(N, 0.0);
-    int64_t a = 0;
-    for (const GroupInfo& G : c->groups)
-        for (int64_t i = 0; i < G.count; ++i, ++a) {
-            if (pot) hp[(size_t)(G.start + i)] = pot[a];
-            if (vir) hv[(size_t)(G.start + i)] = vir[a];
-        }
-    HIPCHK(c, hipMemcpy(c->d.pot, hp.data(), sizeof(double) * N, hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d.vir, hv.data(), sizeof(double) * N, hipMemcpyHostToDevice));
-    return MD_OK;
-}
-
-static int get_pv(md_ctx* c, double* pot, double* vir) {
-    const size_t N = (size_t)std::max<int64_t>(c->n_slots, 1);
-    std::vector<double> hp(N), hv(N);
-    HIPCHK(c, hipMemcpy(hp.data(), c->d.pot, sizeof(double) * N, hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(hv.data(), c->d.vir, sizeof(double) * N, hipMemcpyDeviceToHost));
-    int64_t a = 0;
-    for (const GroupInfo& G : c->groups)
-        for (int64_t i = 0; i < G.count; ++i, ++a) {
-            if (pot) pot[a] = hp[(size_t)(G.start + i)];
-            if (vir) vir[a] = hv[(size_t)(G.start + i)];
-        }
+        a0 = io.a1;
+    } while (a0 < n);
+    if (!put && !pinned) HIPCHK(c, hipStreamSynchronize(c->st));
     return MD_OK;
 }
 
@@ -1504,38 +1509,61 @@ static int next_epoch(md_ctx* c, uint32_t* epoch0) {
     return MD_OK;
 }
 
-extern "C" {
-
-int md_upload_state(md_ctx* c, const double* x, const double* v, const double* box) {
-    if (!c || !x || !v || !box) return fail(c, MD_ERR_ARG, "NULL argument");
-    int rc;
-    for (int b = 0; b < 2; ++b) {
-        rc = c->fp32 ? put_records<float>(c, b, x, v, nullptr, false)
-                     : put_records<double>(c, b, x, v, nullptr, false);
-        if (rc) return rc;
-    }
-    if ((rc = put_pv(c, nullptr, nullptr))) return rc;
+static int put_state(md_ctx* c, const double* x, const double* v, const double* box) {
+    double* const host[5] = {(double*)x, (double*)v, nullptr, nullptr, nullptr};
+    int rc = io_run(c, host, true, [&](const StateIO& io) {
+        return launch_put_state(c->d, c->fp32, (int)c->groups.size(), io, c->st);
+    });
+    if (rc) return rc;
     // the grid buffers keep the headers of earlier fills: continue the epoch
     // count past every epoch used so far so that none of them can match again
     uint32_t epoch0 = 0;
     if ((rc = next_epoch(c, &epoch0))) return rc;
-    return reset_controls(c, box, epoch0);
+    return reset_controls(c, box, epoch0);  // waits for the stream: the caller's arrays are read
+}
+
+// The state in DevState::h_rec / h_pv (kMirrorSlots).
+template <typename FT>
+static void get_mirror(const md_ctx* c, double* x, double* v, double* f, double* pot, double* vir) {
+    int64_t a = 0;
+    for (const GroupInfo& G : c->groups)
+        for (int64_t i = 0; i < G.count; ++i, ++a) {
+            const Rec<FT>& r = ((const Rec<FT>*)c->h_rec)[G.start + i];
+            if (x) {
+                x[3 * a] = r.x;
+                x[3 * a + 1] = r.y;
+                x[3 * a + 2] = r.z;
+            }
+            if (v) {
+                v[3 * a] = r.vx;
+                v[3 * a + 1] = r.vy;
+                v[3 * a + 2] = r.vz;
+            }
+            if (f) {
+                f[3 * a] = (double)r.fx;
+                f[3 * a + 1] = (double)r.fy;
+                f[3 * a + 2] = (double)r.fz;
+            }
+            if (pot) pot[a] = c->h_pv[G.start + i];
+            if (vir) vir[a] = c->h_pv[c->n_slots + G.start + i];
+        }
+}
+
+extern "C" {
+
+int md_upload_state(md_ctx* c, const double* x, const double* v, const double* box) {
+    if (!c || !x || !v || !box) return fail(c, MD_ERR_ARG, "NULL argument");
+    return put_state(c, x, v, box);
 }
 
 int md_upload_forces(md_ctx* c, const double* force, const double* pot, const double* vir) {
     if (!c) return MD_ERR_ARG;
-    std::vector<int> cur;
-    int rc = replica_bufs(c, cur);
+    double* const host[5] = {nullptr, nullptr, (double*)force, (double*)pot, (double*)vir};
+    int rc = io_run(c, host, true, [&](const StateIO& io) {
+        return launch_put_forces(c->d, c->fp32, (int)c->groups.size(), io, c->st);
+    });
     if (rc) return rc;
-    std::vector<double> zero;
-    if (!force) {
-        zero.assign((size_t)c->n_atoms * 3 + 1, 0.0);
-        force = zero.data();
-    }
-    rc = c->fp32 ? put_records<float>(c, 0, nullptr, nullptr, force, true, &cur)
-                 : put_records<double>(c, 0, nullptr, nullptr, force, true, &cur);
-    if (rc) return rc;
-    if ((rc = put_pv(c, pot, vir))) return rc;
+    HIPCHK(c, hipStreamSynchronize(c->st));  // the caller's arrays are read
     c->sums_valid = false;
     c->crec_valid = false;
     return MD_OK;
@@ -1545,21 +1573,26 @@ int md_download_state(md_ctx* c, double* x, double* v, double* force, double* po
                       double* box) {
     if (!c) return MD_ERR_ARG;
     std::vector<RepCtrl> C;
-    int rc = read_ctrl(c, C);
-    if (rc) return rc;
-    if (x || v || force) {
-        std::vector<int> cur(c->R);
-        for (int r = 0; r < c->R; ++r) cur[r] = C[r].cur & 1;
-        rc = c->fp32 ? get_records<float>(c, cur, x, v, force) : get_records<double>(c, cur, x, v, force);
+    int rc;
+    if (c->h_rec && c->crec_valid) {
+        // the last step left the state in host memory and nothing changed it since
+        if (c->fp32) get_mirror<float>(c, x, v, force, pot, vir);
+        else get_mirror<double>(c, x, v, force, pot, vir);
+    } else if (x || v || force || pot || vir) {
+        double* const host[5] = {x, v, force, pot, vir};
+        rc = io_run(c, host, false, [&](const StateIO& io) {
+            return launch_get_state(c->d, c->fp32, (int)c->groups.size(), io, c->st);
+        });
         if (rc) return rc;
     }
-    if (pot || vir)
-        if ((rc = get_pv(c, pot, vir))) return rc;
-    if (box)
-        for (int r = 0; r < c->R; ++r)
-            for (int k = 0; k < 3; ++k) box[3 * r + k] = C[r].box[k];
+    if (!box) return MD_OK;
+    if ((rc = read_ctrl(c, C))) return rc;
+    for (int r = 0; r < c->R; ++r)
+        for (int k = 0; k < 3; ++k) box[3 * r + k] = C[r].box[k];
     return MD_OK;
 }
+
+}  // extern "C"
 
 // Relayout keeping the state (used when block size / force path change).
 static int relayout(md_ctx* c, const md_options& nopt) {
@@ -1593,6 +1626,8 @@ static int relayout(md_ctx* c, const md_options& nopt) {
     }
     return write_ctrl(c, C2);
 }
+
+extern "C" {
 
 int md_set_options(md_ctx* c, const md_options* o) {
     if (!c || !o) return fail(c, MD_ERR_ARG, "NULL argument");

@@ -82,6 +82,13 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// The block's stores to host memory are complete, then `seq` is in *flag.
+__device__ __forceinline__ void signal_host(uint32_t* flag, uint32_t seq) {
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // DPP move of a double from the lane that CTRL selects; lanes without a
 // source lane, or in rows that ROW_MASK leaves out, get `fill`.
 template <int CTRL, int ROW_MASK>

@@ -101,6 +101,7 @@ struct PairParam {
 
 struct GroupInfo {
     int64_t start, count;
+    int64_t first_atom;  // atoms of the groups before it (the caller's particle order)
     int32_t first_block, nblocks;
     int32_t rep, type;
     double mass;   // Particle::mass of the type
@@ -132,7 +133,10 @@ struct RepParams {
     // records to, the one not holding the chunk's starting state (which a
     // replay after an overflow restarts from); -1 on the other paths
     int32_t full_dst;
-    int32_t pad_p;
+    // one replica: the finalize of launch done_launch writes done_seq to
+    // DevState::h_done (0: none does)
+    uint32_t done_seq;
+    int64_t done_launch;
     double cm[kMaxTypes];     // dt / (2 m_t), the half-kick factor (integrator.rs:29)
     double inv_m2[kMaxTypes]; // 1 / m_t^2 (drift-bound bookkeeping only)
 };
@@ -265,6 +269,16 @@ struct DevState {
     int32_t n_reps;
     int32_t par;             // control buffer this launch reads
     int32_t tpb;             // tiles per block of the per-slot kernels
+    // host memory (device addresses) a one-replica run leaves its control block
+    // and statistics in at launch RepParams::done_launch, and the number that
+    // says so
+    RepCtrl* h_ctrl;
+    RepStats* h_stats;
+    uint32_t* h_done;
+    // small one-replica systems of the list path: the full records, potentials
+    // and virials of a chunk's last step go to host memory as well (null: not)
+    void* h_rec;
+    double* h_pv;  // n_slots potentials, then n_slots virials
     int32_t n_bld;           // brick-building blocks
     int32_t n_cu;
     int64_t n_slots;
@@ -430,12 +444,13 @@ hipError_t launch_pack(const DevState& d, bool fp32, int bs, hipStream_t st);
 hipError_t launch_dpos(const DevState& d, int bs, hipStream_t st);
 hipError_t launch_build(const DevState& d, bool fp32, hipStream_t st);
 hipError_t launch_prof_init(const DevState& d, hipStream_t st);
-// Chunk prologue of a one-replica context in one launch: the parameters
-// (from the kernel argument), cleared statistics, and the snapshot a replay
-// restarts from (group sums of n_groups groups, the surrogate's counters when
-// snap_mlp is set, and the control block the next launch reads).
-hipError_t launch_prologue(const DevState& d, const RepParams& p, double* snap_sums, int n_groups,
-                           MlpStat* snap_mlp, RepCtrl* snap_ctrl, int par, hipStream_t st);
+// Start of a one-replica chunk in one launch: the parameters (from the kernel
+// argument), cleared statistics, the snapshot a replay restarts from (group
+// sums of n_groups groups, the surrogate's counters when snap_mlp is set, and
+// the control block the next launch reads), and the controls of the first step
+// (M_PRIME).
+hipError_t launch_prime(const DevState& d, const RepParams& p, double* snap_sums, int n_groups, MlpStat* snap_mlp,
+                        RepCtrl* snap_ctrl, hipStream_t st);
 // Chunk epilogue: the control blocks the next launch reads (n_reps) and the
 // statistics, written into host memory the device can address.
 hipError_t launch_epilogue(const DevState& d, int par, RepCtrl* h_ctrl, RepStats* h_stats, hipStream_t st);
@@ -461,6 +476,21 @@ hipError_t launch_mlp_force(const DevState& d, int bs, bool force_only, hipStrea
 hipError_t launch_mlp_convert(const DevState& d, hipStream_t st);
 
 // initialisers on the device (md_init.hip)
+// Atoms [a0, a1) of the caller's arrays (device addresses, atom a at a - a0;
+// any may be null).
+struct StateIO {
+    double *x, *v, *f;  // 3 per atom
+    double *pot, *vir;
+    int64_t a0, a1;
+};
+// A new state: positions and velocities of both record buffers (zeros for null
+// arrays), forces, potentials and virials 0; the call for a0 = 0 also writes
+// the padding slots.
+hipError_t launch_put_state(const DevState& d, bool fp32, int n_groups, const StateIO& io, hipStream_t st);
+// Forces into each replica's current buffer, potentials, virials (zeros for null arrays).
+hipError_t launch_put_forces(const DevState& d, bool fp32, int n_groups, const StateIO& io, hipStream_t st);
+// The state of each replica's current buffer to the non-null arrays.
+hipError_t launch_get_state(const DevState& d, bool fp32, int n_groups, const StateIO& io, hipStream_t st);
 hipError_t launch_init_blank(const DevState& d, bool fp32, const GroupInfo* groups, int n_groups, int64_t n_slots,
                              hipStream_t st);
 hipError_t launch_init_lattice(void* rec, bool fp32, int64_t slot0, int64_t sites, bool fcc, const double start[3],

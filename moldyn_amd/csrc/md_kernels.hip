@@ -1115,6 +1115,11 @@ __global__ __launch_bounds__(BS, 4) void k_step(DevState d) {
                 o.fz = acc.fz;
                 o.type = (uint32_t)ti;
                 full[s] = o;
+                if (d.h_rec) {
+                    ((Rec<FT>*)d.h_rec)[s] = o;
+                    d.h_pv[s] = (double)acc.pot;
+                    d.h_pv[d.n_slots + s] = (double)acc.vir;
+                }
             }
             part[S_MVX] += vx * m;
             part[S_MVY] += vy * m;
@@ -2003,6 +2008,15 @@ __device__ __forceinline__ int64_t finalize_replica(const DevState& d, int r, in
     copy_words<BS>(ctrl_out(d, r), &s_ctrl, (int)sizeof(RepCtrl));
     if (reduced)
         for (int i = threadIdx.x; i < T * NS; i += BS) d.sums[g0 * NS + i] = s_sums[i];
+    if (mode == M_STEP && s_par.done_seq != 0 && s_ctrl.launches == s_par.done_launch) {
+        // the last launch of a one-replica chunk: the host takes the control
+        // block and the statistics from its own memory, without another kernel
+        // or a wait for the stream (statistics of a build in this very launch
+        // follow at the end of the launches that it makes necessary)
+        copy_words<BS>(d.h_ctrl, &s_ctrl, (int)sizeof(RepCtrl));
+        copy_words<BS>(d.h_stats, d.stats, (int)sizeof(RepStats));
+        signal_host(d.h_done, s_par.done_seq);
+    }
     return mode == M_STEP ? launch : -1;
 }
 
@@ -2362,19 +2376,21 @@ hipError_t launch_build(const DevState& d, bool fp32, hipStream_t st) {
     return hipGetLastError();
 }
 
-__global__ __launch_bounds__(256) void k_prologue(DevState d, RepParams p, double* snap_sums, int n_groups,
-                                                  MlpStat* snap_mlp, RepCtrl* snap_ctrl, int par) {
-    const int t = threadIdx.x;
+// A one-replica chunk's start in one launch, and its end reported by the last
+// finalize (finalize_replica): a step of 1,000 atoms is three kernels instead of
+// five and no wait for the stream, 36.0 -> 30.5 us (median).
+__global__ __launch_bounds__(kFinBS) void k_prime(DevState d, RepParams p, double* snap_sums, int n_groups,
+                                                  MlpStat* snap_mlp, RepCtrl* snap_ctrl) {
     // word copies (every structure is a whole number of 32-bit words)
-    auto copy = [&](void* dst, const void* src, int bytes) {
-        for (int i = t; i < bytes / 4; i += 256) ((uint32_t*)dst)[i] = ((const uint32_t*)src)[i];
-    };
-    copy((void*)d.params, &p, (int)sizeof(RepParams));
-    for (int i = t; i < (int)(sizeof(RepStats) / 4); i += 256) ((uint32_t*)d.stats)[i] = 0u;
-    if (!snap_ctrl) return;  // no snapshot in this prologue
-    copy(snap_sums, d.sums, (int)sizeof(double) * NS * n_groups);
-    if (snap_mlp) copy(snap_mlp, d.mlp_stat, (int)sizeof(MlpStat));
-    copy(snap_ctrl, d.ctrl + (size_t)par * d.n_reps, (int)sizeof(RepCtrl));
+    copy_words<kFinBS>((void*)d.params, &p, (int)sizeof(RepParams));
+    for (int i = threadIdx.x; i < (int)(sizeof(RepStats) / 4); i += kFinBS) ((uint32_t*)d.stats)[i] = 0u;
+    if (snap_ctrl) {
+        copy_words<kFinBS>(snap_sums, d.sums, (int)sizeof(double) * NS * n_groups);
+        if (snap_mlp) copy_words<kFinBS>(snap_mlp, d.mlp_stat, (int)sizeof(MlpStat));
+        copy_words<kFinBS>(snap_ctrl, &ctrl_in(d, 0), (int)sizeof(RepCtrl));
+    }
+    __syncthreads();  // the parameters are read back from memory
+    finalize_replica(d, 0, M_PRIME);
 }
 
 __global__ __launch_bounds__(256) void k_epilogue(DevState d, int par, RepCtrl* h_ctrl, RepStats* h_stats) {
@@ -2384,9 +2400,9 @@ __global__ __launch_bounds__(256) void k_epilogue(DevState d, int par, RepCtrl* 
     for (int i = t; i < (int)(sizeof(RepStats) / 4); i += 256) ((uint32_t*)h_stats)[i] = ((const uint32_t*)d.stats)[i];
 }
 
-hipError_t launch_prologue(const DevState& d, const RepParams& p, double* snap_sums, int n_groups,
-                           MlpStat* snap_mlp, RepCtrl* snap_ctrl, int par, hipStream_t st) {
-    hipLaunchKernelGGL(k_prologue, dim3(1), dim3(256), 0, st, d, p, snap_sums, n_groups, snap_mlp, snap_ctrl, par);
+hipError_t launch_prime(const DevState& d, const RepParams& p, double* snap_sums, int n_groups, MlpStat* snap_mlp,
+                        RepCtrl* snap_ctrl, hipStream_t st) {
+    hipLaunchKernelGGL(k_prime, dim3(1), dim3(kFinBS), 0, st, d, p, snap_sums, n_groups, snap_mlp, snap_ctrl);
     return hipGetLastError();
 }
 
