@@ -34,6 +34,18 @@ enum { K_STEP = 0, K_FINALIZE = 1, K_ALLPAIRS = 2, K_DRIFT = 3, K_BUILD = 4, K_M
 
 }  // namespace
 
+// Device memory that is given back together.  Small arrays share slabs: a
+// context has about 30, and at 4,096 atoms allocating and freeing each by itself
+// (twice: md_set_options lays the context out again) was most of its 0.93 ms
+// set-up (0.5 ms now, with the layout of a context that holds no state yet not
+// carried over through the host).
+struct DevPool {
+    std::vector<void*> blocks;
+    char* cur = nullptr;
+    size_t left = 0;
+};
+constexpr size_t kSlab = (size_t)2 << 20, kSlabMost = (size_t)512 << 10;
+
 struct md_ctx {
     int device = 0;
     hipStream_t st = nullptr;
@@ -56,10 +68,9 @@ struct md_ctx {
     std::vector<int32_t> bld_rep;
     // device
     DevState d{};
-    std::vector<void*> base_allocs;
-    std::vector<void*> list_allocs;
+    DevPool base_allocs;
+    DevPool list_allocs;
     void* snap = nullptr;
-    size_t snap_bytes = 0;
     RepCtrl* snap_ctrl = nullptr;
     bool fp32 = true, list_mode = true;
     bool sums_valid = false;
@@ -91,6 +102,7 @@ struct md_ctx {
     md_stats stats{};
     int longest_list = 0;  // of the last builds, as far as they report it (choose_instances)
     int64_t last_rebuilds = 0, last_refresh = 0, last_splits = 0;
+    bool blank = false;       // no call has changed the blank state of md_create
     bool ctrl_valid = false;  // ctrl holds epochs of fills into the current grid buffers
     // the step records still hold every replica's state as (x, v + F dt / 2m)
     // for step length crec_dt: the next call needs no pack
@@ -99,6 +111,7 @@ struct md_ctx {
     // pinned staging of every control block, statistics and parameter copy
     // of the stepping loop (no pageable transfer there)
     void* h_pin = nullptr;  // the one allocation behind all of them (pinned_staging)
+    size_t h_pin_cap = 0;
     RepCtrl* h_ctrl = nullptr;
     RepStats* h_stats = nullptr;
     RepParams* h_params = nullptr;
@@ -207,22 +220,33 @@ static void rebuild_pairs(md_ctx* c) {
     c->rlist = c->rc_max + c->opt.skin;
 }
 
-static int dalloc(md_ctx* c, std::vector<void*>& owner, void** p, size_t bytes) {
+static int dalloc(md_ctx* c, DevPool& owner, void** p, size_t bytes) {
     *p = nullptr;
-    if (bytes == 0) bytes = 256;
-    hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess) {
-        *p = nullptr;
-        return fail(c, MD_ERR_NOMEM, std::string("hipMalloc(") + std::to_string(bytes) +
-                                         "): " + hipGetErrorString(e));
+    bytes = (std::max<size_t>(bytes, 1) + 255) / 256 * 256;
+    if (bytes <= kSlabMost && bytes <= owner.left) {
+        *p = owner.cur;
+        owner.cur += bytes;
+        owner.left -= bytes;
+        return MD_OK;
     }
-    owner.push_back(*p);
+    const bool slab = bytes <= kSlabMost;
+    void* q = nullptr;
+    hipError_t e = hipMalloc(&q, slab ? kSlab : bytes);
+    if (e != hipSuccess)
+        return fail(c, MD_ERR_NOMEM, std::string("hipMalloc(") + std::to_string(slab ? kSlab : bytes) +
+                                         "): " + hipGetErrorString(e));
+    owner.blocks.push_back(q);
+    *p = q;
+    if (slab) {
+        owner.cur = (char*)q + bytes;
+        owner.left = kSlab - bytes;
+    }
     return MD_OK;
 }
 
-static void free_list(std::vector<void*>& v) {
-    for (void* p : v) (void)hipFree(p);
-    v.clear();
+static void free_list(DevPool& v) {
+    for (void* p : v.blocks) (void)hipFree(p);
+    v = DevPool{};
 }
 
 static void drop_graph(md_ctx* c) {
@@ -237,10 +261,7 @@ static void free_all(md_ctx* c) {
     drop_graph(c);
     free_list(c->list_allocs);
     free_list(c->base_allocs);
-    if (c->snap) (void)hipFree(c->snap);
-    c->snap = nullptr;
-    c->snap_bytes = 0;
-    if (c->snap_ctrl) (void)hipFree(c->snap_ctrl);
+    c->snap = nullptr;  // in base_allocs
     c->snap_ctrl = nullptr;
     if (c->prof_ring) (void)hipFree(c->prof_ring);
     c->prof_ring = nullptr;
@@ -254,8 +275,7 @@ static void free_all(md_ctx* c) {
     }
     c->params_ev = nullptr;
     c->params_pending = false;
-    if (c->h_pin) (void)hipHostFree(c->h_pin);
-    c->h_pin = nullptr;
+    // the pinned block stays for the next layout (md_destroy frees it)
     c->h_ctrl = nullptr;
     c->h_stats = nullptr;
     c->h_params = nullptr;
@@ -440,7 +460,7 @@ static int alloc_mlp(md_ctx* c) {
     int rc;
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(__bf16) * N * kMlpK))) return rc;
     d.mlp_x = (__bf16*)p;
-    HIPCHK(c, hipMemset(p, 0, sizeof(__bf16) * N * kMlpK));
+    HIPCHK(c, hipMemsetAsync(p, 0, sizeof(__bf16) * N * kMlpK, c->st));
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(float) * N * kMlpK))) return rc;
     d.mlp_gam = (float*)p;
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(__bf16) * N * kMlpK))) return rc;
@@ -451,7 +471,7 @@ static int alloc_mlp(md_ctx* c) {
     d.mlp_e = (float*)p;
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(MlpStat) * c->R))) return rc;
     d.mlp_stat = (MlpStat*)p;
-    HIPCHK(c, hipMemset(p, 0, sizeof(MlpStat) * c->R));
+    HIPCHK(c, hipMemsetAsync(p, 0, sizeof(MlpStat) * c->R, c->st));
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(double) * 2 * (size_t)std::max(c->n_blocks, 1)))) return rc;
     d.mlp_judge = (double*)p;
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(MlpConst)))) return rc;
@@ -480,6 +500,7 @@ static int alloc_base(md_ctx* c) {
     const size_t nd = sizeof(double) * (size_t)std::max<int64_t>(N, 1);
     void* p;
     int rc;
+    std::vector<uint8_t> ty;  // read until the wait at the end
     for (int b = 0; b < 2; ++b) {
         if ((rc = dalloc(c, c->base_allocs, &p, rec_size(c) * (size_t)std::max<int64_t>(N, 1)))) return rc;
         d.rec[b] = p;
@@ -492,13 +513,13 @@ static int alloc_base(md_ctx* c) {
         }
         if ((rc = dalloc(c, c->base_allocs, &p, sizeof(double4) * (size_t)std::max<int64_t>(N, 1)))) return rc;
         d.dpos = (double4*)p;
-        std::vector<uint8_t> ty((size_t)std::max<int64_t>(N, 1), 0);
+        ty.assign((size_t)std::max<int64_t>(N, 1), 0);
         for (const GroupInfo& G : c->groups) {
             const int64_t n = (G.count + c->bs - 1) / c->bs * c->bs;
             for (int64_t i = 0; i < n; ++i) ty[(size_t)(G.start + i)] = (uint8_t)G.type;
         }
         if ((rc = dalloc(c, c->base_allocs, &p, ty.size()))) return rc;
-        HIPCHK(c, hipMemcpy(p, ty.data(), ty.size(), hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpyAsync(p, ty.data(), ty.size(), hipMemcpyHostToDevice, c->st));
         d.slot_type = (const uint8_t*)p;
         d.compact = 1;
     }
@@ -510,28 +531,26 @@ static int alloc_base(md_ctx* c) {
         return rc;
     d.blk_group = (const int32_t*)p;
     if (!c->blk_group.empty())
-        HIPCHK(c, hipMemcpy(p, c->blk_group.data(), sizeof(int32_t) * c->blk_group.size(),
-                            hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpyAsync(p, c->blk_group.data(), sizeof(int32_t) * c->blk_group.size(), hipMemcpyHostToDevice, c->st));
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(int32_t) * c->bld_rep.size()))) return rc;
     d.bld_rep = (const int32_t*)p;
-    HIPCHK(c, hipMemcpy(p, c->bld_rep.data(), sizeof(int32_t) * c->bld_rep.size(), hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpyAsync(p, c->bld_rep.data(), sizeof(int32_t) * c->bld_rep.size(), hipMemcpyHostToDevice, c->st));
     d.n_bld = (int32_t)c->bld_rep.size();
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(GroupInfo) * c->groups.size()))) return rc;
     d.groups = (const GroupInfo*)p;
-    HIPCHK(c, hipMemcpy(p, c->groups.data(), sizeof(GroupInfo) * c->groups.size(),
-                        hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpyAsync(p, c->groups.data(), sizeof(GroupInfo) * c->groups.size(), hipMemcpyHostToDevice, c->st));
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(RepInfo) * c->reps.size()))) return rc;
     d.reps = (const RepInfo*)p;
-    HIPCHK(c, hipMemcpy(p, c->reps.data(), sizeof(RepInfo) * c->reps.size(), hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpyAsync(p, c->reps.data(), sizeof(RepInfo) * c->reps.size(), hipMemcpyHostToDevice, c->st));
     if ((rc = dalloc(c, c->base_allocs, &p, 2 * sizeof(RepCtrl) * c->R))) return rc;
     d.ctrl = (RepCtrl*)p;
-    HIPCHK(c, hipMemset(p, 0, 2 * sizeof(RepCtrl) * c->R));
+    HIPCHK(c, hipMemsetAsync(p, 0, 2 * sizeof(RepCtrl) * c->R, c->st));
     c->par = 0;
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(RepParams) * c->R))) return rc;
     d.params = (const RepParams*)p;
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(RepStats)))) return rc;
     d.stats = (RepStats*)p;
-    HIPCHK(c, hipMemset(p, 0, sizeof(RepStats)));
+    HIPCHK(c, hipMemsetAsync(p, 0, sizeof(RepStats), c->st));
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(PairParam) * (size_t)c->T * c->T))) return rc;
     d.pairs = (const PairParam*)p;
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(double) * NS * (size_t)std::max(c->n_blocks, 1))))
@@ -540,10 +559,10 @@ static int alloc_base(md_ctx* c) {
     d.acc_mode = (c->R == 1 && c->T == 1) ? 1 : 0;
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(unsigned long long) * kAccWords))) return rc;
     d.acc = (unsigned long long*)p;
-    HIPCHK(c, hipMemset(p, 0, sizeof(unsigned long long) * kAccWords));
+    HIPCHK(c, hipMemsetAsync(p, 0, sizeof(unsigned long long) * kAccWords, c->st));
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(double) * NS * c->groups.size()))) return rc;
     d.sums = (double*)p;
-    HIPCHK(c, hipMemset(p, 0, sizeof(double) * NS * c->groups.size()));
+    HIPCHK(c, hipMemsetAsync(p, 0, sizeof(double) * NS * c->groups.size(), c->st));
     if (c->list_mode) {
         if ((rc = dalloc(c, c->base_allocs, &p, sizeof(float4) * (size_t)std::max<int64_t>(N, 1)))) return rc;
         d.cpos = (float4*)p;
@@ -571,7 +590,7 @@ static RepCtrl* ctrl_cur(md_ctx* c) { return c->d.ctrl + (size_t)c->par * c->R; 
 
 // States up to kIoPinned bytes pass through pinned host memory that the kernels
 // read and write themselves: one launch and no copy operation (a step and a
-// download of 1,000 atoms: SMALL_FIGURES).  Larger ones are copied between the
+// download of 1,000 atoms: 57 -> 44 us with the above).  Larger ones are copied between the
 // caller's arrays and device staging, at most kIoBytes at a time.
 constexpr size_t kIoPinned = (size_t)256 << 10, kIoBytes = (size_t)128 << 20;
 
@@ -584,16 +603,23 @@ constexpr int64_t kMirrorSlots = 2048;
 // Pinned host staging of the stepping loop's transfers (allocated once per
 // layout).
 static int pinned_staging(md_ctx* c) {
-    if (c->h_pin) return MD_OK;
-    // one allocation (each costs 150 us and more, and the device's first access
-    // to another one a page-table walk over the host link)
+    if (c->h_ctrl) return MD_OK;
+    // one allocation, kept over layouts (each costs 150 us and more, and the
+    // device's first access to another one a page-table walk over the host link)
     auto up = [](size_t n) { return (n + 255) / 256 * 256; };
     const size_t ctrl = up(sizeof(RepCtrl) * c->R), params = up(sizeof(RepParams) * c->R), stats = up(sizeof(RepStats));
     const size_t io = up(std::min<size_t>(kIoPinned, (size_t)c->n_atoms * 11 * sizeof(double)));
     const bool mirror = c->R == 1 && c->d.compact && c->n_slots > 0 && c->n_slots <= kMirrorSlots;
-    const size_t rec = mirror ? rec_size(c) * (size_t)c->n_slots : 0;
+    const size_t rec = mirror ? sizeof(Rec<double>) * (size_t)c->n_slots : 0;
     const size_t pv = mirror ? sizeof(double) * 2 * (size_t)c->n_slots : 0;
-    HIPCHK(c, hipHostMalloc(&c->h_pin, ctrl + params + stats + 256 + io + rec + pv, hipHostMallocDefault));
+    const size_t need = ctrl + params + stats + 256 + io + rec + pv;
+    if (need > c->h_pin_cap) {
+        if (c->h_pin) HIPCHK(c, hipHostFree(c->h_pin));
+        c->h_pin = nullptr;
+        c->h_pin_cap = 0;
+        HIPCHK(c, hipHostMalloc(&c->h_pin, need, hipHostMallocDefault));
+        c->h_pin_cap = need;
+    }
     void* dv = nullptr;
     HIPCHK(c, hipHostGetDevicePointer(&dv, c->h_pin, 0));
     char *h = (char*)c->h_pin, *d = (char*)dv;
@@ -898,11 +924,13 @@ static size_t state_bytes(md_ctx* c) {
 }
 
 static int snapshot_alloc(md_ctx* c) {
-    if (!c->snap) {
-        c->snap_bytes = std::max<size_t>(state_bytes(c), 256);
-        HIPCHK(c, hipMalloc(&c->snap, c->snap_bytes));
-        HIPCHK(c, hipMalloc((void**)&c->snap_ctrl, sizeof(RepCtrl) * c->R));
-    }
+    if (c->snap) return MD_OK;
+    void *p, *q;
+    int rc;
+    if ((rc = dalloc(c, c->base_allocs, &p, state_bytes(c)))) return rc;
+    if ((rc = dalloc(c, c->base_allocs, &q, sizeof(RepCtrl) * c->R))) return rc;
+    c->snap = p;
+    c->snap_ctrl = (RepCtrl*)q;
     return MD_OK;
 }
 
@@ -1051,6 +1079,7 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
                      bool per_rep) {
     if (n < 0) return fail(c, MD_ERR_ARG, "n_steps < 0");
     if (n == 0) return MD_OK;
+    c->blank = false;
     if (c->mlp && !c->mlp_ready) return fail(c, MD_ERR_ARG, "surrogate parameters not set (md_mlp_set_params)");
     for (int r = 0; r < c->R; ++r) {
         const md_thermostat* t = th ? &th[per_rep ? r : 0] : nullptr;
@@ -1376,6 +1405,7 @@ int md_create_replicas(md_ctx** out, int n_replicas, int n_types, const int64_t*
         md_destroy(c);
         return rc;
     }
+    c->blank = true;
     *out = c;
     return MD_OK;
 }
@@ -1389,6 +1419,7 @@ void md_destroy(md_ctx* c) {
     if (!c) return;
     (void)hipStreamSynchronize(c->st);
     free_all(c);
+    if (c->h_pin) (void)hipHostFree(c->h_pin);
     if (c->st) (void)hipStreamDestroy(c->st);
     delete c;
 }
@@ -1553,11 +1584,13 @@ extern "C" {
 
 int md_upload_state(md_ctx* c, const double* x, const double* v, const double* box) {
     if (!c || !x || !v || !box) return fail(c, MD_ERR_ARG, "NULL argument");
+    c->blank = false;
     return put_state(c, x, v, box);
 }
 
 int md_upload_forces(md_ctx* c, const double* force, const double* pot, const double* vir) {
     if (!c) return MD_ERR_ARG;
+    c->blank = false;
     double* const host[5] = {nullptr, nullptr, (double*)force, (double*)pot, (double*)vir};
     int rc = io_run(c, host, true, [&](const StateIO& io) {
         return launch_put_forces(c->d, c->fp32, (int)c->groups.size(), io, c->st);
@@ -1596,6 +1629,14 @@ int md_download_state(md_ctx* c, double* x, double* v, double* force, double* po
 
 // Relayout keeping the state (used when block size / force path change).
 static int relayout(md_ctx* c, const md_options& nopt) {
+    if (c->blank) {
+        // nothing to carry over
+        const std::vector<double> box(c->box0);
+        c->opt = nopt;
+        c->bs = nopt.block_size;
+        int rc = alloc_base(c);
+        return rc ? rc : put_state(c, nullptr, nullptr, box.data());
+    }
     const int64_t n = c->n_atoms;
     std::vector<double> x((size_t)n * 3 + 1), v((size_t)n * 3 + 1), f((size_t)n * 3 + 1),
         pot((size_t)n + 1), vir((size_t)n + 1), box((size_t)c->R * 3);
@@ -1656,12 +1697,13 @@ int md_set_options(md_ctx* c, const md_options* o) {
     } else {
         c->opt = n;
     }
+    const int lc = c->d.list_cap, cc = c->d.cell_cap;  // of the lists as they are allocated
     rebuild_pairs(c);
     if (n.list_capacity > 0) c->d.list_cap = n.list_capacity;
     if (n.cell_capacity > 0) c->d.cell_cap = n.cell_capacity;
     if (n.list_capacity <= 0 || n.cell_capacity <= 0) auto_capacities(c);
-    int rc = alloc_lists(c);
-    if (rc) return rc;
+    int rc = MD_OK;
+    if ((c->d.list_cap != lc || c->d.cell_cap != cc) && (rc = alloc_lists(c))) return rc;
     rc = upload_pairs(c);
     if (rc) return rc;
     std::vector<RepCtrl> C;
@@ -1705,6 +1747,7 @@ int md_set_pair_potential_lj(md_ctx* c, uint16_t t0, uint16_t t1, double sigma, 
 
 int md_update_force(md_ctx* c) {
     if (!c) return MD_ERR_ARG;
+    c->blank = false;
     c->crec_valid = false;
     if (c->mlp && !c->mlp_ready) return fail(c, MD_ERR_ARG, "surrogate parameters not set (md_mlp_set_params)");
     if (c->list_mode) return list_force_eval(c);
@@ -1730,6 +1773,7 @@ int md_update_force(md_ctx* c) {
 
 int md_apply_boundary_conditions(md_ctx* c) {
     if (!c) return MD_ERR_ARG;
+    c->blank = false;
     c->crec_valid = false;
     c->d.par = c->par;
     if (c->n_blocks > 0) HIPCHK(c, launch_wrap(c->d, c->fp32, c->bs, c->st));
@@ -1816,7 +1860,7 @@ int md_thermostat_update(md_ctx* c, md_thermostat* th, double dt, uint16_t type_
     int rc = type_thermo(c, 0, type_id, &t, nullptr, nullptr);
     if (rc) return rc;
     if (th->kind == 1 || th->kind == 2) {
-        c->crec_valid = false;
+        c->blank = c->crec_valid = false;
         const GroupInfo& G = c->groups[c->reps[0].first_group + type_id];
         c->d.par = c->par;
         HIPCHK(c, launch_scale(c->d, c->fp32, G.start, G.count, th->lambda, 0, c->st));
@@ -1844,7 +1888,7 @@ int md_barostat_update(md_ctx* c, md_barostat* ba, uint16_t type_id) {
     if (!c || !ba || type_id >= c->T) return fail(c, MD_ERR_ARG, "bad argument");
     if (ba->kind == 2) return fail(c, MD_ERR_UNIMPLEMENTED, "Barostat::Custom is todo!() in the reference");
     if (ba->kind != 1) return MD_OK;
-    c->crec_valid = false;
+    c->blank = c->crec_valid = false;
     const GroupInfo& G = c->groups[c->reps[0].first_group + type_id];
     c->d.par = c->par;
     HIPCHK(c, launch_scale(c->d, c->fp32, G.start, G.count, ba->myu, 1, c->st));
@@ -1935,6 +1979,7 @@ int md_init_mb_velocities(double* vel, int64_t n, double temperature, double mas
 // boxes; a context that never held a state gets the blank one first
 // (initialize_particles).
 static int edit_begin(md_ctx* c, std::vector<int>& cur, std::vector<double>& boxes) {
+    c->blank = false;
     boxes.assign((size_t)c->R * 3, 0.0);
     cur.assign(c->R, 0);
     if (!c->ctrl_valid) {
