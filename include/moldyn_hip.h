@@ -331,6 +331,13 @@ void md_frame_writer_destroy(md_frame_writer* w);
  * otherwise cap must hold *n_rows.  Errors: md_global_error(). */
 int md_frame_load(const char* dir, int64_t state_number, int64_t cap, int64_t* n_rows, uint16_t* ids, double* x,
                   double* v, double* box);
+/* The same with the file read once: open reads it and counts its rows, read
+ * fills the arrays for them (ids, x and v; box nullable), close frees the
+ * reader.  Errors: md_global_error(). */
+typedef struct md_frame_reader md_frame_reader;
+int md_frame_reader_open(md_frame_reader** out, const char* dir, int64_t state_number, int64_t* n_rows);
+int md_frame_reader_read(md_frame_reader* r, uint16_t* ids, double* x, double* v, double* box);
+void md_frame_reader_close(md_frame_reader* r);
 
 /* GPU formatter of numeric CSV tables in the same text: rows of an optional
  * u64 key column and ncol (1..10) f64 columns, "," between fields and "\n"

@@ -39,7 +39,7 @@ EXPORTS = (
     "md_trainer_set_params", "md_trainer_get_params", "md_trainer_loss", "md_trainer_epoch",
     "md_trainer_predict", "md_frame_writer_create", "md_frame_writer_save", "md_frame_writer_flush",
     "md_frame_writer_stats", "md_frame_writer_last_error", "md_frame_writer_destroy", "md_frame_load",
-    "md_text_create", "md_text_destroy", "md_text_last_error", "md_text_table", "md_csv_write_table",
+    "md_frame_reader_open", "md_frame_reader_read", "md_frame_reader_close", "md_text_create", "md_text_destroy", "md_text_last_error", "md_text_table", "md_csv_write_table",
     "md_init_positions", "md_init_velocities", "md_macro_noalloc",
 )
 
@@ -152,6 +152,10 @@ def load():
     L.md_frame_writer_destroy.argtypes = [vp]
     L.md_frame_writer_destroy.restype = None
     L.md_frame_load.argtypes = [C.c_char_p, C.c_int64, C.c_int64, i64p, C.POINTER(C.c_uint16), dp, dp, dp]
+    L.md_frame_reader_open.argtypes = [C.POINTER(vp), C.c_char_p, C.c_int64, i64p]
+    L.md_frame_reader_read.argtypes = [vp, C.POINTER(C.c_uint16), dp, dp, dp]
+    L.md_frame_reader_close.argtypes = [vp]
+    L.md_frame_reader_close.restype = None
     L.md_text_create.argtypes = [C.POINTER(vp)]
     L.md_text_destroy.argtypes = [vp]
     L.md_text_destroy.restype = None

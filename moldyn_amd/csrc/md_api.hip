@@ -13,8 +13,10 @@
 #include <math.h>
 #include <stdio.h>
 #include <string.h>
+#include <unistd.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <map>
 #include <string>
@@ -1348,6 +1350,13 @@ static int check_device(int* dev) {
     return MD_OK;
 }
 
+// (process << 32) | (device + 1) of the last context made, 0 before the first
+static std::atomic<uint64_t> g_owner{0};
+__attribute__((visibility("hidden"))) int md_context_device(void) {
+    const uint64_t o = g_owner.load(std::memory_order_relaxed);
+    return (o >> 32) == (uint64_t)(uint32_t)getpid() ? (int)(o & 0xffffffffu) - 1 : -1;
+}
+
 int md_create_replicas(md_ctx** out, int n_replicas, int n_types, const int64_t* counts,
                        const double* masses, const double* boxes) {
     if (!out) return fail(nullptr, MD_ERR_ARG, "out is NULL");
@@ -1406,6 +1415,7 @@ int md_create_replicas(md_ctx** out, int n_replicas, int n_types, const int64_t*
         return rc;
     }
     c->blank = true;
+    g_owner.store(((uint64_t)(uint32_t)getpid() << 32) | (uint32_t)(dev + 1), std::memory_order_relaxed);
     *out = c;
     return MD_OK;
 }

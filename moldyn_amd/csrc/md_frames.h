@@ -29,3 +29,7 @@ struct FrameSource {
 // Fills *out for replica `replica` of c (the buffers of the moment: call it
 // again after anything that may reallocate them).
 __attribute__((visibility("hidden"))) int md_frame_source(md_ctx* c, int replica, md::FrameSource* out);
+
+// Device of the last context that this very process made (not the one it was
+// forked from); -1: none.
+extern "C" __attribute__((visibility("hidden"))) int md_context_device(void);

@@ -17,9 +17,13 @@
 // writes the files while the caller keeps stepping: two frames in flight.
 // k_table_rows does the same for plain tables of doubles (bb.csv, macro.csv).
 //
-// Reading.  data/<n>.csv and bb.csv are parsed on the host threads (the
-// columns found by header name, numbers read correctly rounded like Rust's
-// f64::from_str), then uploaded by the caller.
+// Reading.  bb.csv, small state files and files that are not in the writer's own
+// form are parsed on the host threads (the columns found by header name, numbers
+// read correctly rounded like Rust's f64::from_str).  A large data/<n>.csv in
+// the writer's form goes to the device as text: k_line_count / k_line_fill find
+// its lines, k_frame_parse reads a row per thread; the few numbers it cannot
+// round with certainty are read again on the host, and anything unusual in the
+// text sends the whole file there.
 #include <errno.h>
 #include <fcntl.h>
 #include <stdio.h>
@@ -233,6 +237,155 @@ __global__ __launch_bounds__(256) void k_text_gather(const char* __restrict__ re
     for (int64_t i = threadIdx.x; i < len; i += 256) out[off + i] = src[i];
 }
 
+// ------------------------------------------------------------------ reading kernels
+
+constexpr int kLineBytes = 64;  // text per thread of the line kernels
+constexpr int kLineBS = 256;
+
+__device__ __forceinline__ uint32_t newlines_at(const char* __restrict__ text, int64_t size, int64_t p, uint64_t* where) {
+    // bit k of *where: text[p + k] is a newline (text is readable up to a multiple of 64 bytes)
+    uint64_t m = 0;
+    if (p < size) {
+        const uint4* v = reinterpret_cast<const uint4*>(text + p);
+#pragma unroll
+        for (int q = 0; q < kLineBytes / 16; ++q) {
+            const uint4 u = v[q];
+            const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                    m |= (uint64_t)(((w[i] >> (8 * b)) & 0xffu) == 10u) << (16 * q + 4 * i + b);
+        }
+        if (size - p < kLineBytes) m &= (1ull << (size - p)) - 1;
+    }
+    *where = m;
+    return (uint32_t)__popcll(m);
+}
+
+struct OpenNumber {  // a number k_frame_parse leaves to the host
+    int64_t at;      // 6 row + column
+    int64_t off;     // in the text
+    int32_t len, pad;
+};
+constexpr uint32_t kOpenMax = 4096;
+struct ParseMeta {
+    uint32_t irregular, n_open;
+    OpenNumber open[kOpenMax];
+};
+
+__global__ __launch_bounds__(kLineBS) void k_line_count(const char* __restrict__ text, int64_t size,
+                                                        int64_t* __restrict__ blk) {
+    uint64_t m;
+    int total;
+    const int64_t p = ((int64_t)blockIdx.x * kLineBS + threadIdx.x) * kLineBytes;
+    (void)block_scan_excl<kLineBS>((int)newlines_at(text, size, p, &m), total);
+    if (threadIdx.x == 0) blk[blockIdx.x] = total;
+}
+
+// start[i + 1] = one past newline i (i + 1 < cap)
+__global__ __launch_bounds__(kLineBS) void k_line_fill(const char* __restrict__ text, int64_t size,
+                                                       const int64_t* __restrict__ blk_off,
+                                                       int64_t* __restrict__ start, int64_t cap,
+                                                       ParseMeta* __restrict__ meta) {
+    uint64_t m;
+    int total;
+    const int64_t p = ((int64_t)blockIdx.x * kLineBS + threadIdx.x) * kLineBytes;
+    int64_t i = blk_off[blockIdx.x] + block_scan_excl<kLineBS>((int)newlines_at(text, size, p, &m), total);
+    for (; m; m &= m - 1, ++i)
+        if (i + 1 < cap) start[i + 1] = p + __builtin_ctzll(m) + 1;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        start[0] = 0;
+        meta->irregular = 0;
+        meta->n_open = 0;
+    }
+}
+
+// Row r of the state from line r + 1: "id,x,y,z,vx,vy,vz" with numbers as the
+// writer prints them, [-]digits[.digits][e[-]digits].  A block's rows are
+// consecutive text, staged through LDS (a thread's own bytes are 100 and more
+// apart).
+constexpr int kParseBS = 128;
+__global__ __launch_bounds__(kParseBS) void k_frame_parse(const char* __restrict__ text, int64_t size,
+                                                         const int64_t* __restrict__ start, int64_t n_lines,
+                                                         int64_t n_rows, uint16_t* __restrict__ ids,
+                                                         double* __restrict__ x, double* __restrict__ v,
+                                                         ParseMeta* __restrict__ meta) {
+    __shared__ __align__(16) char s_txt[kParseBS * kFrameRowMax + 32];
+    const Pow5Tables tb{d_pow5_inv, d_pow5};
+    const int64_t r0 = (int64_t)blockIdx.x * kParseBS, r = r0 + threadIdx.x;
+    const int64_t r1 = r0 + kParseBS < n_rows ? r0 + kParseBS : n_rows;
+    auto line_end = [&](int64_t l) { return l + 1 < n_lines ? start[l + 1] - 1 : (text[size - 1] == '\n' ? size - 1 : size); };
+    const int64_t b0 = start[r0 + 1] & ~(int64_t)15, b1 = line_end(r1);
+    if (b1 - b0 > (int64_t)sizeof s_txt - 16) {
+        if (threadIdx.x == 0) atomicOr(&meta->irregular, 1u);
+        return;
+    }
+    for (int64_t o = threadIdx.x * 16; o < b1 - b0; o += kParseBS * 16)
+        *reinterpret_cast<uint4*>(s_txt + o) = *reinterpret_cast<const uint4*>(text + b0 + o);
+    __syncthreads();
+    if (r >= r1) return;
+    int p = (int)(start[r + 1] - b0);
+    const int e = (int)(line_end(r + 1) - b0);
+    bool bad = false;
+    auto digit = [&](int i) { return i < e ? (uint32_t)(uint8_t)s_txt[i] - 48u : 99u; };  // <= 9: a digit
+    uint32_t id = 0;
+    int nd = 0;
+    for (uint32_t g; (g = digit(p)) <= 9u && nd < 6; ++p, ++nd) id = id * 10u + g;
+    if (nd == 0 || nd > 5 || id > 65535u) bad = true;
+    double val[6];
+    for (int k = 0; k < 6 && !bad; ++k) {
+        if (p >= e || s_txt[p] != ',') bad = true;
+        ++p;
+        const int f0 = p;
+        const bool neg = p < e && s_txt[p] == '-';
+        p += neg ? 1 : 0;
+        uint64_t w = 0;
+        int q = 0, sig = 0, any = 0;
+        uint32_t g;
+        for (; (g = digit(p)) <= 9u; ++p, ++any) {
+            sig += (sig > 0 || g > 0u) ? 1 : 0;
+            if (sig <= 19) w = w * 10u + g;
+        }
+        if (p < e && s_txt[p] == '.') {
+            int frac = 0;
+            for (++p; (g = digit(p)) <= 9u; ++p, ++frac) {
+                sig += (sig > 0 || g > 0u) ? 1 : 0;
+                if (sig <= 19) w = w * 10u + g;
+                --q;
+            }
+            if (frac == 0) bad = true;
+        }
+        if (any == 0 || sig > 19) bad = true;
+        if (p < e && s_txt[p] == 'e') {
+            ++p;
+            const bool en = p < e && s_txt[p] == '-';
+            p += en ? 1 : 0;
+            int x10 = 0, ed = 0;
+            for (; (g = digit(p)) <= 9u && ed < 5; ++p, ++ed) x10 = x10 * 10 + (int)g;
+            if (ed == 0 || ed > 4) bad = true;
+            q += en ? -x10 : x10;
+        }
+        if (bad) break;
+        double d = 0.0;
+        if (!decimal_to_double(w, q, tb, &d)) {
+            const uint32_t o = atomicAdd(&meta->n_open, 1u);
+            if (o < kOpenMax) meta->open[o] = OpenNumber{6 * r + k, b0 + f0, p - f0, 0};
+        }
+        val[k] = neg ? -d : d;
+    }
+    if (bad || p != e) {
+        atomicOr(&meta->irregular, 1u);
+        return;
+    }
+    ids[r] = (uint16_t)id;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        x[3 * r + k] = val[k];
+        v[3 * r + k] = val[3 + k];
+    }
+}
+
 // ------------------------------------------------------------------ host: device text
 
 struct TextScratch {
@@ -400,12 +553,11 @@ struct CsvText {
 };
 
 // lines of text (\n, \r\n), empty ones skipped as the csv reader does
-void split_lines(const std::string& t, std::vector<std::pair<size_t, size_t>>& out) {
+void split_lines(const char* t, size_t n, std::vector<std::pair<size_t, size_t>>& out) {
     size_t i = 0;
-    const size_t n = t.size();
     while (i < n) {
-        const char* nl = (const char*)memchr(t.data() + i, '\n', n - i);
-        size_t e = nl ? (size_t)(nl - t.data()) : n;
+        const char* nl = (const char*)memchr(t + i, '\n', n - i);
+        size_t e = nl ? (size_t)(nl - t) : n;
         size_t ee = e;
         if (ee > i && t[ee - 1] == '\r') --ee;
         if (ee > i) out.emplace_back(i, ee);
@@ -428,14 +580,14 @@ void split_fields(const char* p, size_t n, std::vector<Field>& out) {
         }
 }
 
-bool parse_csv(const std::string& t, CsvText& c) {
+bool parse_csv(const char* t, size_t n, CsvText& c) {
     std::vector<std::pair<size_t, size_t>> lines;
-    split_lines(t, lines);
+    split_lines(t, n, lines);
     c.head.clear();
     c.rows.clear();
     if (lines.empty()) return true;
     std::vector<Field> f;
-    split_fields(t.data() + lines[0].first, lines[0].second - lines[0].first, f);
+    split_fields(t + lines[0].first, lines[0].second - lines[0].first, f);
     for (const Field& x : f) c.head.emplace_back(x.p, x.n);
     c.rows.assign(lines.begin() + 1, lines.end());
     return true;
@@ -474,7 +626,7 @@ bool parse_u64(Field f, uint64_t max, uint64_t* out) {
 }
 
 // rows of numeric columns `cols` parsed in parallel; first error in err
-int parse_rows(const std::string& t, const CsvText& c, const std::vector<int>& cols, int n_int_cols,
+int parse_rows(const char* t, const CsvText& c, const std::vector<int>& cols, int n_int_cols,
                uint64_t int_max, uint64_t* ints, double* dbls, std::string& err) {
     const int64_t n = (int64_t)c.rows.size();
     const int nd = (int)cols.size() - n_int_cols;
@@ -485,7 +637,7 @@ int parse_rows(const std::string& t, const CsvText& c, const std::vector<int>& c
         std::vector<Field> f;
         const int64_t lo = n * tid / nthreads, hi = n * (tid + 1) / nthreads;
         for (int64_t r = lo; r < hi; ++r) {
-            split_fields(t.data() + c.rows[(size_t)r].first, c.rows[(size_t)r].second - c.rows[(size_t)r].first, f);
+            split_fields(t + c.rows[(size_t)r].first, c.rows[(size_t)r].second - c.rows[(size_t)r].first, f);
             if (f.size() != c.head.size()) {
                 errs[(size_t)tid] = "record " + std::to_string(r + 2) + " has " + std::to_string(f.size()) +
                                     " fields, the header " + std::to_string(c.head.size());
@@ -525,7 +677,7 @@ int load_boxes(const std::string& path, std::vector<double>& boxes, std::string&
         return MD_ERR_ARG;
     }
     CsvText c;
-    parse_csv(t, c);
+    parse_csv(t.data(), t.size(), c);
     const std::vector<int> cols = {column(c, "x"), column(c, "y"), column(c, "z")};
     if (!c.rows.empty() && (cols[0] < 0 || cols[1] < 0 || cols[2] < 0)) {
         err = path + ": missing column x, y or z";
@@ -533,7 +685,7 @@ int load_boxes(const std::string& path, std::vector<double>& boxes, std::string&
     }
     boxes.assign(c.rows.size() * 3, 0.0);
     std::string e2;
-    if (parse_rows(t, c, cols, 0, 0, nullptr, boxes.data(), e2)) {
+    if (parse_rows(t.data(), c, cols, 0, 0, nullptr, boxes.data(), e2)) {
         err = path + ": " + e2;
         return MD_ERR_ARG;
     }
@@ -739,6 +891,225 @@ static void fw_release(md_frame_writer* w) {
     delete w;
 }
 
+// ------------------------------------------------------------------ frame reader
+
+// One state file.  Text of at least kDeviceText bytes that starts with the
+// writer's header is parsed on the device, provided that the process drives one
+// already: it has made a context (a program that only reads files would pay the
+// runtime's start, and a child forked from a GPU program cannot use it).
+// StateToSave.load_from_file on the host threads and on the device: 2,300 rows (260
+// KB) 379 us and about 280, 4,600 rows 755 and 319 us, 18,000 rows 2.9 and 0.53
+// ms, 125,000 rows 11.4 and 1.4 ms, 1,000,000 rows 75 and 37 ms (of which the
+// new arrays' and the text's pages are most); two passes over the file and the
+// host parser before took 0.41, 0.82, 3.2, 14.3 and 166 ms.  Stream, memory and
+// copies of the device path cost about 250 us at any size: the line lies above
+// the crossing.
+constexpr size_t kDeviceText = (size_t)256 << 10;
+
+struct md_frame_reader {
+    std::string base, path;
+    int64_t state = 0;
+    char* text = nullptr;  // the file
+    size_t size = 0;
+    int64_t n_rows = 0;
+    CsvText csv;  // lines found on the host
+    bool on_device = false;
+    // device: one allocation, {x, v, ids} of the rows at `out`, numbers left open
+    int device = -1;
+    hipStream_t st = nullptr;
+    char* dev = nullptr;
+    char* out = nullptr;
+    std::vector<OpenNumber> open;
+    ~md_frame_reader();
+};
+
+// The calling thread's device and capture mode for the reader's work: the work
+// is on a stream of its own, so a capture that another thread has under way need
+// not see its allocations.
+struct ReaderScope {
+    int old = -1;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool ok;
+    explicit ReaderScope(int device) {
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        ok = hipGetDevice(&old) == hipSuccess && (old == device || hipSetDevice(device) == hipSuccess);
+    }
+    ~ReaderScope() {
+        if (old >= 0) (void)hipSetDevice(old);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        (void)hipGetLastError();  // a refused allocation is no error of a later call
+    }
+};
+
+static void fr_device_free(md_frame_reader* r) {
+    if (r->device < 0) return;
+    ReaderScope scope(r->device);
+    if (r->dev) (void)hipFreeAsync(r->dev, r->st);
+    if (r->st) {
+        (void)hipStreamSynchronize(r->st);
+        (void)hipStreamDestroy(r->st);
+    }
+    r->dev = nullptr;
+    r->st = nullptr;
+    r->device = -1;
+    r->on_device = false;
+}
+
+md_frame_reader::~md_frame_reader() {
+    fr_device_free(this);
+    free(text);
+}
+
+// the rows parsed on the device; false: no device, or not a file for it
+static bool fr_device_rows(md_frame_reader* r) {
+    const size_t head = sizeof kFrameHeader - 1;
+    if (r->size < kDeviceText || memcmp(r->text, kFrameHeader, head) != 0) return false;
+    r->device = md_context_device();
+    if (r->device < 0) return false;
+    ReaderScope scope(r->device);
+    if (!scope.ok || hipStreamCreateWithFlags(&r->st, hipStreamNonBlocking) != hipSuccess) {
+        r->st = nullptr;
+        return false;
+    }
+    // Line starts for rows of at least 28 bytes (the writer's shortest, 0 as id and
+    // 0.0 six times, has 26; a file of such rows goes to the host).
+    const int64_t size = (int64_t)r->size, cap = size / 28 + 2;
+    const int64_t per = (int64_t)kLineBS * kLineBytes, blocks = (size + per - 1) / per;
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+    const size_t text_b = up(r->size), start_b = up(sizeof(int64_t) * (size_t)cap),
+                 blk_b = up(sizeof(int64_t) * 2 * (size_t)blocks), meta_b = up(sizeof(TextMeta)),
+                 parse_b = up(sizeof(ParseMeta)), out_b = (size_t)cap * (6 * sizeof(double) + sizeof(uint16_t));
+    void* p = nullptr;
+    if (hipMallocAsync(&p, text_b + start_b + blk_b + meta_b + parse_b + out_b, r->st) != hipSuccess) return false;
+    r->dev = (char*)p;
+    int64_t* start = (int64_t*)(r->dev + text_b);
+    int64_t* blk = (int64_t*)((char*)start + start_b);
+    TextMeta* meta = (TextMeta*)((char*)blk + blk_b);
+    ParseMeta* pm = (ParseMeta*)((char*)meta + meta_b);
+    r->out = (char*)pm + parse_b;
+    int64_t newlines = 0;
+    hipError_t e = hipMemcpyAsync(r->dev, r->text, r->size, hipMemcpyHostToDevice, r->st);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_line_count, dim3((unsigned)blocks), dim3(kLineBS), 0, r->st, r->dev, size, blk);
+        hipLaunchKernelGGL(k_text_scan, dim3(1), dim3(kScanBS), 0, r->st, blk, blocks, blk + blocks, meta,
+                           (const RepCtrl*)nullptr);
+        hipLaunchKernelGGL(k_line_fill, dim3((unsigned)blocks), dim3(kLineBS), 0, r->st, r->dev, size, blk + blocks,
+                           start, cap, pm);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(&newlines, &meta->total, sizeof newlines, hipMemcpyDeviceToHost, r->st);
+    const hipError_t e1 = hipStreamSynchronize(r->st);
+    if (e != hipSuccess || e1 != hipSuccess) return false;
+    const int64_t n_lines = newlines + (r->text[r->size - 1] == '\n' ? 0 : 1), n = n_lines - 1;
+    if (n < 1 || newlines + 1 >= cap) return false;
+    double *dx = (double*)r->out, *dv = dx + 3 * n;
+    uint32_t got[2] = {1, 0};
+    hipLaunchKernelGGL(k_frame_parse, dim3((unsigned)((n + kParseBS - 1) / kParseBS)), dim3(kParseBS), 0, r->st, r->dev,
+                       size, start, n_lines, n, (uint16_t*)(dv + 3 * n), dx, dv, pm);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(got, pm, sizeof got, hipMemcpyDeviceToHost, r->st);
+    const hipError_t e2 = hipStreamSynchronize(r->st);
+    if (e != hipSuccess || e2 != hipSuccess || got[0] || got[1] > kOpenMax) return false;
+    r->open.resize(got[1]);
+    if (got[1] && hipMemcpy(r->open.data(), pm->open, sizeof(OpenNumber) * got[1], hipMemcpyDeviceToHost) != hipSuccess)
+        return false;
+    r->n_rows = n;
+    r->on_device = true;
+    return true;
+}
+
+static void fr_host_lines(md_frame_reader* r) {
+    parse_csv(r->text, r->size, r->csv);
+    r->n_rows = (int64_t)r->csv.rows.size();
+}
+
+// rows: they will be asked for (else only their number)
+static int fr_open(md_frame_reader* r, const char* dir, int64_t state, bool rows) {
+    r->base = dir;
+    while (r->base.size() > 1 && r->base.back() == '/') r->base.pop_back();
+    r->state = state;
+    r->path = r->base + "/data/" + std::to_string(state) + ".csv";
+    const int fd = open(r->path.c_str(), O_RDONLY);
+    struct stat stt;
+    bool ok = fd >= 0 && fstat(fd, &stt) == 0;
+    size_t cap = 0;
+    while (ok) {
+        if (r->size == cap) {  // first: the file's size and a byte more, to see its end
+            cap = cap ? 2 * cap : (stt.st_size > 0 ? (size_t)stt.st_size : (size_t)65535) + 1;
+            char* t = (char*)realloc(r->text, cap);
+            if (!(ok = t != nullptr)) break;
+            r->text = t;
+        }
+        const ssize_t n = read(fd, r->text + r->size, cap - r->size);
+        if (n < 0 && errno == EINTR) continue;
+        ok = n >= 0;
+        if (n <= 0) break;
+        r->size += (size_t)n;
+    }
+    if (fd >= 0) close(fd);
+    if (!ok) return err_out(MD_ERR_ARG, "cannot read " + r->path);
+    if (rows && fr_device_rows(r)) return MD_OK;
+    fr_device_free(r);
+    fr_host_lines(r);
+    return MD_OK;
+}
+
+// bb.csv row `state` (StateToSave::load_bb, save_data.rs:186-190)
+static int fr_box(const std::string& base, int64_t state, double* box) {
+    std::vector<double> boxes;
+    std::string err;
+    if (load_boxes(base + "/bb.csv", boxes, err)) return err_out(MD_ERR_ARG, err);
+    if ((size_t)state >= boxes.size() / 3) return err_out(MD_ERR_ARG, "bb.csv has no row " + std::to_string(state));
+    for (int k = 0; k < 3; ++k) box[k] = boxes[(size_t)state * 3 + k];
+    return MD_OK;
+}
+
+// the arrays from the device; false: left to the host
+static bool fr_fetch(md_frame_reader* r, uint16_t* ids, double* x, double* v) {
+    const size_t n = (size_t)r->n_rows, xyz = sizeof(double) * 3 * n;
+    ReaderScope scope(r->device);
+    if (!scope.ok) return false;
+    hipError_t e = hipMemcpyAsync(x, r->out, xyz, hipMemcpyDeviceToHost, r->st);
+    if (e == hipSuccess) e = hipMemcpyAsync(v, r->out + xyz, xyz, hipMemcpyDeviceToHost, r->st);
+    if (e == hipSuccess) e = hipMemcpyAsync(ids, r->out + 2 * xyz, sizeof(uint16_t) * n, hipMemcpyDeviceToHost, r->st);
+    const hipError_t e2 = hipStreamSynchronize(r->st);
+    if (e != hipSuccess || e2 != hipSuccess) return false;
+    for (const OpenNumber& o : r->open) {
+        double d;
+        if (!parse_f64(Field{r->text + o.off, (size_t)o.len}, &d)) return false;
+        (o.at % 6 < 3 ? x : v)[o.at / 6 * 3 + o.at % 3] = d;
+    }
+    return true;
+}
+
+static int fr_rows(md_frame_reader* r, uint16_t* ids, double* x, double* v) {
+    if (r->on_device) {
+        if (fr_fetch(r, ids, x, v)) return MD_OK;
+        fr_device_free(r);
+        fr_host_lines(r);  // as many rows: the device takes no text with empty lines
+    }
+    const char* names[7] = {"id", "position_x", "position_y", "position_z", "velocity_x", "velocity_y", "velocity_z"};
+    std::vector<int> cols;
+    for (const char* nm : names) {
+        cols.push_back(column(r->csv, nm));
+        if (r->csv.rows.size() && cols.back() < 0) return err_out(MD_ERR_ARG, r->path + ": missing column " + nm);
+    }
+    const size_t n = r->csv.rows.size();
+    std::vector<uint64_t> id64(n);
+    std::vector<double> vals(n * 6);
+    std::string err;
+    if (parse_rows(r->text, r->csv, cols, 1, 65535, id64.data(), vals.data(), err))
+        return err_out(MD_ERR_ARG, r->path + ": " + err);
+    for (size_t i = 0; i < n; ++i) {
+        ids[i] = (uint16_t)id64[i];
+        for (int k = 0; k < 3; ++k) {
+            x[3 * i + k] = vals[6 * i + k];
+            v[3 * i + k] = vals[6 * i + 3 + k];
+        }
+    }
+    return MD_OK;
+}
+
 extern "C" {
 
 int md_text_create(md_text** out) {
@@ -921,47 +1292,45 @@ void md_frame_writer_destroy(md_frame_writer* w) {
     fw_release(w);
 }
 
+int md_frame_reader_open(md_frame_reader** out, const char* dir, int64_t state_number, int64_t* n_rows) {
+    if (!out || !dir || !n_rows || state_number < 0) return err_out(MD_ERR_ARG, "bad argument");
+    *out = nullptr;
+    md_frame_reader* r = new md_frame_reader();
+    const int rc = fr_open(r, dir, state_number, true);
+    if (rc) {
+        delete r;
+        return rc;
+    }
+    *n_rows = r->n_rows;
+    *out = r;
+    return MD_OK;
+}
+
+int md_frame_reader_read(md_frame_reader* r, uint16_t* ids, double* x, double* v, double* box) {
+    if (!r || !ids || !x || !v) return err_out(MD_ERR_ARG, "bad argument");
+    if (box) {
+        const int rc = fr_box(r->base, r->state, box);
+        if (rc) return rc;
+    }
+    return fr_rows(r, ids, x, v);
+}
+
+void md_frame_reader_close(md_frame_reader* r) { delete r; }
+
 int md_frame_load(const char* dir, int64_t state_number, int64_t cap, int64_t* n_rows, uint16_t* ids, double* x,
                   double* v, double* box) {
     if (!dir || !n_rows || state_number < 0) return err_out(MD_ERR_ARG, "bad argument");
+    md_frame_reader r;
+    int rc;
     std::string base(dir);
     while (base.size() > 1 && base.back() == '/') base.pop_back();
-    std::string err;
-    // bb.csv row state_number (StateToSave::load_bb, save_data.rs:186-190)
-    if (box) {
-        std::vector<double> boxes;
-        if (load_boxes(base + "/bb.csv", boxes, err)) return err_out(MD_ERR_ARG, err);
-        if ((size_t)state_number >= boxes.size() / 3)
-            return err_out(MD_ERR_ARG, "bb.csv has no row " + std::to_string(state_number));
-        for (int k = 0; k < 3; ++k) box[k] = boxes[(size_t)state_number * 3 + k];
-    }
-    const std::string path = base + "/data/" + std::to_string(state_number) + ".csv";
-    std::string t;
-    if (!read_file(path, t)) return err_out(MD_ERR_ARG, "cannot read " + path);
-    CsvText c;
-    parse_csv(t, c);
-    *n_rows = (int64_t)c.rows.size();
+    if (box && (rc = fr_box(base, state_number, box))) return rc;
+    if ((rc = fr_open(&r, dir, state_number, ids && x && v))) return rc;
+    *n_rows = r.n_rows;
     if (!ids && !x && !v) return MD_OK;
     if (!ids || !x || !v) return err_out(MD_ERR_ARG, "ids, x and v are given together");
     if (cap < *n_rows) return err_out(MD_ERR_ARG, "capacity below the row count");
-    const char* names[7] = {"id", "position_x", "position_y", "position_z", "velocity_x", "velocity_y", "velocity_z"};
-    std::vector<int> cols;
-    for (const char* nm : names) {
-        cols.push_back(column(c, nm));
-        if (c.rows.size() && cols.back() < 0) return err_out(MD_ERR_ARG, path + ": missing column " + nm);
-    }
-    const size_t n = c.rows.size();
-    std::vector<uint64_t> id64(n);
-    std::vector<double> vals(n * 6);
-    if (parse_rows(t, c, cols, 1, 65535, id64.data(), vals.data(), err)) return err_out(MD_ERR_ARG, path + ": " + err);
-    for (size_t i = 0; i < n; ++i) {
-        ids[i] = (uint16_t)id64[i];
-        for (int k = 0; k < 3; ++k) {
-            x[3 * i + k] = vals[6 * i + k];
-            v[3 * i + k] = vals[6 * i + 3 + k];
-        }
-    }
-    return MD_OK;
+    return fr_rows(&r, ids, x, v);
 }
 
 }  // extern "C"

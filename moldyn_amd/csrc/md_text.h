@@ -304,4 +304,61 @@ MD_TEXT_FN int uint_text(uint64_t v, Out out) {
     return n;
 }
 
+// ------------------------------------------------------------------ decimal to double
+
+// w 10^q correctly rounded (ties to even), w < 2^64.  Returns false where the
+// precision at hand does not decide it (a tie or all but one, a subnormal or
+// overflowing result, an exponent outside the tables): the caller takes an exact
+// parser.  From the mathematics: w times the 125-bit power of 5 is within
+// w < 2^64 units of the exact product, which after normalisation to 192 bits is
+// less than 2^69 units; the 53-bit result is followed by 139 bits, so only a
+// rest whose first 64 bits are one half, or one unit below, is undecided.
+__host__ __device__ inline bool decimal_to_double(uint64_t w, int q, const Pow5Tables& tb, double* out) {
+    if (w == 0) {
+        *out = 0.0;
+        return true;
+    }
+    if (w < (1ull << 53) && q >= -22 && q <= 22) {
+        // both factors exact: one IEEE operation rounds correctly
+        double p = 1.0;
+        for (int k = q < 0 ? -q : q; k > 0; --k) p *= 10.0;
+        *out = q < 0 ? (double)w / p : (double)w * p;
+        return true;
+    }
+    const int k = q < 0 ? -q : q;
+    if (q < 0 ? k >= MD_POW5_INV_COUNT : k >= MD_POW5_COUNT) return false;
+    const uint64_t lo = q < 0 ? tb.inv[k][0] : tb.pos[k][0], hi = q < 0 ? tb.inv[k][1] : tb.pos[k][1];
+    const int bits5 = ((k * 1217359) >> 19) + 1;  // of 5^k
+    int e = q < 0 ? -(bits5 - 1 + 125) - k : bits5 - 125 + k;
+    const unsigned __int128 a = (unsigned __int128)lo * w, b = (unsigned __int128)hi * w;
+    uint64_t n0 = (uint64_t)a;
+    const unsigned __int128 c = (a >> 64) + (uint64_t)b;
+    uint64_t n1 = (uint64_t)c, n2 = (uint64_t)(b >> 64) + (uint64_t)(c >> 64);
+    if (n2 == 0) {
+        n2 = n1;
+        n1 = n0;
+        n0 = 0;
+        e -= 64;
+    }
+    int lz = 0;
+    while (!(n2 >> 63)) {  // at most 63 (short numbers with long exponents)
+        n2 = (n2 << 1) | (n1 >> 63);
+        n1 = (n1 << 1) | (n0 >> 63);
+        n0 <<= 1;
+        ++lz;
+    }
+    e += 191 - lz;  // of the leading bit
+    uint64_t m = n2 >> 11;
+    const uint64_t f = (n2 << 53) | (n1 >> 11), half = 1ull << 63;
+    if (f == half || f == half - 1) return false;
+    if (f > half && ++m >> 53) {
+        m >>= 1;
+        ++e;
+    }
+    if (e < -1022 || e > 1023) return false;
+    const uint64_t u = ((uint64_t)(e + 1023) << 52) | (m & ((1ull << 52) - 1));
+    __builtin_memcpy(out, &u, sizeof u);
+    return true;
+}
+
 }  // namespace md

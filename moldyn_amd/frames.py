@@ -221,20 +221,23 @@ class StateToSave:
 
     @classmethod
     def load_from_file(cls, path, state_number):
-        """save_data.rs:215-229 (md_frame_load)."""
+        """save_data.rs:215-229 (md_frame_reader_*)."""
         lib = L.load()
-        p = os.fsencode(str(path))
         n = C.c_int64()
-        if lib.md_frame_load(p, int(state_number), 0, C.byref(n), None, None, None, None) != 0:
-            raise L.MdError(L.MD_ERR_ARG, lib.md_global_error().decode())
-        ids = np.zeros(n.value, dtype=np.uint16)
-        x = np.zeros((n.value, 3))
-        v = np.zeros((n.value, 3))
-        box = np.zeros(3)
-        rc = lib.md_frame_load(p, int(state_number), n.value, C.byref(n),
-                               ids.ctypes.data_as(C.POINTER(C.c_uint16)), _dp(x), _dp(v), _dp(box))
+        h = C.c_void_p()
+        rc = lib.md_frame_reader_open(C.byref(h), os.fsencode(str(path)), int(state_number), C.byref(n))
         if rc != 0:
             raise L.MdError(rc, lib.md_global_error().decode())
+        try:
+            ids = np.empty(n.value, dtype=np.uint16)
+            x = np.empty((n.value, 3))
+            v = np.empty((n.value, 3))
+            box = np.zeros(3)
+            rc = lib.md_frame_reader_read(h, ids.ctypes.data_as(C.POINTER(C.c_uint16)), _dp(x), _dp(v), _dp(box))
+            if rc != 0:
+                raise L.MdError(rc, lib.md_global_error().decode())
+        finally:
+            lib.md_frame_reader_close(h)
         return cls(ids, x, v, box)
 
     def into_state(self, masses):
