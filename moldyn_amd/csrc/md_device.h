@@ -215,7 +215,7 @@ struct MlpStat {
 struct DevState {
     void* rec[2];            // Rec<float> or Rec<double>, n_slots each
     CRec* crec[2];           // step records of the list path (null on the other paths)
-    double4* dpos;           // dense list path: every slot's drifted position (x, y, z, unused)
+    double4* dpos;           // dense list path: every slot's drifted position and type (x, y, z, type)
     const uint8_t* slot_type;  // type of every slot (padding slots: the group's type)
     int32_t compact;         // the list path steps on crec (k_fin builds from crec)
     float4* cpos;            // list paths: FP32 position of every slot at the last grid fill (dense systems)

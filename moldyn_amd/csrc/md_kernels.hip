@@ -797,6 +797,20 @@ constexpr int wave_scratch_bytes() {
     return 64 * (3 * (int)sizeof(double) + (int)sizeof(typename Acc<FT>::Terms) + 2 * (int)sizeof(int32_t) + 1);
 }
 
+// Entries of its own list that a lane takes at a time in a dense system: their
+// positions are gathered together, the next ones' indices loaded before the
+// terms are computed, and the terms, computed for every entry (an entry past
+// the end repeats the last one) and added in list order where they count, leave
+// the scheduler independent chains.  Bound by these chains: with one wave per
+// SIMD (35,937 particles) nothing else covers them.  One entry at a time, with
+// branches in the minimum image, a division per quotient and the parameters of
+// several types read from memory in three steps, k_step took 49.7 us a launch
+// for 35,937 FP64 particles of two types, 167 for 262,144 and 514 for 1,000,000;
+// this 25.2, 91 and 419; one FP32 type 52 us for 262,144, 191 for 1,000,000;
+// this 39.8 and 139.  FP64 depth 3: 24.0, 98 and 430; FP32 depth 2, 3, 6: 42.2,
+// 39.4, 43.4 for 262,144 and 3: 18.1 against 17.4 for 13,824.
+constexpr int kWalkDepth64 = 2, kWalkDepth32 = 4;
+
 // The list forces of a wave's particles (potential.rs:158-216 over the Verlet
 // lists at the drifted positions).  In sparse systems (!WALK) each lane takes
 // its particle's first entry, whose record the caller gathered a tile ahead
@@ -813,8 +827,8 @@ constexpr int wave_scratch_bytes() {
 template <typename FT, bool MULTI, bool WALK>
 __device__ __forceinline__ Acc<FT> wave_list_forces(const DevState& d, const CRec* __restrict__ src, char* wreg,
                                                     int n_mine, const CRec& o0, int tj0, int32_t e0, int64_t s,
-                                                    double x1, double y1, double z1, int ti, bool split, double lam,
-                                                    double dt, double bx, double by, double bz,
+                                                    double x1, double y1, double z1, const PairParam* prow, bool split,
+                                                    double lam,                                                    double dt, double bx, double by, double bz,
                                                     const PairParam& p0) {
     typedef typename Acc<FT>::Terms Terms;
     constexpr int W = 64;
@@ -835,11 +849,11 @@ __device__ __forceinline__ Acc<FT> wave_list_forces(const DevState& d, const CRe
             yj = wrap1(yj + (o.uy * lam) * dt, by);
             zj = wrap1(zj + (o.uz * lam) * dt, bz);
         }
-        const double dx = min_image(xj - xi, bx);
-        const double dy = min_image(yj - yi, by);
-        const double dz = min_image(zj - zi, bz);
+        const double dx = min_image_s(xj - xi, bx);
+        const double dy = min_image_s(yj - yi, by);
+        const double dz = min_image_s(zj - zi, bz);
         const double r2 = (dx * dx + dy * dy) + dz * dz;
-        const PairParam& pp = MULTI ? d.pairs[ti * d.n_types + tj] : p0;
+        const PairParam& pp = MULTI ? prow[tj] : p0;
         if (!(r2 <= pp.r2max)) return false;
         tm = Acc<FT>::terms(dx, dy, dz, r2, pp);
         return true;
@@ -854,7 +868,7 @@ __device__ __forceinline__ Acc<FT> wave_list_forces(const DevState& d, const CRe
             o.y = q.y;
             o.z = q.z;
             o.ux = o.uy = o.uz = 0.0;
-            return pair(o, MULTI ? (int)d.slot_type[j] : 0, xi, yi, zi, tm, false);
+            return pair(o, MULTI ? (int)q.w : 0, xi, yi, zi, tm, false);
         } else {
             const CRec o = src[j];  // one copy: the record loads as whole 16-byte words
             return pair(o, MULTI ? (int)d.slot_type[j] : 0, xi, yi, zi, tm, !split);
@@ -872,10 +886,37 @@ __device__ __forceinline__ Acc<FT> wave_list_forces(const DevState& d, const CRe
         // at most one entry per lane, or long lists: each lane walks its own
         // list; entry k of the wave's particles is one coalesced row of the
         // column-major lists
-        for (int k = 0; k < n_mine; ++k) {
-            const int32_t j = k == 0 ? e0 : d.nbr[(int64_t)k * d.n_slots + s];
-            Terms tm;
-            if (gathered(j, x1, y1, z1, tm)) acc.add_terms(tm);
+        constexpr int D = sizeof(FT) == 8 ? kWalkDepth64 : kWalkDepth32;
+        const int32_t* const row = d.nbr + s;
+        const int last = n_mine > 0 ? n_mine - 1 : 0;
+        int32_t jn[D];
+        jn[0] = e0;
+#pragma unroll
+        for (int u = 1; u < D; ++u) jn[u] = row[(int64_t)(u < last ? u : last) * d.n_slots];
+        for (int k = 0; k < n_mine; k += D) {
+            double4 q[D];
+#pragma unroll
+            for (int u = 0; u < D; ++u) q[u] = d.dpos[jn[u]];
+#pragma unroll
+            for (int u = 0; u < D; ++u) {
+                const int kn = k + D + u;
+                jn[u] = row[(int64_t)(kn < last ? kn : last) * d.n_slots];
+            }
+            Terms tm[D];
+            bool ok[D];
+#pragma unroll
+            for (int u = 0; u < D; ++u) {
+                const double dx = min_image_s(q[u].x - x1, bx);
+                const double dy = min_image_s(q[u].y - y1, by);
+                const double dz = min_image_s(q[u].z - z1, bz);
+                const double r2 = (dx * dx + dy * dy) + dz * dz;
+                const PairParam& pp = MULTI ? prow[(int)q[u].w] : p0;
+                ok[u] = r2 <= pp.r2max && k + u < n_mine;
+                tm[u] = Acc<FT>::terms(dx, dy, dz, r2, pp);
+            }
+#pragma unroll
+            for (int u = 0; u < D; ++u)
+                if (ok[u]) acc.add_terms(tm[u]);
         }
         return acc;
     }
@@ -919,8 +960,11 @@ __device__ __forceinline__ Acc<FT> wave_list_forces(const DevState& d, const CRe
 // starts.
 // The last step of a chunk also writes the full records (x, v, F) and the
 // per-particle energies.
+// FP64 in dense systems takes the registers of two waves per SIMD: at four it
+// keeps part of the walk in scratch (262,144 particles of two types 99 us a
+// launch, 91 so; FP32 loses, 47 against 43 us).
 template <typename FT, int BS, bool MULTI, bool DENSE>
-__global__ __launch_bounds__(BS, 4) void k_step(DevState d) {
+__global__ __launch_bounds__(BS, DENSE && sizeof(FT) == 8 ? 2 : 4) void k_step(DevState d) {
     const int b = xcd_block(blockIdx.x, gridDim.x);
     const int gi = d.blk_group[b];
     const GroupInfo G = d.groups[gi];
@@ -1001,6 +1045,12 @@ __global__ __launch_bounds__(BS, 4) void k_step(DevState d) {
     // the chunk's starting state
     Rec<FT>* __restrict__ full = (Rec<FT>*)d.rec[P.full_dst & 1];
     const PairParam p0 = wave_uniform(d.pairs[0]);
+    // several types: the pair parameters of the block's type
+    __shared__ PairParam s_pair[MULTI ? kMaxTypes : 1];
+    if (MULTI) {
+        if (lane < d.n_types) s_pair[lane] = d.pairs[ti * d.n_types + lane];
+        __syncthreads();
+    }
     int visits = 0;  // list entries read by this thread (profiling)
     // A wave's 64 records move between HBM and LDS as whole 16-byte words
     // with consecutive lanes on consecutive words (fully coalesced); each
@@ -1087,7 +1137,7 @@ __global__ __launch_bounds__(BS, 4) void k_step(DevState d) {
             }
         }
         const Acc<FT> acc = wave_list_forces<FT, MULTI, DENSE>(d, src, wreg, valid ? nn : 0, o0, tj0, e0, s, x1, y1,
-                                                               z1, ti, split, lam, dt, bx, by, bz, p0);
+                                                               z1, s_pair, split, lam, dt, bx, by, bz, p0);
         if (valid) {
             // integrator.rs:47-53 second half kick, barostat.rs:45-48 scale
             const double vx = v1x + (double)acc.fx * c;
@@ -2300,7 +2350,7 @@ __global__ __launch_bounds__(BS) void k_dpos(DevState d) {
             q.y = wrap1(a.y + (a.uy * lam) * dt, by);
             q.z = wrap1(a.z + (a.uz * lam) * dt, bz);
         }
-        q.w = 0.0;
+        q.w = (double)G.type;
         d.dpos[s] = q;
     }
 }
