@@ -19,6 +19,7 @@
 //    fill can run while the other buffer is being read.  Lists are built from
 //    it brick by brick: a block stages a brick of cells plus a one-cell halo
 //    (ids and positions) in LDS and builds the lists of the brick's atoms.
+//    Dense systems take a wave per cell instead, candidates in registers.
 //  * the per-replica control blocks are double-buffered by launch parity:
 //    every kernel of a launch reads buffer `par`, the finalize writes
 //    `par ^ 1`, so blocks of the same kernel never see a half-updated block.
