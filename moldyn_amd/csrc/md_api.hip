@@ -75,6 +75,9 @@ struct md_ctx {
     void* snap = nullptr;
     RepCtrl* snap_ctrl = nullptr;
     bool fp32 = true, list_mode = true;
+    // all of the layout's arrays, and of the lists', are allocated (at these capacities)
+    bool base_ready = false, lists_ready = false;
+    int list_cap_have = 0, cell_cap_have = 0;
     bool sums_valid = false;
     double last_dt = 0.002;
     double rlist = 0.0, rc_max = 0.0;
@@ -234,9 +237,11 @@ static int dalloc(md_ctx* c, DevPool& owner, void** p, size_t bytes) {
     const bool slab = bytes <= kSlabMost;
     void* q = nullptr;
     hipError_t e = hipMalloc(&q, slab ? kSlab : bytes);
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // reported here, no error of the next launch
         return fail(c, MD_ERR_NOMEM, std::string("hipMalloc(") + std::to_string(slab ? kSlab : bytes) +
                                          "): " + hipGetErrorString(e));
+    }
     owner.blocks.push_back(q);
     *p = q;
     if (slab) {
@@ -261,6 +266,7 @@ static void drop_graph(md_ctx* c) {
 
 static void free_all(md_ctx* c) {
     drop_graph(c);
+    c->base_ready = c->lists_ready = false;
     free_list(c->list_allocs);
     free_list(c->base_allocs);
     c->snap = nullptr;  // in base_allocs
@@ -389,6 +395,7 @@ static int auto_capacities(md_ctx* c) {
 }
 
 static int alloc_lists(md_ctx* c) {
+    c->lists_ready = false;
     free_list(c->list_allocs);
     drop_graph(c);
     // the cleared headers match no epoch; the control blocks keep counting
@@ -397,11 +404,12 @@ static int alloc_lists(md_ctx* c) {
     int rc;
     c->d.mlp_nbr = nullptr;
     c->d.mlp_ncount = nullptr;
+    c->d.nbr = nullptr;
+    c->d.ncount = nullptr;
+    c->d.cell_hdr[0] = c->d.cell_hdr[1] = nullptr;
+    c->d.cell_slots[0] = c->d.cell_slots[1] = nullptr;
     if (!c->list_mode) {
-        c->d.nbr = nullptr;
-        c->d.ncount = nullptr;
-        c->d.cell_hdr[0] = c->d.cell_hdr[1] = nullptr;
-        c->d.cell_slots[0] = c->d.cell_slots[1] = nullptr;
+        c->lists_ready = true;
         return MD_OK;
     }
     const int64_t N = c->n_slots;
@@ -428,7 +436,17 @@ static int alloc_lists(md_ctx* c) {
             return rc;
         c->d.cell_slots[k] = (int32_t*)p;
     }
+    c->list_cap_have = c->d.list_cap;
+    c->cell_cap_have = c->d.cell_cap;
+    c->lists_ready = true;
     return MD_OK;
+}
+
+// After an allocation that failed, a call that needs the arrays is refused
+// until md_set_options has allocated them.
+static int need_arrays(md_ctx* c, bool lists) {
+    if (c->base_ready && (c->lists_ready || !lists)) return MD_OK;
+    return fail(c, MD_ERR_NOMEM, "an allocation of this context failed: set its options again");
 }
 
 static int upload_pairs(md_ctx* c) {
@@ -584,6 +602,7 @@ static int alloc_base(md_ctx* c) {
     if ((rc = alloc_lists(c))) return rc;
     if ((rc = alloc_mlp(c))) return rc;
     HIPCHK(c, hipStreamSynchronize(c->st));
+    c->base_ready = true;
     return MD_OK;
 }
 
@@ -747,8 +766,9 @@ static int reduce_state_sums(md_ctx* c, int passes) {
 
 static int ensure_sums(md_ctx* c) {
     if (c->sums_valid) return MD_OK;
-    std::vector<RepParams> P((size_t)c->R, base_params(c));
     int rc;
+    if ((rc = need_arrays(c, false))) return rc;
+    std::vector<RepParams> P((size_t)c->R, base_params(c));
     if ((rc = write_params(c, P))) return rc;
     if ((rc = reduce_state_sums(c, 2))) return rc;
     HIPCHK(c, hipStreamSynchronize(c->st));
@@ -1081,6 +1101,8 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
                      bool per_rep) {
     if (n < 0) return fail(c, MD_ERR_ARG, "n_steps < 0");
     if (n == 0) return MD_OK;
+    int rc;
+    if ((rc = need_arrays(c, true))) return rc;
     c->blank = false;
     if (c->mlp && !c->mlp_ready) return fail(c, MD_ERR_ARG, "surrogate parameters not set (md_mlp_set_params)");
     for (int r = 0; r < c->R; ++r) {
@@ -1095,7 +1117,6 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
         if (G.count == 0)
             return fail(c, MD_ERR_ARG, "a particle type has no particles (the reference indexes particle_type[0])");
     c->last_dt = dt;
-    int rc;
     if ((rc = ensure_sums(c))) return rc;
     std::vector<RepCtrl> C;
     if ((rc = read_ctrl(c, C))) return rc;
@@ -1292,6 +1313,8 @@ void md_set_global_error(const std::string& msg) { g_error = msg; }
 int md_frame_source(md_ctx* c, int replica, md::FrameSource* out) {
     if (!c || !out) return MD_ERR_ARG;
     if (replica < 0 || replica >= c->R) return fail(c, MD_ERR_ARG, "bad replica");
+    const int rc = need_arrays(c, false);
+    if (rc) return rc;
     md::FrameSource& s = *out;
     s = md::FrameSource{};
     s.st = c->st;
@@ -1456,6 +1479,7 @@ static int io_run(md_ctx* c, double* const (&host)[5], bool put, Launch launch) 
     c->d.par = c->par;
     const bool pinned = per > 0 && (size_t)n * per <= kIoPinned;
     int rc;
+    if ((rc = need_arrays(c, false))) return rc;
     if (pinned) {
         if ((rc = pinned_staging(c))) return rc;
     } else if (per > 0) {
@@ -1639,13 +1663,15 @@ int md_download_state(md_ctx* c, double* x, double* v, double* force, double* po
 
 // Relayout keeping the state (used when block size / force path change).
 static int relayout(md_ctx* c, const md_options& nopt) {
-    if (c->blank) {
+    if (c->blank || !c->base_ready) {
         // nothing to carry over
         const std::vector<double> box(c->box0);
         c->opt = nopt;
         c->bs = nopt.block_size;
         int rc = alloc_base(c);
-        return rc ? rc : put_state(c, nullptr, nullptr, box.data());
+        if (rc || (rc = put_state(c, nullptr, nullptr, box.data()))) return rc;
+        c->blank = true;
+        return MD_OK;
     }
     const int64_t n = c->n_atoms;
     std::vector<double> x((size_t)n * 3 + 1), v((size_t)n * 3 + 1), f((size_t)n * 3 + 1),
@@ -1700,20 +1726,21 @@ int md_set_options(md_ctx* c, const md_options* o) {
     c->crec_valid = false;
     const bool relay = n.block_size != c->opt.block_size || n.force_mode != c->opt.force_mode ||
                        n.cells_per_atom != c->opt.cells_per_atom ||
-                       n.tiles_per_block != c->opt.tiles_per_block;
+                       n.tiles_per_block != c->opt.tiles_per_block || !c->base_ready;
     if (relay) {
         int rc = relayout(c, n);
         if (rc) return rc;
     } else {
         c->opt = n;
     }
-    const int lc = c->d.list_cap, cc = c->d.cell_cap;  // of the lists as they are allocated
     rebuild_pairs(c);
     if (n.list_capacity > 0) c->d.list_cap = n.list_capacity;
     if (n.cell_capacity > 0) c->d.cell_cap = n.cell_capacity;
     if (n.list_capacity <= 0 || n.cell_capacity <= 0) auto_capacities(c);
     int rc = MD_OK;
-    if ((c->d.list_cap != lc || c->d.cell_cap != cc) && (rc = alloc_lists(c))) return rc;
+    const bool have = c->lists_ready && (!c->list_mode || (c->d.list_cap == c->list_cap_have &&
+                                                           c->d.cell_cap == c->cell_cap_have));
+    if (!have && (rc = alloc_lists(c))) return rc;
     rc = upload_pairs(c);
     if (rc) return rc;
     std::vector<RepCtrl> C;
@@ -1757,13 +1784,14 @@ int md_set_pair_potential_lj(md_ctx* c, uint16_t t0, uint16_t t1, double sigma, 
 
 int md_update_force(md_ctx* c) {
     if (!c) return MD_ERR_ARG;
+    int rc = need_arrays(c, true);
+    if (rc) return rc;
     c->blank = false;
     c->crec_valid = false;
     if (c->mlp && !c->mlp_ready) return fail(c, MD_ERR_ARG, "surrogate parameters not set (md_mlp_set_params)");
     if (c->list_mode) return list_force_eval(c);
     std::vector<RepParams> P((size_t)c->R, base_params(c));
-    int rc = write_params(c, P);
-    if (rc) return rc;
+    if ((rc = write_params(c, P))) return rc;
     std::vector<RepCtrl> C;
     if ((rc = read_ctrl(c, C))) return rc;
     if ((rc = choose_instances(c, C, false))) return rc;
@@ -1783,6 +1811,8 @@ int md_update_force(md_ctx* c) {
 
 int md_apply_boundary_conditions(md_ctx* c) {
     if (!c) return MD_ERR_ARG;
+    const int rc = need_arrays(c, false);
+    if (rc) return rc;
     c->blank = false;
     c->crec_valid = false;
     c->d.par = c->par;
@@ -1898,13 +1928,14 @@ int md_barostat_update(md_ctx* c, md_barostat* ba, uint16_t type_id) {
     if (!c || !ba || type_id >= c->T) return fail(c, MD_ERR_ARG, "bad argument");
     if (ba->kind == 2) return fail(c, MD_ERR_UNIMPLEMENTED, "Barostat::Custom is todo!() in the reference");
     if (ba->kind != 1) return MD_OK;
+    int rc = need_arrays(c, false);
+    if (rc) return rc;
     c->blank = c->crec_valid = false;
     const GroupInfo& G = c->groups[c->reps[0].first_group + type_id];
     c->d.par = c->par;
     HIPCHK(c, launch_scale(c->d, c->fp32, G.start, G.count, ba->myu, 1, c->st));
     std::vector<RepCtrl> C;
-    int rc = read_ctrl(c, C);
-    if (rc) return rc;
+    if ((rc = read_ctrl(c, C))) return rc;
     for (int k = 0; k < 3; ++k) C[0].box[k] *= ba->myu;
     C[0].flags &= ~(F_HAVE_LIST | F_GRID_FRESH);
     c->sums_valid = false;
@@ -1989,6 +2020,8 @@ int md_init_mb_velocities(double* vel, int64_t n, double temperature, double mas
 // boxes; a context that never held a state gets the blank one first
 // (initialize_particles).
 static int edit_begin(md_ctx* c, std::vector<int>& cur, std::vector<double>& boxes) {
+    int rc = need_arrays(c, false);
+    if (rc) return rc;
     c->blank = false;
     boxes.assign((size_t)c->R * 3, 0.0);
     cur.assign(c->R, 0);
@@ -2000,8 +2033,7 @@ static int edit_begin(md_ctx* c, std::vector<int>& cur, std::vector<double>& box
         return reset_controls(c, boxes.data(), 0);
     }
     std::vector<RepCtrl> C;
-    int rc = read_ctrl(c, C);
-    if (rc) return rc;
+    if ((rc = read_ctrl(c, C))) return rc;
     for (int r = 0; r < c->R; ++r) {
         cur[r] = C[(size_t)r].cur & 1;
         for (int k = 0; k < 3; ++k) boxes[(size_t)r * 3 + k] = C[(size_t)r].box[k];
@@ -2084,7 +2116,7 @@ int md_get_stats(md_ctx* c, md_stats* out) {
     s.mean_list_len = 0.0;
     s.max_list_len = 0;
     s.list_visits = c->list_visits;
-    if (c->list_mode && c->n_slots > 0) {
+    if (c->list_mode && c->lists_ready && c->n_slots > 0) {
         std::vector<int32_t> nc((size_t)c->n_slots);
         if (hipMemcpy(nc.data(), c->d.ncount, sizeof(int32_t) * nc.size(), hipMemcpyDeviceToHost) == hipSuccess) {
             double sum = 0;
