@@ -132,6 +132,7 @@ struct md_ctx {
     size_t io_cap = 0;
     void* io_pin = nullptr;
     void* io_pin_dev = nullptr;
+    size_t io_pin_cap = 0;
     // host copy of the control blocks the next launch reads, valid while no
     // finalize, graph replay, snapshot restore or layout change has run since
     std::vector<RepCtrl> ctrl_cache;
@@ -612,7 +613,8 @@ static RepCtrl* ctrl_cur(md_ctx* c) { return c->d.ctrl + (size_t)c->par * c->R; 
 // States up to kIoPinned bytes pass through pinned host memory that the kernels
 // read and write themselves: one launch and no copy operation (a step and a
 // download of 1,000 atoms: 57 -> 44 us with the above).  Larger ones are copied between the
-// caller's arrays and device staging, at most kIoBytes at a time.
+// caller's arrays and device staging, at most kIoBytes at a time, or, where the
+// device has no room for that, go through the pinned memory in pieces.
 constexpr size_t kIoPinned = (size_t)256 << 10, kIoBytes = (size_t)128 << 20;
 
 // Systems up to this many slots leave the state of a call's last step in host
@@ -657,6 +659,7 @@ static int pinned_staging(md_ctx* c) {
     c->h_done = (uint32_t*)take(256, (void**)&c->d.h_done);
     *c->h_done = 0;
     c->io_pin = take(io, &c->io_pin_dev);
+    c->io_pin_cap = io;
     c->h_rec = mirror ? take(rec, &c->d.h_rec) : nullptr;
     c->h_pv = mirror ? (double*)take(pv, (void**)&c->d.h_pv) : nullptr;
     HIPCHK(c, hipEventCreateWithFlags(&c->params_ev, hipEventDisableTiming));
@@ -1477,25 +1480,26 @@ static int io_run(md_ctx* c, double* const (&host)[5], bool put, Launch launch) 
     for (int k = 0; k < 5; ++k) per += host[k] ? sizeof(double) * width[k] : 0;
     const int64_t n = c->n_atoms;
     c->d.par = c->par;
-    const bool pinned = per > 0 && (size_t)n * per <= kIoPinned;
+    bool pinned = per > 0 && (size_t)n * per <= kIoPinned;
     int rc;
     if ((rc = need_arrays(c, false))) return rc;
-    if (pinned) {
-        if ((rc = pinned_staging(c))) return rc;
-    } else if (per > 0) {
+    if (!pinned && per > 0) {
         const size_t need = std::min((size_t)n * per, kIoBytes);
         if (need > c->io_cap) {
             if (c->io_dev) HIPCHK(c, hipFree(c->io_dev));
             c->io_dev = nullptr;
             c->io_cap = 0;
-            if (hipMalloc(&c->io_dev, need) != hipSuccess) {
+            if (hipMalloc(&c->io_dev, need) == hipSuccess) {
+                c->io_cap = need;
+            } else {
+                (void)hipGetLastError();
                 c->io_dev = nullptr;
-                return fail(c, MD_ERR_NOMEM, "hipMalloc(" + std::to_string(need) + "): transfer staging");
+                pinned = true;
             }
-            c->io_cap = need;
         }
     }
-    const int64_t chunk = pinned || per == 0 ? n : (int64_t)(c->io_cap / per);
+    if (pinned && (rc = pinned_staging(c))) return rc;
+    const int64_t chunk = per == 0 ? n : (int64_t)((pinned ? c->io_pin_cap : c->io_cap) / per);
     int64_t a0 = 0;
     do {
         StateIO io{};
@@ -1524,10 +1528,9 @@ static int io_run(md_ctx* c, double* const (&host)[5], bool put, Launch launch) 
         };
         if (put && (rc = move(true))) return rc;
         HIPCHK(c, launch(io));
-        if (!put) {
-            if (pinned) HIPCHK(c, hipStreamSynchronize(c->st));
-            if ((rc = move(false))) return rc;
-        }
+        // pinned: the results are there, or the next piece may take the place of this one
+        if (pinned && (!put || io.a1 < n)) HIPCHK(c, hipStreamSynchronize(c->st));
+        if (!put && (rc = move(false))) return rc;
         a0 = io.a1;
     } while (a0 < n);
     if (!put && !pinned) HIPCHK(c, hipStreamSynchronize(c->st));

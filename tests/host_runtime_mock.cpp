@@ -242,10 +242,45 @@ static void layout() {
     CHECK(g_live == 0);
 }
 
+// States move as well on a device without room for staging: everything in and
+// out again, with the last piece not a whole one.
+static void staging() {
+    const int64_t n = 60001;
+    const size_t budget = g_budget;
+    const double mass = 66.335, box[3] = {30.0, 30.0, 30.0};
+    std::vector<double> x(3 * n), v(3 * n), f(3 * n), pot(n), vir(n);
+    for (int64_t i = 0; i < n; ++i) {
+        for (int k = 0; k < 3; ++k) {
+            x[3 * i + k] = 1e-4 * (double)i + k;
+            v[3 * i + k] = -1e-3 * (double)(3 * i + k);
+            f[3 * i + k] = (double)(float)(0.25 * (double)i + k);
+        }
+        pot[i] = 3.0 * (double)i;
+        vir[i] = -1.0 * (double)i;
+    }
+    for (int room = 0; room < 2; ++room) {
+        md_ctx* e = nullptr;
+        CHECK(md_create(&e, 1, &n, &mass, box) == MD_OK);
+        if (!room) g_budget = g_live;
+        const int failed = g_failed_allocs;
+        CHECK(md_upload_state(e, x.data(), v.data(), box) == MD_OK);
+        CHECK(md_upload_forces(e, f.data(), pot.data(), vir.data()) == MD_OK);
+        std::vector<double> x2(3 * n), v2(3 * n), f2(3 * n), p2(n), w2(n);
+        CHECK(md_download_state(e, x2.data(), v2.data(), f2.data(), p2.data(), w2.data(), nullptr) == MD_OK);
+        CHECK(x2 == x && v2 == v && f2 == f && p2 == pot && w2 == vir);
+        CHECK((g_failed_allocs > failed) == !room);
+        CHECK(md_update_force(e) == MD_OK);  // a refused staging is no error of a later launch
+        g_budget = budget;
+        md_destroy(e);
+    }
+    CHECK(g_live == 0);
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "lists") lists();
     else if (what == "layout") layout();
+    else if (what == "staging") staging();
     else return 2;
     printf("%s passed\n", what.c_str());
     return 0;

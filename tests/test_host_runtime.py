@@ -30,7 +30,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["lists", "layout"])
+@pytest.mark.parametrize("case", ["lists", "layout", "staging"])
 def test_out_of_device_memory(program, case):
     r = subprocess.run([program, case], capture_output=True, text=True, timeout=120,
                        env=dict(os.environ, ASAN_OPTIONS="detect_leaks=1:abort_on_error=1"))
