@@ -611,11 +611,16 @@ static int alloc_base(md_ctx* c) {
 static RepCtrl* ctrl_cur(md_ctx* c) { return c->d.ctrl + (size_t)c->par * c->R; }
 
 // States up to kIoPinned bytes pass through pinned host memory that the kernels
-// read and write themselves: one launch and no copy operation (a step and a
-// download of 1,000 atoms: 57 -> 44 us with the above).  Larger ones are copied between the
-// caller's arrays and device staging, at most kIoBytes at a time, or, where the
-// device has no room for that, go through the pinned memory in pieces.
-constexpr size_t kIoPinned = (size_t)256 << 10, kIoBytes = (size_t)128 << 20;
+// read and write themselves: one launch and no copy operation.  Larger ones are
+// copied between the caller's arrays and device staging, at most kIoBytes at a
+// time, or, where the device has no room for that, go through the pinned memory
+// in pieces.  A download of everything, pinned and staged: 3,375 atoms (297 KB)
+// 37 and 78-190 us, 8,000 55 and 97 us, 13,824 83 and 124 us, 19,683 (1.7 MB)
+// 105 and 150 us; positions and velocities of 27,000 atoms (1.3 MB) 81 and 100 us.
+// A staged copy per array costs most where arrays are small, and 2 MB is as far
+// as pinned memory was tried: its price is the block itself (creating a context
+// of 19,683 atoms takes the 0.82 ms it took with 256 KB).
+constexpr size_t kIoPinned = (size_t)2 << 20, kIoBytes = (size_t)128 << 20;
 
 // Systems up to this many slots leave the state of a call's last step in host
 // memory as well, so that a download right after it needs no kernel, no copy and

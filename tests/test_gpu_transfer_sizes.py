@@ -1,0 +1,48 @@
+"""Uploads and downloads on both sides of the size where they stop passing
+through pinned memory (2 MB: 23,831 atoms of everything, 43,690 of positions and
+velocities): the same bits come back, and a download costs no jump where it used
+to change its way (256 KB: 2,978 atoms)."""
+import time
+
+import numpy as np
+import pytest
+
+import moldyn_amd as M
+from tests.common import AR_MASS
+
+pytestmark = pytest.mark.gpu
+
+
+def engine(n, mode="fp64_list"):
+    rng = np.random.default_rng(n)
+    box = [10.0 * n ** (1 / 3)] * 3
+    x, v = rng.uniform(0.0, box[0], (n, 3)), rng.normal(size=(n, 3))
+    e = M.Engine([n], [AR_MASS], box, force_mode=mode)
+    e.upload(x, v, box)
+    return e, x, v, rng
+
+
+@pytest.mark.parametrize("n", [2978, 2979, 23831, 23832, 43690, 43691])
+def test_round_trip(n):
+    e, x, v, rng = engine(n)
+    f, pot, vir = rng.normal(size=(n, 3)), rng.normal(size=n), rng.normal(size=n)
+    e.upload_forces(f, pot, vir)
+    d = e.download()
+    for name, want in (("x", x), ("v", v), ("force", f), ("pot", pot), ("virial", vir)):
+        assert np.array_equal(d[name], want), name
+    d = e.download(("x", "v"))
+    assert np.array_equal(d["x"], x) and np.array_equal(d["v"], v)
+    e.close()
+
+
+def test_no_jump_in_time():
+    def best(n):
+        e = engine(n)[0]
+        t = []
+        for _ in range(60):
+            t0 = time.perf_counter()
+            e.download()
+            t.append(time.perf_counter() - t0)
+        e.close()
+        return min(t[10:])
+    assert best(3375) < 1.7 * best(2744)
