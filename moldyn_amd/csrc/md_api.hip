@@ -866,8 +866,8 @@ static double expected_neighbours(const md_ctx* c, const std::vector<RepCtrl>& C
 // (`stepping`) takes it for clusters up to 2^18 cells only.
 // All-pairs path: k_ap_force keeps the pairs in range of a particle in a list
 // of kApCap = 96 entries and puts them in order afterwards; above half of that
-// on average too many particles overflow it and are summed one thread each, and
-// the ordering costs more than it saves.
+// on average the ordering, and a second pass over the candidates of particles
+// with more, cost more than they save.
 static int choose_instances(md_ctx* c, std::vector<RepCtrl>& C, bool stepping) {
     const int was = c->d.dense;
     if (c->list_mode)
