@@ -584,10 +584,6 @@ static int alloc_base(md_ctx* c) {
     if ((rc = dalloc(c, c->base_allocs, &p, sizeof(double) * NS * c->groups.size()))) return rc;
     d.sums = (double*)p;
     HIPCHK(c, hipMemsetAsync(p, 0, sizeof(double) * NS * c->groups.size(), c->st));
-    if (c->list_mode) {
-        if ((rc = dalloc(c, c->base_allocs, &p, sizeof(float4) * (size_t)std::max<int64_t>(N, 1)))) return rc;
-        d.cpos = (float4*)p;
-    }
     d.n_types = c->T;
     d.n_cu = c->n_cu;
     d.n_blocks = c->n_blocks;
@@ -868,8 +864,7 @@ static double expected_neighbours(const md_ctx* c, const std::vector<RepCtrl>& C
 // of kApCap = 96 entries and puts them in order afterwards; above half of that
 // on average the ordering, and a second pass over the candidates of particles
 // with more, cost more than they save.
-static int choose_instances(md_ctx* c, std::vector<RepCtrl>& C, bool stepping) {
-    const int was = c->d.dense;
+static void choose_instances(md_ctx* c, const std::vector<RepCtrl>& C, bool stepping) {
     if (c->list_mode)
         c->d.dense = expected_neighbours(c, C, c->rlist) >= (double)kLaneWalk ||
                              (c->longest_list > kClumpedList && (!stepping || c->total_cells <= (int64_t)1 << 18))
@@ -877,14 +872,6 @@ static int choose_instances(md_ctx* c, std::vector<RepCtrl>& C, bool stepping) {
                          : 0;
     else
         c->d.dense = expected_neighbours(c, C, c->rc_max) > 48.0 ? 1 : 0;
-    // grids filled while sparse hold no FP32 positions for the dense builder
-    if (!c->list_mode || was || !c->d.dense) return MD_OK;
-    bool fresh = false;
-    for (RepCtrl& X : C) {
-        fresh = fresh || (X.flags & F_GRID_FRESH);
-        X.flags &= ~F_GRID_FRESH;
-    }
-    return fresh ? write_ctrl(c, C) : MD_OK;
 }
 
 // One step launch: list paths k_step + k_fin (which also builds lists),
@@ -1052,7 +1039,7 @@ static int list_force_eval(md_ctx* c) {
     for (int attempt = 0; attempt < 8; ++attempt) {
         std::vector<RepCtrl> C;
         if ((rc = read_ctrl(c, C))) return rc;
-        if ((rc = choose_instances(c, C, false))) return rc;
+        choose_instances(c, C, false);
         for (int r = 0; r < c->R; ++r) {
             RepCtrl& X = C[r];
             X.ins_epoch = X.fill_epoch + 1u;
@@ -1167,7 +1154,7 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
         // snapshot and the first controls in one kernel instead of several copies
         const bool one = c->R == 1;
         bool snap_in_prime = false;
-        if ((rc = choose_instances(c, C, true))) return rc;
+        choose_instances(c, C, true);
         if (c->list_mode) {
             if (one && !records_in_snapshot(c)) {
                 if ((rc = snapshot_alloc(c))) return rc;
@@ -1802,7 +1789,7 @@ int md_update_force(md_ctx* c) {
     if ((rc = write_params(c, P))) return rc;
     std::vector<RepCtrl> C;
     if ((rc = read_ctrl(c, C))) return rc;
-    if ((rc = choose_instances(c, C, false))) return rc;
+    choose_instances(c, C, false);
     c->d.par = c->par;
     if (c->d.dense) {
         if (c->n_blocks > 0) HIPCHK(c, launch_allpairs(c->d, c->bs, true, c->st));

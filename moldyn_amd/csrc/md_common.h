@@ -507,8 +507,6 @@ __device__ __forceinline__ int cell_coord(double x, double b, int m) {
 __device__ __forceinline__ void grid_insert(const DevState& d, const RepCtrl& C,
                                             const RepInfo& R, int64_t slot, double x, double y,
                                             double z) {
-    // the wave-per-cell builder's copy of the position
-    if (d.dense) d.cpos[slot] = make_float4((float)x, (float)y, (float)z, 0.0f);
     const uint32_t ep = C.ins_epoch;
     const int buf = ep & 1;
     const int* gd = C.gdim[buf];

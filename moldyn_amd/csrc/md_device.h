@@ -219,7 +219,6 @@ struct DevState {
     double4* dpos;           // dense list path: every slot's drifted position and type (x, y, z, type)
     const uint8_t* slot_type;  // type of every slot (padding slots: the group's type)
     int32_t compact;         // the list path steps on crec (k_fin builds from crec)
-    float4* cpos;            // list paths: FP32 position of every slot at the last grid fill (dense systems)
     int32_t dense;           // long lists expected: lanes walk their own lists, a wave per cell builds them
                              // (all-pairs path: many pairs in range, a thread per particle sums as it goes)
     double* pot;

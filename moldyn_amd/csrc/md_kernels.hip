@@ -638,11 +638,10 @@ __device__ __forceinline__ void sort_candidates(const DevState& d, const int32_t
 // a wave per cell: cells wave0, wave0 + n_waves, ...  The particles of the
 // cell's stencil (up to 27 cells, 240 to 500 particles in a liquid) are the
 // candidates of every particle of the cell.  Their slot ids are sorted once;
-// 256 at a time they then sit in registers with their FP32 positions (left by
-// the fill in d.cpos), four per lane in ascending order, and each particle of
-// the cell takes one distance test per register, a ballot for each entry's
-// place, and one store: the entries come out in ascending order without a sort
-// per particle.
+// 256 at a time they then sit in registers with their positions in FP32, four
+// per lane in ascending order, and each particle of the cell takes one distance
+// test per register, a ballot for each entry's place, and one store: the entries
+// come out in ascending order without a sort per particle.
 // FP32 test: an FP32 component differs from the FP64 one by at most
 // (1.01 + 1.01 + 2.02 + 1 + 1.01) 2^-24 L for positions within 1.01 L (roundings
 // of the two positions, the difference, the box and the image); 20 2^-24 L
@@ -653,7 +652,9 @@ __device__ __forceinline__ void sort_candidates(const DevState& d, const int32_t
 // waves per SIMD to cover it, and the sort's lane exchanges.  Bricks of cells
 // staged in LDS by 512 threads, one lane scanning per particle and a sort per
 // list (the dense builder before, one block per CU) took 920 us for 262,144
-// liquid particles, this 151 us; 685 and 35 us for 4,096 (343 cells on 256 CUs).
+// liquid particles, this 149 us; 685 and 35 us for 4,096 (343 cells on 256 CUs).
+// An FP32 copy of the positions, 16 bytes a slot written at every grid fill, in
+// place of the records: 145 us.
 // A sparse gas (a cell per particle or more) would leave a wave one particle
 // at a time: it keeps the bricks (1,000,000 particles: 146 us).
 template <bool MULTI>
@@ -731,7 +732,11 @@ __device__ __forceinline__ void cell_build(const DevState& d, const RepCtrl& C, 
                     }
                 }
             } else {
-                const float4 hp = d.cpos[hi];
+                auto pos_f = [&](int64_t j) {
+                    const double* o = recs[j];
+                    return make_float4((float)o[0], (float)o[1], (float)o[2], 0.0f);
+                };
+                const float4 hp = pos_f(hi);
                 for (int w0 = 0; w0 < total; w0 += 256) {
                     float x[4], y[4], z[4];
                     int32_t id[4];
@@ -739,7 +744,7 @@ __device__ __forceinline__ void cell_build(const DevState& d, const RepCtrl& C, 
                     for (int r = 0; r < 4; ++r) {
                         const int e = w0 + 64 * r + wl;
                         id[r] = e < total ? (int32_t)sid[e] : 0;
-                        const float4 p = d.cpos[id[r]];
+                        const float4 p = pos_f(id[r]);
                         x[r] = e < total ? p.x : __builtin_nanf("");
                         y[r] = p.y;
                         z[r] = p.z;

@@ -276,11 +276,29 @@ static void staging() {
     CHECK(g_live == 0);
 }
 
+// Device memory of a list context per slot: records, step records, drifted
+// positions, type, potential and virial, a list of 8 entries and its length, and
+// two cells of 8 slots and a header in both grid buffers; small arrays aside.
+static void footprint() {
+    const int64_t n = 1 << 20;
+    md_ctx* c = nullptr;
+    const double mass = 66.335, box[3] = {400.0, 400.0, 400.0};
+    CHECK(md_create(&c, 1, &n, &mass, box) == MD_OK);
+    md_stats st;
+    CHECK(md_get_stats(c, &st) == MD_OK);
+    const size_t per = 2 * sizeof(Rec<float>) + 2 * sizeof(CRec) + sizeof(double4) + 1 + 2 * sizeof(double) +
+                       sizeof(int32_t) * (st.list_capacity + 1) + 2 * 2 * (8 + sizeof(int32_t) * st.cell_capacity);
+    printf("%.2f bytes per slot, %zu expected\n", (double)g_live / n, per);
+    CHECK(g_live <= per * n + ((size_t)4 << 20));
+    md_destroy(c);
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "lists") lists();
     else if (what == "layout") layout();
     else if (what == "staging") staging();
+    else if (what == "footprint") footprint();
     else return 2;
     printf("%s passed\n", what.c_str());
     return 0;
