@@ -22,6 +22,7 @@
 //
 // All code is built with -ffp-contract=off: the FP64 paths must not form FMAs
 // the reference (Rust) never forms.  The FP32 pair kernel uses explicit fmaf.
+#include <limits.h>
 #include <math.h>
 
 #include <type_traits>
@@ -200,10 +201,11 @@ __device__ __forceinline__ int brick_count(const RepCtrl& C) {
     return n;
 }
 
-// Bricks bi0, bi0 + stride, ... of a replica (all threads of the block).
+// Bricks bi0, bi0 + stride, ... below `end` of a replica (all threads of the block).
 template <typename RT, int BS, bool MULTI>
 __device__ __forceinline__ void brick_build(const DevState& d, const RepCtrl& C, const RepParams& P,
-                            const RepInfo& R, const RT* __restrict__ recs, int bi0, int stride) {
+                            const RepInfo& R, const RT* __restrict__ recs, int bi0, int stride,
+                            int end = INT_MAX) {
     const uint32_t ep = C.fill_epoch;
     const int buf = ep & 1;
     const int* gd = C.gdim[buf];
@@ -239,7 +241,7 @@ __device__ __forceinline__ void brick_build(const DevState& d, const RepCtrl& C,
         const bool w = (whole >> k) & 1;
         nbk[k] = w ? 1 : (gd[k] + be[k] - 1) / be[k];
     }
-    const int nbricks = nbk[0] * nbk[1] * nbk[2];
+    const int nbricks = min(nbk[0] * nbk[1] * nbk[2], end);
     BrickLds& L = brick_lds();
     int* const s_off = L.off;
     int* const s_cen = L.cen;
@@ -2173,7 +2175,7 @@ __device__ __forceinline__ void prof_fold(const DevState& d, int64_t launch, boo
 
 // Build block b's share of the lists of the replicas flagged F_BUILD in this
 // launch, from the step records (compact) or the full ones; returns the launch index when it built any, else -1.
-template <typename FT, bool MULTI, bool REPS, bool DENSE>
+template <typename FT, bool MULTI, bool REPS, bool DENSE, bool RUNS>
 __device__ __forceinline__ int64_t build_lists(const DevState& d, int b, bool compact) {
     if constexpr (DENSE) {
         // the cells of every building replica, numbered replica after replica,
@@ -2258,7 +2260,11 @@ __device__ __forceinline__ int64_t build_lists(const DevState& d, int b, bool co
         // rebuild at different launches, so a share fixed per replica would
         // leave most blocks idle while a large replica builds).  A block's
         // bricks within one replica are one strided run: one builder call
-        // per (replica, block).
+        // per (replica, block).  RUNS (all replicas build): each block takes a
+        // run of consecutive bricks, whose halos it shares in cache: 256
+        // replicas of 1,000 particles of a gas 79 us, dealt 118 (a share
+        // of the blocks fixed per replica 84; 500 to 32,768 particles each,
+        // update_force 805, 866 and 1,134 us).
         __shared__ int s_rb[kFinBS + 1];
         __shared__ int s_work[kFinBS];
         __shared__ int s_nwork;
@@ -2274,12 +2280,17 @@ __device__ __forceinline__ int64_t build_lists(const DevState& d, int b, bool co
             lds_barrier();
             block_exclusive_scan<kFinBS>(s_rb, n);
             const int tot = __builtin_amdgcn_readfirstlane(s_rb[n]);  // uniform: scalar registers
+            // RUNS: the block's bricks of this chunk
+            const int t0 = (int)((int64_t)tot * b / nb), t1 = (int)((int64_t)tot * (b + 1) / nb);
             // replicas holding bricks of this block (in any order: each
             // brick's lists depend on the brick alone)
             if ((int)threadIdx.x < n) {
                 const int64_t lo = base + s_rb[threadIdx.x], hi = base + s_rb[threadIdx.x + 1];
                 const int64_t g0 = lo + ((b - lo % nb) % nb + nb) % nb;
-                if (g0 < hi) s_work[atomicAdd(&s_nwork, 1)] = threadIdx.x;
+                const bool some = RUNS ? s_rb[threadIdx.x] < t1 && s_rb[threadIdx.x + 1] > t0 &&
+                                             s_rb[threadIdx.x] < s_rb[threadIdx.x + 1]
+                                       : g0 < hi;
+                if (some) s_work[atomicAdd(&s_nwork, 1)] = threadIdx.x;
             }
             lds_barrier();
             const int nwork = __builtin_amdgcn_readfirstlane(s_nwork);
@@ -2287,14 +2298,16 @@ __device__ __forceinline__ int64_t build_lists(const DevState& d, int b, bool co
                 const int idx = __builtin_amdgcn_readfirstlane(s_work[w]);
                 const int64_t lo = base + __builtin_amdgcn_readfirstlane(s_rb[idx]);
                 const int r = r0 + idx;
-                const int bi0 = (int)(((b - lo % nb) % nb + nb) % nb);
+                const int first = (int)(lo - base);
+                const int bi0 = RUNS ? (t0 > first ? t0 - first : 0) : (int)(((b - lo % nb) % nb + nb) % nb);
+                const int stride = RUNS ? 1 : nb, end = RUNS ? t1 - first : INT_MAX;
                 const RepCtrl& C = ctrl_in(d, r);
                 const RepInfo R = d.reps[r];
                 if (compact)
-                    brick_build<CRec, kFinBS, MULTI>(d, C, d.params[r], R, d.crec[C.build_src], bi0, nb);
+                    brick_build<CRec, kFinBS, MULTI>(d, C, d.params[r], R, d.crec[C.build_src], bi0, stride, end);
                 else
                     brick_build<Rec<FT>, kFinBS, MULTI>(d, C, d.params[r], R,
-                                                               (const Rec<FT>*)d.rec[C.build_src], bi0, nb);
+                                                               (const Rec<FT>*)d.rec[C.build_src], bi0, stride, end);
                 launch = C.launches;
             }
             base += tot;
@@ -2316,7 +2329,7 @@ __global__ __launch_bounds__(kFinBS, DENSE ? 4 : 2) void k_fin(DevState d, int m
     int64_t launch = -1;
     if (b < d.n_reps) launch = finalize_replica(d, b, mode);
     if (BUILD) {
-        const int64_t l = build_lists<FT, MULTI, REPS, DENSE>(d, b, d.compact != 0);
+        const int64_t l = build_lists<FT, MULTI, REPS, DENSE, false>(d, b, d.compact != 0);
         launch = l >= 0 ? l : launch;
     }
     if (launch >= 0) {
@@ -2329,7 +2342,7 @@ __global__ __launch_bounds__(kFinBS, DENSE ? 4 : 2) void k_fin(DevState d, int m
 // whose flags ask for it, from the full records.
 template <typename FT, bool MULTI, bool REPS, bool DENSE>
 __global__ __launch_bounds__(kFinBS, DENSE ? 4 : 2) void k_build(DevState d) {
-    build_lists<FT, MULTI, REPS, DENSE>(d, blockIdx.x, false);
+    build_lists<FT, MULTI, REPS, DENSE, true>(d, blockIdx.x, false);
 }
 
 // ---------------------------------------------------------------- small helpers
