@@ -122,8 +122,7 @@ struct md_ctx {
     RepParams* h_params = nullptr;
     void* h_rec = nullptr;            // DevState::h_rec and h_pv as the host sees them
     double* h_pv = nullptr;
-    uint32_t* h_done = nullptr;       // number of the last kernel that signalled its end
-    uint32_t done_seq = 0;            // number of the last one asked to
+    uint32_t* h_done = nullptr;       // RepParams::done once that launch has ended, 0 before
     hipEvent_t params_ev = nullptr;  // the last parameter upload (h_params is reused after it)
     bool params_pending = false;
     // staging of uploads and downloads: device memory (at most kIoBytes), and
@@ -289,7 +288,6 @@ static void free_all(md_ctx* c) {
     c->h_stats = nullptr;
     c->h_params = nullptr;
     c->h_done = nullptr;
-    c->done_seq = 0;
     c->h_rec = nullptr;
     c->h_pv = nullptr;
     c->io_pin = c->io_pin_dev = nullptr;
@@ -667,14 +665,14 @@ static int pinned_staging(md_ctx* c) {
     return MD_OK;
 }
 
-// Waits until a kernel has written done_seq to h_done (true), or until the
+// Waits until a kernel has written `number` to h_done (true), or until the
 // stream is done without it (false).  A kernel's own word arrives some
 // microseconds before the stream reports its end, which is what a step of a
 // small system and its download mostly consist of; after a while the wait
 // becomes the runtime's.
-static int wait_done(md_ctx* c, bool* done) {
+static int wait_done(md_ctx* c, uint32_t number, bool* done) {
     const auto t0 = std::chrono::steady_clock::now();
-    auto seen = [&] { return __atomic_load_n(c->h_done, __ATOMIC_ACQUIRE) == c->done_seq; };
+    auto seen = [&] { return number != 0 && __atomic_load_n(c->h_done, __ATOMIC_ACQUIRE) == number; };
     while (!(*done = seen())) {
         if (std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(200)) continue;
         HIPCHK(c, hipStreamSynchronize(c->st));
@@ -1171,9 +1169,10 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
         }
         if (one) {
             if ((rc = pinned_staging(c))) return rc;
-            P[0].done_seq = ++c->done_seq;
-            if (c->done_seq == 0) P[0].done_seq = c->done_seq = 1;
-            P[0].done_launch = C[0].launches + cn;
+            // launch numbers start again with a new state; the last chunk's
+            // signal is there (it was waited for), so none is under way
+            __atomic_store_n(c->h_done, 0u, __ATOMIC_RELEASE);
+            P[0].done = (uint32_t)(C[0].launches + cn);
             // the snapshot's layout without records: the group sums, then the
             // surrogate's counters (snapshot())
             char* sb = (char*)c->snap;
@@ -1206,7 +1205,7 @@ static int run_steps(md_ctx* c, double dt, md_thermostat* th, md_barostat* ba, i
         RepStats s;
         for (int iter = 0;; ++iter) {
             bool done = false;
-            if (one && iter == 0 && (rc = wait_done(c, &done))) return rc;
+            if (one && iter == 0 && (rc = wait_done(c, P[0].done, &done))) return rc;
             if (done) {
                 C.assign(c->h_ctrl, c->h_ctrl + 1);
                 s = *c->h_stats;

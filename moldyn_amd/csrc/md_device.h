@@ -134,13 +134,15 @@ struct RepParams {
     // records to, the one not holding the chunk's starting state (which a
     // replay after an overflow restarts from); -1 on the other paths
     int32_t full_dst;
-    // one replica: the finalize of launch done_launch writes done_seq to
-    // DevState::h_done (0: none does)
-    uint32_t done_seq;
-    int64_t done_launch;
+    // one replica: the finalize of the launch with this number (its low 32 bits)
+    // writes it to DevState::h_done (0: none does)
+    uint32_t done;
     double cm[kMaxTypes];     // dt / (2 m_t), the half-kick factor (integrator.rs:29)
     double inv_m2[kMaxTypes]; // 1 / m_t^2 (drift-bound bookkeeping only)
 };
+// Two 128-byte lines: with 8 bytes more the finalize of 1,000,000 particles took
+// 7.3 us instead of 7.0 (median), of 64 replicas of 4,096 16.4 instead of 16.3.
+static_assert(sizeof(RepParams) == 256, "every finalize waits for it");
 
 struct RepCtrl {
     double box[3];             // box at the start of the launch
@@ -270,8 +272,7 @@ struct DevState {
     int32_t par;             // control buffer this launch reads
     int32_t tpb;             // tiles per block of the per-slot kernels
     // host memory (device addresses) a one-replica run leaves its control block
-    // and statistics in at launch RepParams::done_launch, and the number that
-    // says so
+    // and statistics in at launch RepParams::done, and that number to say so
     RepCtrl* h_ctrl;
     RepStats* h_stats;
     uint32_t* h_done;

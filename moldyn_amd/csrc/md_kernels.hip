@@ -2002,9 +2002,10 @@ __device__ __forceinline__ void copy_words(void* dst, const void* src, int bytes
 // Finalize of replica r by one block: group sums (from the block partials of
 // this launch, or the stored ones when the launch did not step), then one
 // thread advances the controls on register copies of the LDS-staged inputs,
-// and the block writes the control block of the next launch.  Returns the
-// launch index when the replica did work in this launch, else -1.
-__device__ __forceinline__ int64_t finalize_replica(const DevState& d, int r, int mode) {
+// and the block writes the control block of the next launch.  Returns whether
+// the replica did work in this launch.
+template <bool REPS>
+__device__ __forceinline__ bool finalize_replica(const DevState& d, int r, int mode) {
     constexpr int BS = kFinBS;
     const int T = d.n_types;
     const int64_t g0 = (int64_t)r * T;  // groups are replica-major
@@ -2031,13 +2032,12 @@ __device__ __forceinline__ int64_t finalize_replica(const DevState& d, int r, in
     }
     __syncthreads();
     const uint32_t f0 = s_ctrl.flags;
-    const int64_t launch = s_ctrl.launches;
     if (mode == M_STEP && (f0 & F_EXIT)) {
         // target reached: carry the block over to the buffer the next launch reads
         if (threadIdx.x == 0) s_ctrl.launches++;
         __syncthreads();
         copy_words<BS>(ctrl_out(d, r), &s_ctrl, (int)sizeof(RepCtrl));
-        return -1;
+        return false;
     }
     // the new group sums are stored at the end: a store before a barrier would
     // make every thread wait for its completion
@@ -2093,7 +2093,7 @@ __device__ __forceinline__ int64_t finalize_replica(const DevState& d, int r, in
     }
     if (mode == M_REDUCE) {
         for (int i = threadIdx.x; i < T * NS; i += BS) d.sums[g0 * NS + i] = s_sums[i];
-        return -1;
+        return false;
     }
     if (threadIdx.x == 0) {
         RepCtrl C = s_ctrl;
@@ -2105,16 +2105,16 @@ __device__ __forceinline__ int64_t finalize_replica(const DevState& d, int r, in
     copy_words<BS>(ctrl_out(d, r), &s_ctrl, (int)sizeof(RepCtrl));
     if (reduced)
         for (int i = threadIdx.x; i < T * NS; i += BS) d.sums[g0 * NS + i] = s_sums[i];
-    if (mode == M_STEP && s_par.done_seq != 0 && s_ctrl.launches == s_par.done_launch) {
+    if (!REPS && mode == M_STEP && s_par.done != 0 && (uint32_t)s_ctrl.launches == s_par.done) {
         // the last launch of a one-replica chunk: the host takes the control
         // block and the statistics from its own memory, without another kernel
         // or a wait for the stream (statistics of a build in this very launch
         // follow at the end of the launches that it makes necessary)
         copy_words<BS>(d.h_ctrl, &s_ctrl, (int)sizeof(RepCtrl));
         copy_words<BS>(d.h_stats, d.stats, (int)sizeof(RepStats));
-        signal_host(d.h_done, s_par.done_seq);
+        signal_host(d.h_done, s_par.done);
     }
-    return mode == M_STEP ? launch : -1;
+    return mode == M_STEP;
 }
 
 // Fold the per-block records of this launch's per-slot kernels into the
@@ -2174,16 +2174,17 @@ __device__ __forceinline__ void prof_fold(const DevState& d, int64_t launch, boo
 }
 
 // Build block b's share of the lists of the replicas flagged F_BUILD in this
-// launch, from the step records (compact) or the full ones; returns the launch index when it built any, else -1.
+// launch, from the step records (compact) or the full ones; returns whether it
+// built any.
 template <typename FT, bool MULTI, bool REPS, bool DENSE, bool RUNS>
-__device__ __forceinline__ int64_t build_lists(const DevState& d, int b, bool compact) {
+__device__ __forceinline__ bool build_lists(const DevState& d, int b, bool compact) {
     if constexpr (DENSE) {
         // the cells of every building replica, numbered replica after replica,
         // are shared out among the grid's waves; few cells go to as many blocks
         // as there are, many keep neighbours in a block
         __shared__ uint32_t s_sid[kFinBS / 64][kCellCand];
         const int w = threadIdx.x >> 6, nw = (int)gridDim.x * (kFinBS / 64);
-        int64_t launch = -1;
+        bool built = false;
         auto build = [&](int r, int w0) {
             const RepCtrl& C = ctrl_in(d, r);
             const PosView recs = compact ? PosView{(const char*)d.crec[C.build_src], (int)sizeof(CRec)}
@@ -2198,7 +2199,7 @@ __device__ __forceinline__ int64_t build_lists(const DevState& d, int b, bool co
         if constexpr (!REPS) {
             const RepCtrl& C = ctrl_in(d, 0);
             if ((C.flags & (F_BUILD | F_EXIT)) == F_BUILD) {
-                launch = C.launches;
+                built = true;
                 build(0, cells_of(C) < (uint32_t)nw ? w * (int)gridDim.x + b : b * (kFinBS / 64) + w);
             }
         } else {
@@ -2222,7 +2223,7 @@ __device__ __forceinline__ int64_t build_lists(const DevState& d, int b, bool co
                     const unsigned long long any = __ballot(mine);
                     if (!any) continue;
                     const int rq = r0 + 64 * q;
-                    if (launch < 0) launch = ctrl_in(d, rq + __builtin_ctzll(any)).launches;
+                    built = true;
                     const uint32_t cells = mine ? cells_of(ctrl_in(d, rq + wl)) : 0u;
                     const uint32_t incl = (uint32_t)wave_scan_incl((int)cells);
                     const uint32_t at = (off + incl - cells) % (uint32_t)nw;
@@ -2235,12 +2236,12 @@ __device__ __forceinline__ int64_t build_lists(const DevState& d, int b, bool co
                 }
             }
         }
-        if (launch >= 0 && b == 0 && threadIdx.x == 0) atomicMax(&d.stats->max_len, 1);
-        return launch;
+        if (built && b == 0 && threadIdx.x == 0) atomicMax(&d.stats->max_len, 1);
+        return built;
     } else {
-    int64_t launch = -1;
+    bool built = false;
     if constexpr (!REPS) {
-        if (b >= d.n_bld) return -1;
+        if (b >= d.n_bld) return false;
         // one system: the build blocks share its bricks
         const RepCtrl& C = ctrl_in(d, 0);
         if ((C.flags & (F_BUILD | F_EXIT)) == F_BUILD) {
@@ -2250,10 +2251,10 @@ __device__ __forceinline__ int64_t build_lists(const DevState& d, int b, bool co
             else
                 brick_build<Rec<FT>, kFinBS, MULTI>(d, C, d.params[0], R, (const Rec<FT>*)d.rec[C.build_src], b,
                                                     d.n_bld);
-            launch = C.launches;
+            built = true;
         }
     } else {
-        if (b >= d.n_bld) return -1;
+        if (b >= d.n_bld) return false;
         // several replicas: the bricks of every replica building in this
         // launch, numbered replica after replica, are shared out among all
         // build blocks: block b takes bricks b, b + n_bld, ... (replicas
@@ -2308,13 +2309,13 @@ __device__ __forceinline__ int64_t build_lists(const DevState& d, int b, bool co
                 else
                     brick_build<Rec<FT>, kFinBS, MULTI>(d, C, d.params[r], R,
                                                                (const Rec<FT>*)d.rec[C.build_src], bi0, stride, end);
-                launch = C.launches;
+                built = true;
             }
             base += tot;
             lds_barrier();  // s_rb and s_work are read before the next chunk rewrites them
         }
     }
-    return launch;
+    return built;
     }
 }
 
@@ -2326,15 +2327,12 @@ __global__ __launch_bounds__(kFinBS, DENSE ? 4 : 2) void k_fin(DevState d, int m
     // k_allpairs) while the first blocks finalize
     if (d.prof && mode == M_STEP && b == (int)gridDim.x - 1)
         prof_fold(d, ctrl_in(d, 0).launches, !BUILD || d.mlp_w != nullptr);
-    int64_t launch = -1;
-    if (b < d.n_reps) launch = finalize_replica(d, b, mode);
-    if (BUILD) {
-        const int64_t l = build_lists<FT, MULTI, REPS, DENSE, false>(d, b, d.compact != 0);
-        launch = l >= 0 ? l : launch;
-    }
-    if (launch >= 0) {
+    bool worked = false;
+    if (b < d.n_reps) worked = finalize_replica<REPS>(d, b, mode);
+    if (BUILD) worked = build_lists<FT, MULTI, REPS, DENSE, false>(d, b, d.compact != 0) || worked;
+    if (worked) {
         __syncthreads();
-        prof_mark(d, launch, P_FIN, t_start);
+        prof_mark(d, ctrl_in(d, 0).launches, P_FIN, t_start);  // replicas count alike
     }
 }
 
@@ -2535,7 +2533,7 @@ __global__ __launch_bounds__(kFinBS) void k_prime(DevState d, RepParams p, doubl
         copy_words<kFinBS>(snap_ctrl, &ctrl_in(d, 0), (int)sizeof(RepCtrl));
     }
     __syncthreads();  // the parameters are read back from memory
-    finalize_replica(d, 0, M_PRIME);
+    finalize_replica<false>(d, 0, M_PRIME);
 }
 
 __global__ __launch_bounds__(256) void k_epilogue(DevState d, int par, RepCtrl* h_ctrl, RepStats* h_stats) {
