@@ -971,7 +971,9 @@ __device__ __forceinline__ Acc<FT> wave_list_forces(const DevState& d, const CRe
 // FP64 in dense systems takes the registers of two waves per SIMD: at four it
 // keeps part of the walk in scratch (262,144 particles of two types 99 us a
 // launch, 91 so; FP32 loses, 47 against 43 us).
-template <typename FT, int BS, bool MULTI, bool DENSE>
+// MIRROR: and into host memory, for DevState::h_rec (a branch on it at run time
+// cost every other system 1.1 us of 48.9 a launch, 256 replicas of 500 to 32,768).
+template <typename FT, int BS, bool MULTI, bool DENSE, bool MIRROR>
 __global__ __launch_bounds__(BS, DENSE && sizeof(FT) == 8 ? 2 : 4) void k_step(DevState d) {
     const int b = xcd_block(blockIdx.x, gridDim.x);
     const int gi = d.blk_group[b];
@@ -1173,7 +1175,7 @@ __global__ __launch_bounds__(BS, DENSE && sizeof(FT) == 8 ? 2 : 4) void k_step(D
                 o.fz = acc.fz;
                 o.type = (uint32_t)ti;
                 full[s] = o;
-                if (d.h_rec) {
+                if (MIRROR) {
                     ((Rec<FT>*)d.h_rec)[s] = o;
                     d.h_pv[s] = (double)acc.pot;
                     d.h_pv[d.n_slots + s] = (double)acc.vir;
@@ -2458,12 +2460,17 @@ hipError_t launch_dpos(const DevState& d, int bs, hipStream_t st) {
 
 hipError_t launch_step(const DevState& d, bool fp32, int bs, hipStream_t st) {
     const bool multi = d.n_types > 1;
-#define KS(FT, B, M)                                                                        \
-    do {                                                                                    \
-        if (d.dense)                                                                        \
-            hipLaunchKernelGGL((k_step<FT, B, M, true>), dim3(d.n_blocks), dim3(B), 0, st, d);  \
-        else                                                                                \
-            hipLaunchKernelGGL((k_step<FT, B, M, false>), dim3(d.n_blocks), dim3(B), 0, st, d); \
+#define KS1(FT, B, M, DN)                                                                          \
+    do {                                                                                           \
+        if (d.h_rec)                                                                               \
+            hipLaunchKernelGGL((k_step<FT, B, M, DN, true>), dim3(d.n_blocks), dim3(B), 0, st, d);  \
+        else                                                                                       \
+            hipLaunchKernelGGL((k_step<FT, B, M, DN, false>), dim3(d.n_blocks), dim3(B), 0, st, d); \
+    } while (0)
+#define KS(FT, B, M)                  \
+    do {                              \
+        if (d.dense) KS1(FT, B, M, true); \
+        else KS1(FT, B, M, false);    \
     } while (0)
 #define L(B)                           \
     if (fp32) {                        \
@@ -2476,6 +2483,7 @@ hipError_t launch_step(const DevState& d, bool fp32, int bs, hipStream_t st) {
     MD_BS_SWITCH(bs, L)
 #undef L
 #undef KS
+#undef KS1
     return hipGetLastError();
 }
 
