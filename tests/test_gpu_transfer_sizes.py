@@ -35,6 +35,19 @@ def test_round_trip(n):
     e.close()
 
 
+def test_list_statistics_in_pieces():
+    """700 replicas of two or three neighbours: their list lengths take more room
+    than the pinned memory of so few particles."""
+    counts = np.array([2, 3] * 350)
+    x = np.concatenate([1.0 + 0.4 * np.arange(n)[:, None] * [1.0, 0.0, 0.0] for n in counts])
+    e = M.Engine(counts[:, None], [AR_MASS], [[5.0] * 3] * 700, force_mode="fp64_list")
+    e.upload(x, np.zeros_like(x), [[5.0] * 3] * 700)
+    e.update_force()
+    st = e.stats()
+    assert st["mean_list_len"] == (2 * 1 + 3 * 2) / 5 and st["max_list_len"] == 2
+    e.close()
+
+
 def test_no_jump_in_time():
     def best(n):
         e = engine(n)[0]
