@@ -333,20 +333,26 @@ __host__ __device__ __forceinline__ double sums_about_com(double q, const double
 struct PairTerms64 {
     double gx, gy, gz, u, t;
 };
+
+// a / r, correctly rounded as the division is, for y = 1 / r correctly rounded:
+// the first correction leaves a quotient within one unit in its last place, the
+// second the rounded one (P. Markstein, Computation of elementary functions on
+// the IBM RISC System/6000, 1990).  Five operations instead of a division's
+// eleven.  The remainders have to be exact: it holds for finite a of at least
+// 2^-960 and for zeros (-0 gives +0, and so would a difference of coordinates
+// below that, which only a sum of nothing else would show), r in [2^-1000,
+// 2^1000] and quotients from 2^-1022 to below 2^1023 (a y may overflow above).
+__host__ __device__ __forceinline__ double quotient(double a, double r, double y) {
+    double q = a * y;
+    q = fma(fma(-r, q, a), y, q);
+    return fma(fma(-r, q, a), y, q);
+}
+
 __device__ __forceinline__ PairTerms64 pair_exact_terms(double dx, double dy, double dz, double r2,
                                                         const PairParam& p) {
     const double r = sqrt(r2);
     const double y = 1.0 / r;
-    // a / r, correctly rounded as the division is: with y the correctly rounded
-    // reciprocal, the first correction leaves a quotient within one unit in its
-    // last place, the second the rounded one (P. Markstein, Computation of
-    // elementary functions on the IBM RISC System/6000, 1990).  Five operations
-    // instead of a division's eleven.
-    auto over_r = [&](double a) {
-        double q = a * y;
-        q = fma(fma(-r, q, a), y, q);
-        return fma(fma(-r, q, a), y, q);
-    };
+    auto over_r = [&](double a) { return quotient(a, r, y); };
     const double sr = over_r(p.sigma);
     const double s2 = sr * sr;
     const double s4 = s2 * s2;
