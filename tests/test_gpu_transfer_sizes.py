@@ -35,6 +35,29 @@ def test_round_trip(n):
     e.close()
 
 
+@pytest.mark.parametrize("mode", ["fp64_list", "fp32_list"])
+def test_round_trip_in_pieces(mode):
+    """3.3 million atoms of three replicas and two types: more than 128 MB, which
+    move in pieces that end inside waves, groups and replicas."""
+    counts = np.array([[700001, 399990], [1, 1100003], [650000, 450007]])
+    n, rng = int(counts.sum()), np.random.default_rng(2)
+    box = [[400.0] * 3, [410.0] * 3, [420.0] * 3]
+    x, v, f = rng.uniform(0.0, 400.0, (n, 3)), rng.normal(size=(n, 3)), rng.normal(size=(n, 3))
+    if mode == "fp32_list":
+        f = f.astype(np.float32).astype(np.float64)
+    pot, vir = rng.normal(size=n), rng.normal(size=n)
+    e = M.Engine(counts, [AR_MASS, 20.0], box, force_mode=mode)
+    e.upload(x, v, box)
+    e.upload_forces(f, pot, vir)
+    d = e.download()
+    for name, want in (("x", x), ("v", v), ("force", f), ("pot", pot), ("virial", vir), ("box", np.array(box))):
+        assert np.array_equal(d[name], want), name
+    e.upload_forces(None, pot, None)
+    d = e.download(("force", "pot", "virial"))
+    assert not d["force"].any() and np.array_equal(d["pot"], pot) and not d["virial"].any()
+    e.close()
+
+
 def test_list_statistics_in_pieces():
     """700 replicas of two or three neighbours: their list lengths take more room
     than the pinned memory of so few particles."""
