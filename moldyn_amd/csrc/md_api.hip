@@ -132,6 +132,7 @@ struct md_ctx {
     void* io_pin = nullptr;
     void* io_pin_dev = nullptr;
     size_t io_pin_cap = 0;
+    hipEvent_t io_ev[2] = {nullptr, nullptr};  // the kernel on either half of io_pin
     // host copy of the control blocks the next launch reads, valid while no
     // finalize, graph replay, snapshot restore or layout change has run since
     std::vector<RepCtrl> ctrl_cache;
@@ -283,6 +284,10 @@ static void free_all(md_ctx* c) {
     }
     c->params_ev = nullptr;
     c->params_pending = false;
+    for (hipEvent_t& e : c->io_ev) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
     // the pinned block stays for the next layout (md_destroy frees it)
     c->h_ctrl = nullptr;
     c->h_stats = nullptr;
@@ -604,17 +609,22 @@ static int alloc_base(md_ctx* c) {
 // Control blocks of the buffer the next launch reads.
 static RepCtrl* ctrl_cur(md_ctx* c) { return c->d.ctrl + (size_t)c->par * c->R; }
 
-// States up to kIoPinned bytes pass through pinned host memory that the kernels
-// read and write themselves: one launch and no copy operation.  Larger ones are
-// copied between the caller's arrays and device staging, at most kIoBytes at a
-// time, or, where the device has no room for that, go through the pinned memory
-// in pieces.  A download of everything, pinned and staged: 3,375 atoms (297 KB)
-// 37 and 78-190 us, 8,000 55 and 97 us, 13,824 83 and 124 us, 19,683 (1.7 MB)
-// 105 and 150 us; positions and velocities of 27,000 atoms (1.3 MB) 81 and 100 us.
-// A staged copy per array costs most where arrays are small, and 2 MB is as far
-// as pinned memory was tried: its price is the block itself (creating a context
-// of 19,683 atoms takes the 0.82 ms it took with 256 KB).
-constexpr size_t kIoPinned = (size_t)2 << 20, kIoBytes = (size_t)128 << 20;
+// Uploads up to kIoPinned bytes, and downloads up to that for each array asked
+// for, pass through a block of kIoPinned bytes of pinned host memory that the
+// kernels read and write themselves, without a copy operation; a download of more
+// than the block takes its halves in turn, one being filled while the other is
+// copied out.  Larger states are copied between the caller's arrays and device
+// staging, at most kIoBytes at a time, or, where the device has no room for that,
+// go through the pinned block in pieces.  A staged copy costs some 15 us per
+// array, hence the rule for downloads, in pieces and staged: all five arrays of
+// 3,375 atoms (297 KB) 45 and 78 us, of 8,000 76 and 96, of 13,824 119 and 123, of
+// 19,683 162 and 149; positions and velocities of 8,000 (384 KB) 45 and 54, of
+// 10,648 55 and 59, of 13,824 70 and 67, of 19,683 92 and 81.  An upload of
+// positions and velocities of 5,832 atoms (280 KB) takes 45 us both ways, of 10,648
+// 63 and 51.  A larger block would need no pieces (everything of 8,000 atoms 55 us),
+// but the host takes 1.4 us for its first access to each page of it, which a
+// program that makes a context for a few calls does not get back.
+constexpr size_t kIoPinned = (size_t)256 << 10, kIoBytes = (size_t)128 << 20;
 
 // Systems up to this many slots leave the state of a call's last step in host
 // memory as well, so that a download right after it needs no kernel, no copy and
@@ -662,6 +672,7 @@ static int pinned_staging(md_ctx* c) {
     c->h_rec = mirror ? take(rec, &c->d.h_rec) : nullptr;
     c->h_pv = mirror ? (double*)take(pv, (void**)&c->d.h_pv) : nullptr;
     HIPCHK(c, hipEventCreateWithFlags(&c->params_ev, hipEventDisableTiming));
+    for (hipEvent_t& e : c->io_ev) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
     return MD_OK;
 }
 
@@ -1467,15 +1478,19 @@ int md_get_options(const md_ctx* c, md_options* out) {
 template <typename Launch>
 static int io_run(md_ctx* c, double* const (&host)[5], bool put, Launch launch) {
     static const int width[5] = {3, 3, 3, 1, 1};
-    size_t per = 0;
-    for (int k = 0; k < 5; ++k) per += host[k] ? sizeof(double) * width[k] : 0;
+    size_t per = 0, arrays = 0;
+    for (int k = 0; k < 5; ++k) {
+        per += host[k] ? sizeof(double) * width[k] : 0;
+        arrays += host[k] ? 1 : 0;
+    }
     const int64_t n = c->n_atoms;
+    const size_t bytes = (size_t)n * per;
     c->d.par = c->par;
-    bool pinned = per > 0 && (size_t)n * per <= kIoPinned;
+    bool pinned = bytes <= (put ? kIoPinned : arrays * kIoPinned);
     int rc;
     if ((rc = need_arrays(c, false))) return rc;
-    if (!pinned && per > 0) {
-        const size_t need = std::min((size_t)n * per, kIoBytes);
+    if (!pinned) {
+        const size_t need = std::min(bytes, kIoBytes);
         if (need > c->io_cap) {
             if (c->io_dev) HIPCHK(c, hipFree(c->io_dev));
             c->io_dev = nullptr;
@@ -1490,40 +1505,67 @@ static int io_run(md_ctx* c, double* const (&host)[5], bool put, Launch launch) 
         }
     }
     if (pinned && (rc = pinned_staging(c))) return rc;
-    const int64_t chunk = per == 0 ? n : (int64_t)((pinned ? c->io_pin_cap : c->io_cap) / per);
-    int64_t a0 = 0;
-    do {
+    // more than the pinned block holds: pieces take its halves in turn
+    const bool halves = pinned && bytes > c->io_pin_cap;
+    const size_t room = pinned ? (halves ? c->io_pin_cap / 2 : c->io_pin_cap) : c->io_cap;
+    const int64_t chunk = per == 0 ? n : (int64_t)(room / per);
+    // the arrays of atoms [a0, a0 + chunk) one after the other from `base`
+    auto at = [&](int64_t a0, void* base) {
         StateIO io{};
         io.a0 = a0;
         io.a1 = std::min(n, a0 + chunk);
-        double** dev[5] = {&io.x, &io.v, &io.f, &io.pot, &io.vir};
-        size_t off = 0;
-        size_t at[5];
+        double** p[5] = {&io.x, &io.v, &io.f, &io.pot, &io.vir};
+        char* q = (char*)base;
         for (int k = 0; k < 5; ++k) {
             if (!host[k]) continue;
-            at[k] = off;
-            *dev[k] = (double*)((char*)(pinned ? c->io_pin_dev : c->io_dev) + off);
-            off += sizeof(double) * width[k] * (size_t)(io.a1 - io.a0);
+            *p[k] = (double*)q;
+            q += sizeof(double) * width[k] * (size_t)(io.a1 - io.a0);
         }
-        auto move = [&](bool to_device) -> int {
-            for (int k = 0; k < 5; ++k) {
-                if (!host[k]) continue;
-                double* h = host[k] + (size_t)width[k] * a0;
-                const size_t bytes = sizeof(double) * width[k] * (size_t)(io.a1 - io.a0);
-                if (pinned && to_device) memcpy((char*)c->io_pin + at[k], h, bytes);
-                else if (pinned) memcpy(h, (char*)c->io_pin + at[k], bytes);
-                else if (to_device) HIPCHK(c, hipMemcpyAsync(*dev[k], h, bytes, hipMemcpyHostToDevice, c->st));
-                else HIPCHK(c, hipMemcpyAsync(h, *dev[k], bytes, hipMemcpyDeviceToHost, c->st));
-            }
-            return MD_OK;
-        };
-        if (put && (rc = move(true))) return rc;
+        return io;
+    };
+    auto move = [&](const StateIO& io, bool to_device) -> int {
+        double* const p[5] = {io.x, io.v, io.f, io.pot, io.vir};
+        for (int k = 0; k < 5; ++k) {
+            if (!host[k]) continue;
+            double* h = host[k] + (size_t)width[k] * io.a0;
+            const size_t size = sizeof(double) * width[k] * (size_t)(io.a1 - io.a0);
+            if (pinned && to_device) memcpy(p[k], h, size);
+            else if (pinned) memcpy(h, p[k], size);
+            else if (to_device) HIPCHK(c, hipMemcpyAsync(p[k], h, size, hipMemcpyHostToDevice, c->st));
+            else HIPCHK(c, hipMemcpyAsync(h, p[k], size, hipMemcpyDeviceToHost, c->st));
+        }
+        return MD_OK;
+    };
+    StateIO last{};  // halves, from the device: the piece still to be copied
+    int half = 0;
+    int64_t a0 = 0;
+    do {
+        const size_t off = halves && half ? room : 0;
+        const StateIO io = at(a0, (char*)(pinned ? c->io_pin_dev : c->io_dev) + off);
+        const StateIO mine = pinned ? at(a0, (char*)c->io_pin + off) : io;
+        if (put) {
+            if (halves && a0 >= 2 * chunk) HIPCHK(c, hipEventSynchronize(c->io_ev[half]));
+            if ((rc = move(mine, true))) return rc;
+        }
         HIPCHK(c, launch(io));
-        // pinned: the results are there, or the next piece may take the place of this one
-        if (pinned && (!put || io.a1 < n)) HIPCHK(c, hipStreamSynchronize(c->st));
-        if (!put && (rc = move(false))) return rc;
+        if (halves) HIPCHK(c, hipEventRecord(c->io_ev[half], c->st));
+        if (!put && halves) {
+            if (a0 > 0) {
+                HIPCHK(c, hipEventSynchronize(c->io_ev[half ^ 1]));
+                if ((rc = move(last, false))) return rc;
+            }
+            last = mine;
+        } else if (!put) {
+            if (pinned) HIPCHK(c, hipStreamSynchronize(c->st));
+            if ((rc = move(mine, false))) return rc;
+        }
+        half ^= 1;
         a0 = io.a1;
     } while (a0 < n);
+    if (!put && halves) {
+        HIPCHK(c, hipEventSynchronize(c->io_ev[half ^ 1]));
+        return move(last, false);
+    }
     if (!put && !pinned) HIPCHK(c, hipStreamSynchronize(c->st));
     return MD_OK;
 }

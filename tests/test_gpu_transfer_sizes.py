@@ -1,7 +1,8 @@
-"""Uploads and downloads on both sides of the size where they stop passing
-through pinned memory (2 MB: 23,831 atoms of everything, 43,690 of positions and
-velocities): the same bits come back, and a download costs no jump where it used
-to change its way (256 KB: 2,978 atoms)."""
+"""Uploads and downloads where they change their way: pinned memory (up to 256
+KB: 2,978 atoms of everything), its halves in turn (downloads up to 256 KB an
+array: 14,894 atoms of everything, 10,922 of positions and velocities), device
+staging, and pieces of that (128 MB).  The same bits come back, and a download
+costs no jump at the first of these sizes."""
 import time
 
 import numpy as np
@@ -22,7 +23,7 @@ def engine(n, mode="fp64_list"):
     return e, x, v, rng
 
 
-@pytest.mark.parametrize("n", [2978, 2979, 23831, 23832, 43690, 43691])
+@pytest.mark.parametrize("n", [2978, 2979, 4468, 7447, 10922, 10923, 14894, 14895, 30000])
 def test_round_trip(n):
     e, x, v, rng = engine(n)
     f, pot, vir = rng.normal(size=(n, 3)), rng.normal(size=n), rng.normal(size=n)
