@@ -159,15 +159,6 @@ __device__ void build_list_global(const DevState& d, const RepCtrl& C, const Rep
     list_close(d, slot, n);
 }
 
-
-// The reference's minimum image (potential.rs:186-200) as selects, for the
-// list builder's exact tests: the same values as min_image, without a branch
-// per component in the candidate loops.
-__device__ __forceinline__ double min_image_sel(double r, double b) {
-    const double h = b / 2.0;
-    return r < -h ? r + b : (r > h ? r - b : r);
-}
-
 // LDS of a brick: one object per kernel, shared by the builders of both
 // record types.
 struct BrickLds {
@@ -518,9 +509,9 @@ __device__ __forceinline__ void brick_build(const DevState& d, const RepCtrl& C,
                     if (b2 == a) continue;
                     if (MULTI && (int)s_ty[b2] < ti) continue;
                     const int32_t j = s_id[b2];
-                    const double dx = min_image_sel(s_x[b2] - xi, bx);
-                    const double dy = min_image_sel(s_y[b2] - yi, by);
-                    const double dz = min_image_sel(s_z[b2] - zi, bz);
+                    const double dx = min_image_s(s_x[b2] - xi, bx);
+                    const double dy = min_image_s(s_y[b2] - yi, by);
+                    const double dz = min_image_s(s_z[b2] - zi, bz);
                     const double r2 = (dx * dx + dy * dy) + dz * dz;
                     if (!(r2 <= rl2)) continue;
                     lst.push(j);

@@ -328,7 +328,7 @@ __host__ __device__ inline bool decimal_to_double(uint64_t w, int q, const Pow5T
     const int k = q < 0 ? -q : q;
     if (q < 0 ? k >= MD_POW5_INV_COUNT : k >= MD_POW5_COUNT) return false;
     const uint64_t lo = q < 0 ? tb.inv[k][0] : tb.pos[k][0], hi = q < 0 ? tb.inv[k][1] : tb.pos[k][1];
-    const int bits5 = ((k * 1217359) >> 19) + 1;  // of 5^k
+    const int bits5 = (int)txt_pow5bits(k);
     int e = q < 0 ? -(bits5 - 1 + 125) - k : bits5 - 125 + k;
     const unsigned __int128 a = (unsigned __int128)lo * w, b = (unsigned __int128)hi * w;
     uint64_t n0 = (uint64_t)a;
