@@ -383,10 +383,10 @@ __host__ __device__ inline void brick_dims(const int* gd, int64_t n_atoms, int* 
     const double per_cell = (double)n_atoms / ((double)gd[0] * gd[1] * gd[2]);
     const int g0 = gd[0], g1 = gd[1], g2 = gd[2];
     // edges e (cubic), then e with the last one or two axes a cell longer:
-    // in dense systems a cubic brick that fits the staging capacity leaves
-    // most threads without a centre particle, and one cell more along an
-    // axis or two doubles the centre (scalars only: the device control
-    // update keeps its state in registers)
+    // where cells hold several particles and lists are still short, a cubic
+    // brick that fits the staging capacity leaves most threads without a centre
+    // particle, and one cell more along an axis or two doubles the centre
+    // (scalars only: the device control update keeps its state in registers)
     int b0 = 1, b1 = 1, b2 = 1;
     double best_own = -1.0, best_halo = 0.0;
     for (int e = 1; e <= kBrickEdge; ++e) {

@@ -14,11 +14,15 @@
 //           then the Berendsen / Nose-Hoover lambda, psi and Berendsen mu of
 //           the next step (thermostat.rs:24-72, barostat.rs:21-56), box
 //           rescale and the list-validity decision for the next launch; its
-//           other blocks build the Verlet lists brick by brick in launches
-//           flagged F_BUILD (k_step does nothing in those).
+//           other blocks build the Verlet lists in launches flagged F_BUILD
+//           (k_step does nothing in those): brick by brick in sparse systems,
+//           a wave per cell in dense ones.
 // Everything stays on the device; the host replays a graph of launches.
-// The O(N^2) FP64 path (k_drift + k_allpairs) restates update_force exactly:
-// same pair criterion, same operation order, j ascending.
+// The O(N^2) FP64 path restates update_force exactly: same pair criterion, same
+// operation order, j ascending.  k_ap_force finds and sums the pairs of 16
+// particles per block (a step: k_drift before it, k_ap_finish after it); where
+// more than 48 pairs per particle are in range, k_allpairs sums with a thread per
+// particle (k_drift before it in a step).
 //
 // All code is built with -ffp-contract=off: the FP64 paths must not form FMAs
 // the reference (Rust) never forms.  The FP32 pair kernel uses explicit fmaf.
@@ -845,7 +849,10 @@ constexpr int wave_scratch_bytes() {
 // for 35,937 FP64 particles of two types, 167 for 262,144 and 514 for 1,000,000;
 // this 25.2, 91 and 419; one FP32 type 52 us for 262,144, 191 for 1,000,000;
 // this 39.8 and 139.  FP64 depth 3: 24.0, 98 and 430; FP32 depth 2, 3, 6: 42.2,
-// 39.4, 43.4 for 262,144 and 3: 18.1 against 17.4 for 13,824.
+// 39.4, 43.4 for 262,144 and 3: 18.1 against 17.4 for 13,824.  FP32 liquids of two
+// types, 200 steps of 4,096, 35,937 and 262,144 particles: 16.0, 19.9 and 44.6 ms
+// before, 6.8, 9.5 and 26.2 with depth 4; of three types 16.0, 20.2 and 61.9, now
+// 7.3, 10.8 and 32.6 (that instance keeps 15 registers in scratch).
 constexpr int kWalkDepth64 = 2, kWalkDepth32 = 4;
 
 // The list forces of a wave's particles (potential.rs:158-216 over the Verlet
@@ -865,7 +872,7 @@ template <typename FT, bool MULTI, bool WALK>
 __device__ __forceinline__ Acc<FT> wave_list_forces(const DevState& d, const CRec* __restrict__ src, char* wreg,
                                                     int n_mine, const CRec& o0, int tj0, int32_t e0, int64_t s,
                                                     double x1, double y1, double z1, const PairParam* prow, bool split,
-                                                    double lam,                                                    double dt, double bx, double by, double bz,
+                                                    double lam, double dt, double bx, double by, double bz,
                                                     const PairParam& p0) {
     typedef typename Acc<FT>::Terms Terms;
     constexpr int W = 64;
@@ -997,10 +1004,11 @@ __device__ __forceinline__ Acc<FT> wave_list_forces(const DevState& d, const CRe
 // starts.
 // The last step of a chunk also writes the full records (x, v, F) and the
 // per-particle energies.
-// FP64 in dense systems takes the registers of two waves per SIMD: at four it
-// keeps part of the walk in scratch (262,144 particles of two types 99 us a
-// launch, 91 so; FP32 loses, 47 against 43 us).
-// MIRROR: and into host memory, for DevState::h_rec (a branch on it at run time
+// FP64 in dense systems may take the registers of two waves per SIMD and takes
+// those of three (138 VGPRs, 146 with several types): bound to four it keeps part
+// of the walk in scratch (262,144 particles of two types 99 us a launch, 91 so;
+// FP32 loses, 47 against 43 us).
+// MIRROR: the last step's state goes into host memory too, for DevState::h_rec (a branch on it at run time
 // cost every other system 1.1 us of 48.9 a launch, 256 replicas of 500 to 32,768).
 template <typename FT, int BS, bool MULTI, bool DENSE, bool MIRROR>
 __global__ __launch_bounds__(BS, DENSE && sizeof(FT) == 8 ? 2 : 4) void k_step(DevState d) {
